@@ -4,19 +4,21 @@
 // whose per-element lhs/rhs go through SolverAlgorithm::apply_coeff ->
 // TpetraLinearSystem::sumInto, src/TpetraLinearSystem.C:1457-1522).
 //
-// Two scatter strategies share the same per-(element, row-node) arithmetic
-// (hex8_device.hpp):
-//   * owner-computes row gather (mode 0): one thread per matrix row walks the
-//     elements incident to its node, accumulates its row in LDS and the block
-//     writes its contiguous CSR segment once, coalesced.  No atomics, fully
-//     deterministic, and zeroSystem's memset of the values can be folded in.
-//   * element-centric atomic scatter (mode 1): eight waves per block, wave w
-//     computing row w of 64 elements, FP64 atomic adds into the CSR.
+// All kernels share the row arithmetic of hex8_row.hpp: one thread evaluates the
+// row of one node in one incident element, its corners numbered relative to that
+// node, on one code path for all eight local nodes.  Two scatter strategies:
+//   * owner-computes row tiles (modes 0 and 2): a block owns consecutive rows,
+//     eight threads per row take its incident elements, the rows meet in the LDS
+//     copy of the block's CSR segment, which is written once, coalesced; a pending
+//     zeroSystem is folded into that write.
+//   * element-centric atomic scatter (mode 1): a block evaluates one local node's
+//     row of a chunk of elements, FP64 atomic adds into the CSR.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
 
 #include "hex8_device.hpp"
+#include "hex8_row.hpp"
 #include "internal.hpp"
 
 namespace nalu {
@@ -24,138 +26,281 @@ namespace {
 
 inline unsigned blocks_for(int64_t n, int per) { return (unsigned)std::max<int64_t>(1, (n + per - 1) / per); }
 
-__device__ __forceinline__ void load_nodes(const int32_t* __restrict__ conn, int64_t e, int32_t (&nd)[8]) {
+// ---------------------------------------------------------------- element data in relative order
+struct RowElem {
+  uint32_t nd[8];  // nodes by relative corner (hex8_row.hpp)
+  int la;          // the row's local node
+  int64_t e;
+};
+
+__device__ __forceinline__ RowElem row_elem(const int32_t* __restrict__ conn, int64_t e, int la) {
   const int4* c4 = reinterpret_cast<const int4*>(conn + 8 * e);
   const int4 a = c4[0], b = c4[1];
-  nd[0] = a.x; nd[1] = a.y; nd[2] = a.z; nd[3] = a.w;
-  nd[4] = b.x; nd[5] = b.y; nd[6] = b.z; nd[7] = b.w;
+  RowElem r{{(uint32_t)a.x, (uint32_t)a.y, (uint32_t)a.z, (uint32_t)a.w, (uint32_t)b.x, (uint32_t)b.y, (uint32_t)b.z,
+             (uint32_t)b.w},
+            la, e};
+  hexrow::relative_order(r.nd, la);
+  return r;
 }
 
-template <typename R>
-__device__ __forceinline__ void load_vec3(const double* __restrict__ f, const int32_t (&nd)[8], R (&v)[8][3]) {
-#pragma unroll
-  for (int n = 0; n < 8; ++n)
-#pragma unroll
-    for (int d = 0; d < 3; ++d) v[n][d] = R(f[3 * (int64_t)nd[n] + d]);
-}
-
-// Element coordinates in the arithmetic type R.  The FP32 path works on
-// coordinates relative to the element's first node, the differences formed in
-// FP64, so that short edges of stretched elements keep their relative accuracy.
-template <typename R>
-__device__ __forceinline__ void load_coords(const double* __restrict__ f, const int32_t (&nd)[8], R (&x)[8][3]) {
-  if constexpr (std::is_same<R, double>::value) {
-    load_vec3(f, nd, x);
-  } else {
-    const double o[3] = {f[3 * (int64_t)nd[0]], f[3 * (int64_t)nd[0] + 1], f[3 * (int64_t)nd[0] + 2]};
-#pragma unroll
-    for (int n = 0; n < 8; ++n)
-#pragma unroll
-      for (int d = 0; d < 3; ++d) x[n][d] = R(f[3 * (int64_t)nd[n] + d] - o[d]);
-  }
-}
-
-template <typename R>
-__device__ __forceinline__ void load_scalar(const double* __restrict__ f, const int32_t (&nd)[8], R (&v)[8]) {
-#pragma unroll
-  for (int n = 0; n < 8; ++n) v[n] = R(f[nd[n]]);
-}
-
-// ---------------------------------------------------------------- physics ops
-// Each op evaluates row LA of its element matrix, calling emit(c, value) once
-// per column node c, and returns the row's rhs contribution.  R is the
-// arithmetic type (double, or float for the mixed-precision path); Jacobians
-// and their determinants are always formed in FP64.
-template <bool SHIFT, typename R = double>
-struct ScalarDiffOp {
-  using real = R;
-  const double* q;
-  const double* k;
-  template <int LA, class Emit>
-  __device__ __forceinline__ R row(const int32_t (&nd)[8], const R (&x)[8][3], Emit&& emit) const {
-    const hex8::Gather gt{nd};
-    return hex8::row_scalar_diff<LA, SHIFT, double>(x, gt, q, k, emit);
-  }
+// A vector field [N][3] and, with it, a scalar field [N] (or none), as the caller
+// holds them, or (PACK) copied together to 16-byte entries of one array per half:
+// (v0, v1) and (v2, s) in double, (v0, v1, v2, s) in float.  The vector cache
+// serves four lanes a cycle from one 64-byte line each.  Neighbouring lanes read
+// neighbouring nodes, so a load of 16-byte entries takes 16 cycles for 1 KB, one of
+// a scalar field 16 cycles for 512 B, and the two loads of a 24-byte [N][3] entry
+// about 55 cycles for 1.5 KB.  That rate bounds the row kernels, which read each
+// node's fields for up to eight elements of eight rows, so larger systems first
+// copy the fields of a pass (k_pack, k_pack_flux; 40 us for continuity at 128^3).
+// Entry offsets are 32-bit.
+template <typename T>
+struct alignas(16) Half {
+  T v[16 / sizeof(T)];
+};
+template <typename T = double>
+struct Field4 {
+  const Half<T>* h[2];  // PACK (the second for double only)
+  const double* vec;    // otherwise [N][3]
+  const double* scal;   // and [N], or null
 };
 
-template <bool SHIFT_MDOT, bool SHIFT_POISSON, bool REDUCED, typename R = double>
-struct ContinuityOp {
-  using real = R;
-  const double* rho;
-  const double* p;
-  const double* u;
-  const double* gp;
-  double tau;
-  double* mdot_out = nullptr;  // [E][12]: the mdot of each scs, written by the row of its left node
-  template <int LA, class Emit>
-  __device__ __forceinline__ R row(const int32_t (&nd)[8], const R (&x)[8][3], Emit&& emit) const {
-    const hex8::Gather gt{nd};
-    return hex8::row_continuity<LA, SHIFT_MDOT, SHIFT_POISSON, REDUCED, double>(x, gt, rho, p, u, gp, R(tau), emit);
-  }
-  // the same row, also delivering the mdot of the scs it owns (mdot_out != nullptr)
-  template <int LA, class Emit>
-  __device__ __forceinline__ R row_e(const int32_t (&nd)[8], const R (&x)[8][3], int64_t e, Emit&& emit) const {
-    const hex8::Gather gt{nd};
-    double* mo = mdot_out + 12 * e;
-    return hex8::row_continuity<LA, SHIFT_MDOT, SHIFT_POISSON, REDUCED, double>(
-        x, gt, rho, p, u, gp, R(tau), emit, [&](int ip, R v) { mo[ip] = (double)v; });
-  }
-};
-
-// ops whose rows can also write per-element outputs (row_e)
-template <class Op, class = void>
-struct HasRowE : std::false_type {};
-template <class Op>
-struct HasRowE<Op, std::void_t<decltype(&Op::mdot_out)>> : std::true_type {};
-
-// dispatch a wave-uniform (or mostly uniform) runtime row index to the
-// compile-time specialisation
-template <class Op, class Emit>
-__device__ __forceinline__ typename Op::real dispatch_row(const Op& op, int la, const int32_t (&nd)[8],
-                                                          const typename Op::real (&x)[8][3], Emit&& emit) {
-  switch (la) {
-    case 0: return op.template row<0>(nd, x, emit);
-    case 1: return op.template row<1>(nd, x, emit);
-    case 2: return op.template row<2>(nd, x, emit);
-    case 3: return op.template row<3>(nd, x, emit);
-    case 4: return op.template row<4>(nd, x, emit);
-    case 5: return op.template row<5>(nd, x, emit);
-    case 6: return op.template row<6>(nd, x, emit);
-    default: return op.template row<7>(nd, x, emit);
-  }
+template <typename T>
+__device__ __forceinline__ Half<T> half_at(const Half<T>* __restrict__ f, uint32_t n) {
+  return *reinterpret_cast<const Half<T>*>(reinterpret_cast<const char*>(f) + (uint32_t)(16 * n));
 }
 
-// dispatch_row with the element index, for ops with per-element outputs when
-// they are requested
-template <class Op, class Emit>
-__device__ __forceinline__ typename Op::real dispatch_row_e(const Op& op, int la, const int32_t (&nd)[8],
-                                                            const typename Op::real (&x)[8][3], int64_t e,
-                                                            Emit&& emit) {
-  if constexpr (HasRowE<Op>::value) {
-    if (op.mdot_out) {
-      switch (la) {
-        case 0: return op.template row_e<0>(nd, x, e, emit);
-        case 1: return op.template row_e<1>(nd, x, e, emit);
-        case 2: return op.template row_e<2>(nd, x, e, emit);
-        case 3: return op.template row_e<3>(nd, x, e, emit);
-        case 4: return op.template row_e<4>(nd, x, e, emit);
-        case 5: return op.template row_e<5>(nd, x, e, emit);
-        case 6: return op.template row_e<6>(nd, x, e, emit);
-        default: return op.template row_e<7>(nd, x, e, emit);
+template <bool PACK, typename R>
+__device__ __forceinline__ void load1(const double* __restrict__ f, const uint32_t (&nd)[8], R (&v)[8]) {
+#pragma unroll
+  for (int m = 0; m < 8; ++m)
+    v[m] = PACK ? R(*reinterpret_cast<const double*>(reinterpret_cast<const char*>(f) + (uint32_t)(8 * nd[m])))
+                : R(f[nd[m]]);
+}
+// vector part component-major, v[i][m]; scalar part s[m] (SCAL)
+template <bool PACK, bool SCAL, typename T, typename R, typename S>
+__device__ __forceinline__ void load4(const Field4<T>& f, const uint32_t (&nd)[8], R (&v)[3][8], S (&s)[8]) {
+#pragma unroll
+  for (int m = 0; m < 8; ++m) {
+    if (PACK) {
+      const Half<T> r = half_at(f.h[0], nd[m]);
+      if constexpr (sizeof(T) == 8) {
+        const Half<T> r2 = half_at(f.h[1], nd[m]);
+        v[0][m] = R(r.v[0]);
+        v[1][m] = R(r.v[1]);
+        v[2][m] = R(r2.v[0]);
+        if (SCAL) s[m] = S(r2.v[1]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) v[i][m] = R(r.v[i]);
+        if (SCAL) s[m] = S(r.v[3]);
       }
+    } else {
+      const double* q = f.vec + 3 * (uint64_t)nd[m];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) v[i][m] = R(q[i]);
+      if (SCAL) s[m] = S(f.scal[nd[m]]);
     }
   }
-  return dispatch_row(op, la, nd, x, emit);
+}
+template <bool PACK, typename R>
+__device__ __forceinline__ void load3(const Field4<double>& f, const uint32_t (&nd)[8], R (&v)[3][8]) {
+  R none[8];
+  load4<PACK, false>(f, nd, v, none);
 }
 
-__device__ __forceinline__ int32_t pick(const int32_t (&nd)[8], int la) {
-  int32_t node = nd[0];
-#pragma unroll
-  for (int c = 1; c < 8; ++c) node = (la == c) ? nd[c] : node;
-  return node;
+// Copies of up to six (vector, scalar) field pairs, 2 nnodes entries each.
+struct PackList {
+  const double* vec[6];
+  const double* scal[6];
+  int n;
+};
+__global__ __launch_bounds__(256) void k_pack(PackList L, int64_t nnodes, Half<double>* __restrict__ dst) {
+  const int64_t a = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (a >= nnodes) return;
+  for (int k = 0; k < L.n; ++k) {
+    const double* f = L.vec[k] + 3 * a;
+    dst[2 * k * nnodes + a] = {{f[0], f[1]}};
+    dst[(2 * k + 1) * nnodes + a] = {{f[2], L.scal[k] ? L.scal[k][a] : 0.0}};
+  }
 }
+// Copies of (coordinates, p) and, in the arithmetic type, of the mass flux vector rho u + tau Gp.
+template <typename R>
+__global__ __launch_bounds__(256) void k_pack_flux(const double* __restrict__ coords, const double* __restrict__ p,
+                                                   const double* __restrict__ rho, const double* __restrict__ u,
+                                                   const double* __restrict__ gp, double tau, int64_t nnodes,
+                                                   Half<double>* __restrict__ x, Half<R>* __restrict__ W) {
+  const int64_t a = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (a >= nnodes) return;
+  const R r = R(rho[a]);
+  R w[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) w[i] = r * R(u[3 * a + i]) + R(tau) * R(gp[3 * a + i]);
+  x[a] = {{coords[3 * a], coords[3 * a + 1]}};
+  x[nnodes + a] = {{coords[3 * a + 2], p[a]}};
+  if constexpr (sizeof(R) == 8) {
+    W[a] = {{w[0], w[1]}};
+    W[nnodes + a] = {{w[2], 0.0}};
+  } else {
+    W[a] = {{w[0], w[1], w[2], 0.0f}};
+  }
+}
+
+using hex8::static_for;
+
+// Phase boundaries of a row's evaluation.  Left alone, the compiler interleaves
+// the three directions and hoists every field load to the top, which takes up to
+// twice the registers (half the waves in flight, or spills).  An empty asm that
+// "modifies" a value orders what produces it before what uses it, and volatile
+// asms keep their order: pin the results of one phase, then the inputs of the next.
+template <typename T>
+__device__ __forceinline__ void pin(T& v) {
+  asm volatile("" : "+v"(v));
+}
+template <typename T, int N>
+__device__ __forceinline__ void pin(T (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) pin(v[i]);
+}
+__device__ __forceinline__ void pin(hexrow::Edges& E) { pin(E.e); }
+// loads through a node list pinned here stay after it
+__device__ __forceinline__ void pin(RowElem& r) { pin(r.nd); }
 
 // ---------------------------------------------------------------- scalar systems
+// Each op evaluates the row of r.la in element r.e: v[m] gets the entry of
+// relative corner m's column, the return value is the row's rhs contribution
+// (times rhs_scale).  R is the arithmetic type of the physics (double, or float
+// for the mixed-precision path); the geometry is always FP64.
+
+// ScalarDiffElemKernel (src/kernel/ScalarDiffElemKernel.C:66-111): entry -sum_scs k_ip dN/dx . A_out, rhs -entry . q
+template <bool SHIFT, bool PACK, typename R>
+struct ScalarDiffOp {
+  Field4<> xk;      // coordinates and conductivity
+  const double* q;
+  double rhs_scale() const { return 1.0; }
+  __device__ __forceinline__ double eval(RowElem& r, double (&v)[8]) const {
+    R g[3][3], kn[8], qn[8], w[8];
+    {
+      double x[3][8];
+      load4<PACK, true>(xk, r.nd, x, kn);
+      hexrow::Edges E;
+      hexrow::edges(x, E);
+      const double h = hexrow::handed(r.la);
+      static_for<3>([&](auto dd) {
+        constexpr int D = decltype(dd)::value;
+        double A[3];
+        hexrow::Cof K;
+        hexrow::area_cofactors<D, SHIFT>(E, h, A, K);
+        hexrow::metric<SHIFT>(K, A, g[D]);
+        pin(g[D]);
+        pin(E);
+      });
+    }
+    pin(r);
+    load1<PACK>(q, r.nd, qn);
+#pragma unroll
+    for (int m = 0; m < 8; ++m) w[m] = R(0);
+    static_for<3>([&](auto dd) {
+      constexpr int D = decltype(dd)::value;
+      const R kip = hexrow::at_scs<D, false>(kn);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) g[D][i] *= kip;
+      hexrow::slope<D, SHIFT>(g[D], [&](int m, R t) { w[m] -= t; });
+    });
+    R rhs = R(0);
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      rhs -= w[m] * qn[m];
+      v[m] = (double)w[m];
+    }
+    return (double)rhs;
+  }
+};
+
+// ContinuityAdvElemKernel (src/kernel/ContinuityAdvElemKernel.C:88-148) with the mass
+// flow rate of ComputeMdotElemAlgorithm (src/ComputeMdotElemAlgorithm.C:204-232) at
+// each scs: mdot = (rho u + tau Gp)_ip . A - tau grad p . A; entry -sum_scs dN_lhs/dx . A_out,
+// rhs -sum mdot_out / tau (the division is left to rhs_scale).  MDOT: the row of the
+// left node also writes the scs's mdot (each scs has exactly one left node, so the
+// rows of an element deliver all twelve).
+template <bool SHIFT_MDOT, bool SHIFT_POISSON, bool REDUCED, bool MDOT, bool PACK, typename R>
+struct ContinuityOp {
+  Field4<> xp;        // coordinates and pressure
+  Field4<R> W4;       // PACK: rho u + tau Gp (k_pack_flux)
+  Field4<> ur;        // otherwise u and rho,
+  const double* gp;   // and Gp
+  double tau;
+  double* mdot_out;  // [E][12] (MDOT)
+  double rhs_scale() const { return 1.0 / tau; }
+  __device__ __forceinline__ double eval(RowElem& r, double (&v)[8]) const {
+    constexpr bool LHS_SHIFT = SHIFT_POISSON || REDUCED, TWO = LHS_SHIFT != SHIFT_POISSON;
+    // geometry: area vectors and metrics of the three directions
+    R A[3][3], g[3][3], gp_[TWO ? 3 : 1][3], pn[8];
+    {
+      double x[3][8];
+      load4<PACK, true>(xp, r.nd, x, pn);
+      hexrow::Edges E;
+      hexrow::edges(x, E);
+      const double h = hexrow::handed(r.la);
+      static_for<3>([&](auto dd) {
+        constexpr int D = decltype(dd)::value;
+        double a[3];
+        hexrow::Cof K;
+        hexrow::area_cofactors<D, LHS_SHIFT>(E, h, a, K);
+        hexrow::metric<LHS_SHIFT>(K, a, g[D]);
+        if constexpr (TWO) {
+          hexrow::cofactors<D, SHIFT_POISSON>(E, K);
+          hexrow::metric<SHIFT_POISSON>(K, a, gp_[D]);
+          pin(gp_[D]);
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) A[D][i] = R(a[i]);
+        pin(A[D]);
+        pin(g[D]);
+        pin(E);
+      });
+    }
+    // flux through the scs and matrix entries
+    pin(r);
+    R W[3][8], w[8], out = R(0);
+    if constexpr (PACK) {
+      R none[8];
+      load4<true, false>(W4, r.nd, W, none);
+    } else {
+      R rn[8], gn[3][8];
+      load4<false, true>(ur, r.nd, W, rn);
+      load3<false>(Field4<>{{}, gp, nullptr}, r.nd, gn);
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int m = 0; m < 8; ++m) W[i][m] = rn[m] * W[i][m] + R(tau) * gn[i][m];
+    }
+#pragma unroll
+    for (int m = 0; m < 8; ++m) w[m] = R(0);
+    static_for<3>([&](auto dd) {
+      constexpr int D = decltype(dd)::value;
+      R dp = R(0);
+      hexrow::slope<D, LHS_SHIFT>(g[D], [&](int m, R t) {
+        w[m] -= t;
+        if constexpr (!TWO) dp += pn[m] * t;
+      });
+      if constexpr (TWO) {
+        R ps[3];
+        hexrow::param_grad<D, SHIFT_POISSON>(pn, ps);
+        dp = ps[0] * gp_[D][0] + ps[1] * gp_[D][1] + ps[2] * gp_[D][2];
+      }
+      R f = -R(tau) * dp;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) f += hexrow::at_scs<D, SHIFT_MDOT>(W[i]) * A[D][i];
+      out += f;
+      if constexpr (MDOT)
+        if (hexrow::scs_is_left(r.la, D)) mdot_out[12 * r.e + hexrow::scs_of(r.la, D)] = (double)f;
+    });
+#pragma unroll
+    for (int m = 0; m < 8; ++m) v[m] = (double)w[m];
+    return -(double)out;
+  }
+};
+
 // Element-centric kernels: a block handles one local row node LA of a chunk of
 // kChunk elements.  The eight LA-blocks of a chunk are consecutive in the
 // dispatch order of one XCD (block b runs on XCD b % 8), so the chunk's nodal
@@ -181,91 +326,127 @@ inline unsigned chunk_blocks(int64_t nelem) {
   return (unsigned)(((nchunk + 7) / 8) * 8 * NL);
 }
 
-template <class Op, int LA>
-__device__ __forceinline__ void scalar_atomic_body(const Op& op, const int32_t* __restrict__ conn,
-                                                   const double* __restrict__ coords, const int32_t* __restrict__ lid,
-                                                   const int32_t* __restrict__ nrp,
-                                                   const uint64_t* __restrict__ elem_pos, int64_t e,
-                                                   double* __restrict__ vals, double* __restrict__ rhs) {
-  int32_t nd[8];
-  load_nodes(conn, e, nd);
-  typename Op::real x[8][3];
-  load_coords(coords, nd, x);
-  const int32_t row = lid[nd[LA]];
-  double* rowp = vals + nrp[row];
-  const uint64_t pk = elem_pos[8 * e + LA];
-  const double rr = (double)op.template row<LA>(nd, x, [&](int c, auto v) {
-    unsafeAtomicAdd(rowp + (int)((pk >> (8 * c)) & 0xff), (double)v);
-  });
-  unsafeAtomicAdd(rhs + row, rr);
-}
-
 template <class Op>
 __global__ __launch_bounds__(kChunk) void k_scalar_atomic(Op op, const int32_t* __restrict__ conn,
-                                                          const double* __restrict__ coords,
                                                           const int32_t* __restrict__ lid,
                                                           const int32_t* __restrict__ nrp,
-                                                          const uint64_t* __restrict__ elem_pos, int64_t nelem,
-                                                          double* __restrict__ vals, double* __restrict__ rhs) {
+                                                          ElemPos elem_pos, int64_t nelem,
+                                                          double rhs_scale, double* __restrict__ vals,
+                                                          double* __restrict__ rhs) {
   const ChunkMap cm = chunk_map<8>(nelem);
   if (!cm.valid) return;
-  switch (cm.la) {
-#define NALU_SA(L) \
-  case L: scalar_atomic_body<Op, L>(op, conn, coords, lid, nrp, elem_pos, cm.e, vals, rhs); break;
-    NALU_SA(0) NALU_SA(1) NALU_SA(2) NALU_SA(3) NALU_SA(4) NALU_SA(5) NALU_SA(6) NALU_SA(7)
-#undef NALU_SA
-  }
+  RowElem r = row_elem(conn, cm.e, cm.la);
+  const int32_t row = lid[r.nd[0]];
+  double* rowp = vals + nrp[row];
+  const uint64_t pk = hexrow::relative_bytes(elem_pos(cm.e, cm.la), cm.la);
+  double v[8];
+  const double rr = op.eval(r, v);
+#pragma unroll
+  for (int m = 0; m < 8; ++m) unsafeAtomicAdd(rowp + hexrow::pos(pk, m), v[m]);
+  unsafeAtomicAdd(rhs + row, rr * rhs_scale);
 }
 
-// Owner-computes row gather.  Block b owns rows [b*B, b*B+B); its CSR segment
-// lives in LDS while the rows accumulate, then is streamed out once.
+// Owner-computes row tile.  A wave owns kRowsPerWave consecutive rows and the LDS
+// copy of their CSR segment; lane (s, j) takes the s-th, (s + kSlots)-th, ...
+// incident element of row j.  Consecutive lanes are consecutive rows, so that a
+// load of one relative corner covers runs of neighbouring nodes.  Row sums are LDS
+// atomics of one wave in program order (and a fixed cross-lane tree for the
+// diagonal and the rhs, which all lanes of a row share), so results do not depend
+// on timing; the segment leaves in one coalesced pass.  No block barrier: waves
+// are independent.  Bound by the vector cache's address rate (68 % busy) and, at two
+// to three waves per SIMD, latency.  128^3 continuity with mdot: 0.75 ms (1.26 ms
+// for one thread per row over eight compile-time local nodes); the segregated
+// momentum with mass 1.40 ms (3.42 ms).
+constexpr int kSlots = 4;  // lanes of a row
+constexpr int kRowsPerWave = 64 / kSlots;
+constexpr int kRowWaves = 4;  // waves to a block
+constexpr int kRowThreads = 64 * kRowWaves;
+constexpr int kRowsPerBlock = kRowsPerWave * kRowWaves;
+constexpr size_t kMaxLds = 160 * 1024;  // LDS of one gfx950 CU, the most one block can hold
+
+// sum over the lanes of a row, in every lane
+__device__ __forceinline__ double row_sum(double v) {
+#pragma unroll
+  for (int s = kRowsPerWave; s < 64; s <<= 1) v += __shfl_xor(v, s);
+  return v;
+}
+
+// orders a wave's LDS accesses around a change of the lanes' roles
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// the wave's rows, and this lane's place in them
+struct WaveRows {
+  int64_t r0, r1, r;  // rows [r0, r1) of the wave, row of the lane (may be >= r1)
+  int lane, slot;
+  int32_t q, q1;      // next and last incidence entry of the lane
+};
+__device__ __forceinline__ WaveRows wave_rows(const int32_t* __restrict__ row_node,
+                                              const int32_t* __restrict__ inc_ptr, int64_t nrows) {
+  WaveRows w;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  w.lane = threadIdx.x & 63;
+  w.slot = w.lane / kRowsPerWave;
+  w.r0 = ((int64_t)blockIdx.x * (blockDim.x >> 6) + wave) * kRowsPerWave;
+  w.r1 = min(w.r0 + (int64_t)kRowsPerWave, nrows);
+  w.r = w.r0 + w.lane % kRowsPerWave;
+  w.q = w.q1 = 0;
+  if (w.r < w.r1) {
+    const int32_t a = row_node ? row_node[w.r] : (int32_t)w.r;
+    w.q = inc_ptr[a] + w.slot;
+    w.q1 = inc_ptr[a + 1];
+  }
+  return w;
+}
+
 template <class Op>
-__global__ __launch_bounds__(256) void k_scalar_gather(Op op, const int32_t* __restrict__ conn,
-                                                       const double* __restrict__ coords,
-                                                       const int32_t* __restrict__ row_node,
-                                                       const int32_t* __restrict__ inc_ptr,
-                                                       const int32_t* __restrict__ inc_elem,
-                                                       const int32_t* __restrict__ nrp,
-                                                       const uint64_t* __restrict__ elem_pos, int64_t nrows,
-                                                       double* __restrict__ vals, double* __restrict__ rhs,
-                                                       int accumulate) {
-  // the row segments accumulate in FP64 (FP32 LDS accumulation for the mixed
-  // path halved the LDS per row but made the pass slower)
-  using A = double;
-  extern __shared__ __align__(16) unsigned char seg_raw[];
-  A* seg = reinterpret_cast<A*>(seg_raw);
-  const int64_t r0 = (int64_t)blockIdx.x * blockDim.x;
-  const int64_t rend = min(r0 + (int64_t)blockDim.x, nrows);
-  const int64_t r = r0 + threadIdx.x;
-  const int32_t s0 = nrp[r0], s1 = nrp[rend];
-  const int nseg = s1 - s0;
-  for (int i = threadIdx.x; i < nseg; i += blockDim.x) seg[i] = A(0);
-  __syncthreads();
-  double rr = 0.0;
-  if (r < nrows) {
-    const int32_t a = row_node ? row_node[r] : (int32_t)r;
-    A* myrow = seg + (nrp[r] - s0);
-    const int32_t q1 = inc_ptr[a + 1];
-    for (int32_t q = inc_ptr[a]; q < q1; ++q) {
+__global__ __launch_bounds__(kRowThreads, 3) void k_scalar_rows(Op op, const int32_t* __restrict__ conn,
+                                                             const int32_t* __restrict__ row_node,
+                                                             const int32_t* __restrict__ inc_ptr,
+                                                             const int32_t* __restrict__ inc_elem,
+                                                             const int32_t* __restrict__ nrp,
+                                                             ElemPos elem_pos, int64_t nrows,
+                                                             int row_len, double rhs_scale, double* __restrict__ vals,
+                                                             double* __restrict__ rhs, int accumulate) {
+  extern __shared__ double seg_all[];
+  double* seg = seg_all + (size_t)(threadIdx.x >> 6) * kRowsPerWave * row_len;
+  const WaveRows w = wave_rows(row_node, inc_ptr, nrows);
+  if (w.r0 >= nrows) return;
+  const int32_t s0 = nrp[w.r0];
+  const int nseg = nrp[w.r1] - s0;
+  for (int i = w.lane; i < nseg; i += 64) seg[i] = 0.0;
+  wave_sync();
+  double rr = 0.0, diag = 0.0;
+  double* myrow = seg;
+  int at = 0;
+  if (w.q < w.q1) {
+    myrow = seg + (nrp[w.r] - s0);
+    for (int32_t q = w.q; q < w.q1; q += kSlots) {
       const int32_t t = inc_elem[q];
-      const int64_t e = t >> 3;
-      const int la = t & 7;
-      int32_t nd[8];
-      load_nodes(conn, e, nd);
-      typename Op::real x[8][3];
-      load_coords(coords, nd, x);
-      const uint64_t pk = elem_pos[t];
-      rr += (double)dispatch_row_e(op, la, nd, x, e,
-                                   [&](int c, auto v) { myrow[(int)((pk >> (8 * c)) & 0xff)] += (A)v; });
+      RowElem el = row_elem(conn, t >> 3, t & 7);
+      const uint64_t pk = hexrow::relative_bytes(elem_pos(t >> 3, t & 7), t & 7);
+      double v[8];
+      rr += op.eval(el, v);
+      diag += v[0];
+      at = hexrow::pos(pk, 0);
+#pragma unroll
+      for (int m = 1; m < 8; ++m) unsafeAtomicAdd(myrow + hexrow::pos(pk, m), v[m]);
     }
   }
-  __syncthreads();
+  rr = row_sum(rr);
+  diag = row_sum(diag);
+  if (w.slot == 0 && w.q < w.q1) unsafeAtomicAdd(myrow + at, diag);
+  wave_sync();
+  double* out = vals + s0;
   if (accumulate) {
-    for (int i = threadIdx.x; i < nseg; i += blockDim.x) vals[s0 + i] += (double)seg[i];
-    if (r < nrows) rhs[r] += rr;
+    for (int i = w.lane; i < nseg; i += 64) out[i] += seg[i];
+    if (w.slot == 0 && w.r < w.r1) rhs[w.r] += rr * rhs_scale;
   } else {
-    for (int i = threadIdx.x; i < nseg; i += blockDim.x) __builtin_nontemporal_store((double)seg[i], &vals[s0 + i]);
-    if (r < nrows) rhs[r] = rr;
+    for (int i = w.lane; i < nseg; i += 64) __builtin_nontemporal_store(seg[i], out + i);
+    if (w.slot == 0 && w.r < w.r1) rhs[w.r] = rr * rhs_scale;
   }
 }
 
@@ -273,277 +454,322 @@ __global__ __launch_bounds__(256) void k_scalar_gather(Op op, const int32_t* __r
 // MomentumMassElemKernel (src/kernel/MomentumMassElemKernel.C:95-170) and
 // ContinuityMassElemKernel (src/kernel/ContinuityMassElemKernel.C:84-118).  The
 // scv ip of an element belongs to one node (HexSCV::ipNodeMap_), so a node's
-// rows receive exactly the contributions of the scvs at that node: k_mass_gather
-// gives each node one thread that walks its incident elements (ip = the node's
-// local index) and adds into its rows and rhs in place (no atomics, no LDS);
-// the numDof 3 forms (k_mass_tile3, and the mass option of k_momentum_tile)
-// accumulate node tiles in LDS.
+// rows receive exactly the contributions of the scvs at that node.
 struct MassArgs {
-  const double* rho[3];  // Nm1, N, Np1 (nodal)
-  const double* u[3];    // Nm1, N, Np1 (nodal, 3 components; momentum only)
-  const double* gjp;     // projected pressure gradient (momentum only)
+  Field4<> s[3];         // velocity (momentum only) and density of the states Nm1, N, Np1
+  Field4<> gjp;          // projected pressure gradient (momentum only)
   double dt, g1, g2, g3;
   int balanced;          // densFac = rhoNp1 (balanced force) or 1
 };
 
-// ATOMIC: the row is shared with other threads (LDS row segment of a node tile)
-template <int LA, bool MOM, bool LUMPED, bool SEG, bool ATOMIC = false>
-__device__ __forceinline__ void mass_row(const MassArgs& A, const int32_t (&nd)[8], const double (&x)[8][3],
-                                         uint64_t pk, double* __restrict__ row, int32_t L, double (&rh)[3]) {
-  const double scV = hex8::scv_volume<LA>(x);
-  double rs[3] = {0.0, 0.0, 0.0}, us[3][3] = {}, g[3] = {0.0, 0.0, 0.0};
+// MomentumMassElemKernel at the row's scv: rh += its rhs; the return value times
+// scv_shape(m) is the diagonal lhs entry of corner m's block.
+template <bool LUMPED, bool PACK>
+__device__ __forceinline__ double momentum_mass_row(const MassArgs& A, const uint32_t (&nd)[8],
+                                                    const double (&x)[3][8], double h, double (&rh)[3]) {
+  double rs[3], acc[3] = {0.0, 0.0, 0.0}, f[8], f3[3][8];
+  const double g[3] = {A.g3, A.g2, A.g1};
+  double vol = hexrow::scv_volume(x, h);
+  pin(vol);
 #pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const double r = hex8::scv_shape<LA, LUMPED>(c);
-    if (LUMPED && c != LA) continue;
+  for (int st = 0; st < 3; ++st) {
+    load4<PACK, true>(A.s[st], nd, f3, f);
+    rs[st] = hexrow::at_scv<LUMPED>(f);
 #pragma unroll
-    for (int st = 0; st < 3; ++st) rs[st] += r * A.rho[st][nd[c]];
-    if (MOM) {
-#pragma unroll
-      for (int st = 0; st < 3; ++st)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) us[st][j] += r * A.u[st][3 * (int64_t)nd[c] + j];
-#pragma unroll
-      for (int j = 0; j < 3; ++j) g[j] += r * A.gjp[3 * (int64_t)nd[c] + j];
-    }
+    for (int i = 0; i < 3; ++i) acc[i] += g[st] * rs[st] * hexrow::at_scv<LUMPED>(f3[i]);
+    pin(acc);
+    asm volatile("" ::: "memory");
   }
-  if (MOM) {
-    const double densFac = A.balanced ? rs[2] : 1.0;
+  load3<PACK>(A.gjp, nd, f3);
+  const double vdt = vol / A.dt;
+  const double vd = A.balanced ? vol * rs[2] : vol;
 #pragma unroll
-    for (int j = 0; j < 3; ++j)
-      rh[j] += -(A.g1 * rs[2] * us[2][j] + A.g2 * rs[1] * us[1][j] + A.g3 * rs[0] * us[0][j]) * scV / A.dt -
-               g[j] * scV * densFac;
+  for (int i = 0; i < 3; ++i) rh[i] -= acc[i] * vdt + hexrow::at_scv<LUMPED>(f3[i]) * vd;
+  pin(rh);
+  return A.g1 * rs[2] * vdt;
+}
+
+// ---------------------------------------------------------------- momentum
+// MomentumAdvDiffElemKernel (src/kernel/MomentumAdvDiffElemKernel.C:72-186), the
+// row block of one node.  Rows (la, i), columns (c, j); per scs, with A outward
+// and mdot the outflow:
+//   lhs += delta_ij (N_adv(c) mdot - mu_ip dN_c/dx . A) - mu_ip dN_c/dx_i A_j
+//   rhs -= mdot u_ip,i + 2/3 mu_ip divU A_i incl
+//          - mu_ip sum_c dN_c/dx_i (A . u_c) - mu_ip sum_c (dN_c/dx . A) u_c,i
+// The advected u_ip uses the lhs's N_adv, so apart from the divU term the rhs is
+// -sum_c lhs(c) u_c.  mdot3: outflow through the scs of directions 0, 1, 2.
+// emit(m, blk) receives the 3x3 block blk[i][j] of relative corner m.
+struct MomentumFields {
+  Field4<> x;          // coordinates and viscosity
+  Field4<> u;          // velocity (PACK: with the density of the mass kernel's Np1 state, if it is the same field)
+  const double* mdot;  // [E][12]
+  double incl_divu;
+};
+
+// per direction: cofactor columns / det (along D, D+1, D+2) and mu_ip A
+template <typename R>
+struct MomentumGeo {
+  R b[3][3][3], mA[3][3];
+};
+template <bool SHIFT, typename R>
+__device__ __forceinline__ void momentum_geometry(const double (&x)[3][8], const R (&mn)[8], double h, RowElem& el,
+                                                  MomentumGeo<R>& G) {
+  R muip[3];
+  static_for<3>([&](auto dd) { muip[decltype(dd)::value] = hexrow::at_scs<decltype(dd)::value, false>(mn); });
+  hexrow::Edges E;
+  hexrow::edges(x, E);
+  static_for<3>([&](auto dd) {
+    constexpr int D = decltype(dd)::value;
+    double A[3];
+    hexrow::Cof K;
+    hexrow::area_cofactors<D, SHIFT>(E, h, A, K);
+    const double f0 = K.inv * hexrow::Scale<SHIFT>::c0, f1 = K.inv * hexrow::Scale<SHIFT>::c1;
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      if (LUMPED && c != LA) continue;
-      const double lf = hex8::scv_shape<LA, LUMPED>(c) * A.g1 * rs[2] * scV / A.dt;
-      const int p = (int)((pk >> (8 * c)) & 0xff);
-      if (SEG) {
-        row[p] += lf;
-      } else if (ATOMIC) {
+    for (int i = 0; i < 3; ++i) {
+      G.mA[D][i] = muip[D] * R(A[i]);
+      G.b[D][0][i] = R(K.c[0][i] * f0);
+      G.b[D][1][i] = R(K.c[1][i] * f1);
+      G.b[D][2][i] = R(K.c[2][i] * f1);
+    }
+    pin(G.b[D]);
+    pin(G.mA[D]);
+    pin(E);
+  });
+  pin(el);
+}
+
+// outflow through the scs of directions 0, 1, 2 of local node la
+template <typename R>
+__device__ __forceinline__ void load_mdot3(const double* __restrict__ mdot, const RowElem& r, R (&m3)[3]) {
 #pragma unroll
-        for (int j = 0; j < 3; ++j) unsafeAtomicAdd(row + 3 * j * L + 3 * p + j, lf);
-      } else {
+  for (int d = 0; d < 3; ++d) {
+    const double v = mdot[12 * r.e + hexrow::scs_of(r.la, d)];
+    m3[d] = R(hexrow::scs_is_left(r.la, d) ? v : -v);
+  }
+}
+
+template <bool SKEW, bool SHIFT, bool PACK, typename R, class Emit>
+__device__ __forceinline__ void momentum_row(const MomentumFields& F, RowElem& el, const double (&x)[3][8], const R (&mn)[8],
+                                             double h, double (&rhs)[3], Emit&& emit) {
+  MomentumGeo<R> G;
+  momentum_geometry<SHIFT>(x, mn, h, el, G);
+  R u[3][8], mdot3[3], rr[3] = {R(0), R(0), R(0)};
+  load_mdot3(F.mdot, el, mdot3);
+  load3<PACK>(F.u, el.nd, u);
+  if (F.incl_divu != 0.0) {
+    static_for<3>([&](auto dd) {
+      constexpr int D = decltype(dd)::value;
+      R divu = R(0);
 #pragma unroll
-        for (int j = 0; j < 3; ++j) row[3 * j * L + 3 * p + j] += lf;
+      for (int i = 0; i < 3; ++i) {
+        R du[3];
+        hexrow::param_grad<D, SHIFT>(u[i], du);
+        divu += G.b[D][0][i] * du[0] + G.b[D][1][i] * du[1] + G.b[D][2][i] * du[2];
       }
-    }
-  } else {
-    const double projTimeScale = A.dt / A.g1;
-    rh[0] += -(A.g1 * rs[2] + A.g2 * rs[1] + A.g3 * rs[0]) * scV / A.dt / projTimeScale;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) rr[i] -= R(2.0 / 3.0) * divu * G.mA[D][i] * R(F.incl_divu);
+    });
   }
-}
-
-// ---------------------------------------------------------------- node-tile gather
-// Owner-computes with one thread per (row node, local index): a block owns
-// kTileNodes consecutive rows; thread (node j, slot s) evaluates row s of every
-// element in which node j has local index s (one element on a structured
-// lattice).  The slot is uniform across a wave, so the per-LA code path never
-// diverges.  Contributions accumulate in the LDS copy of the block's CSR
-// segment (LDS FP64 atomics: the 8 slots of a node share its row), which is
-// then written to HBM once, coalesced -- no global atomics, no separate zero pass.
-constexpr int kTileNodes = 64;
-constexpr int kTileThreads = kTileNodes * 8;
-constexpr size_t kMaxLds = 160 * 1024;  // LDS of one gfx950 CU, the most one block can hold
-
-template <class Op>
-__global__ __launch_bounds__(kTileThreads) void k_scalar_tile(Op op, const int32_t* __restrict__ conn,
-                                                              const double* __restrict__ coords,
-                                                              const int32_t* __restrict__ row_node,
-                                                              const int32_t* __restrict__ inc_ptr,
-                                                              const int32_t* __restrict__ inc_elem,
-                                                              const int32_t* __restrict__ nrp,
-                                                              const uint64_t* __restrict__ elem_pos, int64_t nrows,
-                                                              double* __restrict__ vals, double* __restrict__ rhs,
-                                                              int accumulate) {
-  extern __shared__ double seg[];
-  const int64_t r0 = (int64_t)blockIdx.x * kTileNodes;
-  const int64_t r1 = min(r0 + (int64_t)kTileNodes, nrows);
-  const int32_t s0 = nrp[r0], s1 = nrp[r1];
-  const int nseg = s1 - s0;
-  double* rseg = seg + nseg;
-  for (int i = threadIdx.x; i < nseg + kTileNodes; i += blockDim.x) seg[i] = 0.0;
-  __syncthreads();
-  const int slot = __builtin_amdgcn_readfirstlane(threadIdx.x / kTileNodes);  // wave-uniform local index
-  const int j = threadIdx.x % kTileNodes;
-  const int64_t r = r0 + j;
-  if (r < r1) {
-    const int32_t a = row_node ? row_node[r] : (int32_t)r;
-    double* myrow = seg + (nrp[r] - s0);
-    double acc = 0.0;
-    for (int32_t q = inc_ptr[a]; q < inc_ptr[a + 1]; ++q) {
-      const int32_t t = inc_elem[q];
-      if ((t & 7) != slot) continue;
-      const int64_t e = t >> 3;
-      int32_t nd[8];
-      load_nodes(conn, e, nd);
-      typename Op::real x[8][3];
-      load_coords(coords, nd, x);
-      const uint64_t pk = elem_pos[t];
-      acc += (double)dispatch_row(op, slot, nd, x, [&](int c, auto v) {
-        unsafeAtomicAdd(myrow + (int)((pk >> (8 * c)) & 0xff), (double)v);
-      });
-    }
-    if (acc != 0.0) unsafeAtomicAdd(rseg + j, acc);
-  }
-  __syncthreads();
-  if (accumulate) {
-    for (int i = threadIdx.x; i < nseg; i += blockDim.x) vals[s0 + i] += seg[i];
-    for (int i = threadIdx.x; i < r1 - r0; i += blockDim.x) rhs[r0 + i] += rseg[i];
-  } else {
-    for (int i = threadIdx.x; i < nseg; i += blockDim.x) __builtin_nontemporal_store(seg[i], &vals[s0 + i]);
-    for (int i = threadIdx.x; i < r1 - r0; i += blockDim.x) rhs[r0 + i] = rseg[i];
-  }
-}
-
-template <int LA, bool SKEW, bool SHIFT, typename R>
-__device__ __forceinline__ void momentum_row_lds(const int32_t (&nd)[8], const R (&x)[8][3],
-                                                 const double* __restrict__ u, const double* __restrict__ mu,
-                                                 const double* __restrict__ md, double incl_divu, double* myrow,
-                                                 int32_t L, uint64_t pk, double (&rh)[3]) {
-  const hex8::Gather gt{nd};
-  const R m3[3] = {R(md[hex8::adj_ip(LA, 0)]), R(md[hex8::adj_ip(LA, 1)]), R(md[hex8::adj_ip(LA, 2)])};
-  R rr[3] = {R(0), R(0), R(0)};
-  hex8::row_momentum<LA, SKEW, SHIFT, double>(x, gt, u, mu, m3, R(incl_divu), rr, [&](int c, const R (&blk)[3][3]) {
-    const int p = (int)((pk >> (8 * c)) & 0xff);
+  static_for<8>([&](auto mm) {
+    constexpr int m = decltype(mm)::value;
+    R T[3][3], a = R(0);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
-      for (int jj = 0; jj < 3; ++jj) unsafeAtomicAdd(myrow + 3 * i * L + 3 * p + jj, (double)blk[i][jj]);
+      for (int j = 0; j < 3; ++j) T[i][j] = R(0);
+    static_for<3>([&](auto dd) {
+      constexpr int D = decltype(dd)::value;
+      constexpr double s0 = hexrow::scs_slope<D, SHIFT>(m, 0), s1 = hexrow::scs_slope<D, SHIFT>(m, 1),
+                       s2 = hexrow::scs_slope<D, SHIFT>(m, 2), N = hexrow::scs_shape<D, SKEW>(m);
+      if constexpr (s0 != 0.0 || s1 != 0.0 || s2 != 0.0) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          R dn = R(0);
+          if constexpr (s0 != 0.0) dn += R(s0) * G.b[D][0][i];
+          if constexpr (s1 != 0.0) dn += R(s1) * G.b[D][1][i];
+          if constexpr (s2 != 0.0) dn += R(s2) * G.b[D][2][i];
+#pragma unroll
+          for (int j = 0; j < 3; ++j) T[i][j] += dn * G.mA[D][j];
+        }
+      }
+      if constexpr (N != 0.0) a += R(N) * mdot3[D];
+    });
+    a -= T[0][0] + T[1][1] + T[2][2];
+    R blk[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        blk[i][j] = i == j ? a - T[i][j] : -T[i][j];
+        rr[i] -= blk[i][j] * u[j][m];
+      }
+    }
+    emit(m, blk);
+    pin(rr);
+    pin(G.mA);
   });
 #pragma unroll
-  for (int i = 0; i < 3; ++i) rh[i] += (double)rr[i];
+  for (int i = 0; i < 3; ++i) rhs[i] += (double)rr[i];
 }
 
-// Momentum (numDof 3) node-tile gather: the block's segment holds the 3 rows of
-// each of its nodes (rows 3a..3a+2 are contiguous in the CSR).  MASS (1
-// consistent, 2 lumped) adds the momentum mass kernel of the same element and
-// scv in the same pass, as one element algorithm runs its kernel list over an
-// element: one LDS segment, one write of the matrix.
-template <bool SKEW, bool SHIFT, typename R, int MASS = 0>
-__global__ __launch_bounds__(kTileThreads) void k_momentum_tile(
-    const int32_t* __restrict__ conn, const double* __restrict__ coords, const double* __restrict__ u,
-    const double* __restrict__ mu, const double* __restrict__ mdot, double incl_divu,
+// The segregated form: the transpose-gradient term -mu_ip dN_c/dx_i A_j stays on
+// the rhs only, so the three components share the scalar entries am[m].
+template <bool SKEW, bool SHIFT, bool PACK, typename R>
+__device__ __forceinline__ void momentum_row_seg(const MomentumFields& F, RowElem& el, const double (&x)[3][8],
+                                                 const R (&mn)[8], double h, R (&am)[8], double (&rhs)[3]) {
+  MomentumGeo<R> G;
+  momentum_geometry<SHIFT>(x, mn, h, el, G);
+  R u[3][8], mdot3[3], rr[3] = {R(0), R(0), R(0)};
+  load_mdot3(F.mdot, el, mdot3);
+  load3<PACK>(F.u, el.nd, u);
+#pragma unroll
+  for (int m = 0; m < 8; ++m) am[m] = R(0);
+  static_for<3>([&](auto dd) {
+    constexpr int D = decltype(dd)::value;
+    R g[3], divu = R(0), du[3][3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g[k] = G.b[D][k][0] * G.mA[D][0] + G.b[D][k][1] * G.mA[D][1] + G.b[D][k][2] * G.mA[D][2];
+    hexrow::slope<D, SHIFT>(g, [&](int m, R t) { am[m] -= t; });
+    static_for<8>([&](auto mm) {
+      constexpr int m = decltype(mm)::value;
+      constexpr double N = hexrow::scs_shape<D, SKEW>(m);
+      if constexpr (N != 0.0) am[m] += R(N) * mdot3[D];
+    });
+    // mu sum_c dN_c/dx_i (A . u_c) = sum_k b_k,i (du/dt_k . mu A)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) hexrow::param_grad<D, SHIFT>(u[j], du[j]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const R w = du[0][k] * G.mA[D][0] + du[1][k] * G.mA[D][1] + du[2][k] * G.mA[D][2];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        rr[i] += G.b[D][k][i] * w;
+        divu += G.b[D][k][i] * du[i][k];
+      }
+    }
+    if (F.incl_divu != 0.0) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) rr[i] -= R(2.0 / 3.0) * divu * G.mA[D][i] * R(F.incl_divu);
+    }
+    pin(am);
+    pin(rr);
+  });
+#pragma unroll
+  for (int m = 0; m < 8; ++m)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) rr[i] -= am[m] * u[i][m];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) rhs[i] += (double)rr[i];
+}
+
+// Momentum (numDof 3) row tile: a block owns kMomRows consecutive nodes and the LDS
+// copy of their three rows each (rows 3a..3a+2 are contiguous in the CSR; 62 KB for
+// 27-column rows, two blocks to a CU), accumulated with LDS atomics.  Eight threads
+// to a node; the two of one wave take the s-th and the (7-s)-th incident element,
+// opposite corners on a lattice, which share no column but the node's own.  ADV:
+// the advection-diffusion kernel; MASS (0 none, 1 consistent, 2 lumped): the
+// momentum mass kernel of the same element and scv, in the same pass as one
+// element algorithm runs its kernel list.  96^3 with mass: 0.94 ms (2.75 ms for 64
+// nodes to a block, one block to a CU, and eight compile-time local nodes).
+constexpr int kMomRows = 32;
+constexpr int kMomThreads = 8 * kMomRows;
+template <bool ADV, bool SKEW, bool SHIFT, bool PACK, typename R, int MASS>
+__global__ __launch_bounds__(kMomThreads) void k_momentum_rows(
+    MomentumFields F, MassArgs MA, const int32_t* __restrict__ conn,
     const int32_t* __restrict__ row_node, const int32_t* __restrict__ inc_ptr, const int32_t* __restrict__ inc_elem,
-    const int32_t* __restrict__ nrp, const uint64_t* __restrict__ elem_pos, int64_t nnodes,
-    double* __restrict__ vals, double* __restrict__ rhs, int accumulate, MassArgs MA) {
+    const int32_t* __restrict__ nrp, ElemPos elem_pos, int64_t nnodes,
+    double* __restrict__ vals, double* __restrict__ rhs, int accumulate) {
   extern __shared__ double seg[];
-  const int64_t a0 = (int64_t)blockIdx.x * kTileNodes;
-  const int64_t a1 = min(a0 + (int64_t)kTileNodes, nnodes);
-  const int64_t s0 = 9 * (int64_t)nrp[a0], s1 = 9 * (int64_t)nrp[a1];
-  const int nseg = (int)(s1 - s0);
+  const int64_t a0 = (int64_t)blockIdx.x * kMomRows;
+  const int64_t a1 = min(a0 + (int64_t)kMomRows, nnodes);
+  const int64_t s0 = 9 * (int64_t)nrp[a0];
+  const int nseg = (int)(9 * (int64_t)nrp[a1] - s0);
   double* rseg = seg + nseg;
-  for (int i = threadIdx.x; i < nseg + 3 * kTileNodes; i += blockDim.x) seg[i] = 0.0;
+  for (int i = threadIdx.x; i < nseg + 3 * kMomRows; i += kMomThreads) seg[i] = 0.0;
   __syncthreads();
-  const int slot = __builtin_amdgcn_readfirstlane(threadIdx.x / kTileNodes);
-  const int j = threadIdx.x % kTileNodes;
+  const int j = threadIdx.x % kMomRows, wave = threadIdx.x >> 6;
+  const int slot = (threadIdx.x & 32) ? 7 - wave : wave;
   const int64_t r = a0 + j;
   if (r < a1) {
     const int32_t a = row_node ? row_node[r] : (int32_t)r;
-    const int32_t L = nrp[r + 1] - nrp[r];
+    const int32_t L3 = 3 * (nrp[r + 1] - nrp[r]), q1 = inc_ptr[a + 1];
     double* myrow = seg + (9 * (int64_t)nrp[r] - s0);
-    double rh[3] = {0, 0, 0};
-    for (int32_t q = inc_ptr[a]; q < inc_ptr[a + 1]; ++q) {
+    double rh[3] = {0.0, 0.0, 0.0};
+    for (int32_t q = inc_ptr[a] + slot; q < q1; q += 8) {
       const int32_t t = inc_elem[q];
-      if ((t & 7) != slot) continue;
-      const int64_t e = t >> 3;
-      int32_t nd[8];
-      load_nodes(conn, e, nd);
-      R x[8][3];
-      load_coords(coords, nd, x);
-      const uint64_t pk = elem_pos[t];
-      const double* md = mdot + 12 * e;
-      switch (slot) {
-#define NALU_MT(Lx) \
-  case Lx: momentum_row_lds<Lx, SKEW, SHIFT, R>(nd, x, u, mu, md, incl_divu, myrow, L, pk, rh); break;
-        NALU_MT(0) NALU_MT(1) NALU_MT(2) NALU_MT(3) NALU_MT(4) NALU_MT(5) NALU_MT(6) NALU_MT(7)
-#undef NALU_MT
-      }
-      if (MASS) {
-        double xd[8][3];
-        load_vec3(coords, nd, xd);
-        switch (slot) {
-#define NALU_MM(Lx) \
-  case Lx: mass_row<Lx, true, MASS == 2, false, true>(MA, nd, xd, pk, myrow, L, rh); break;
-          NALU_MM(0) NALU_MM(1) NALU_MM(2) NALU_MM(3) NALU_MM(4) NALU_MM(5) NALU_MM(6) NALU_MM(7)
-#undef NALU_MM
+      RowElem el = row_elem(conn, t >> 3, t & 7);
+      const uint64_t pk = hexrow::relative_bytes(elem_pos(t >> 3, t & 7), t & 7);
+      const double h = hexrow::handed(t & 7);
+      double x[3][8], lf = 0.0;
+      R mn[8];
+      load4<PACK, ADV>(F.x, el.nd, x, mn);
+      if constexpr (MASS != 0) lf = momentum_mass_row<MASS == 2, PACK>(MA, el.nd, x, h, rh);
+      if constexpr (ADV) {
+        momentum_row<SKEW, SHIFT, PACK, R>(F, el, x, mn, h, rh, [&](int m, const R (&blk)[3][3]) {
+          double* at = myrow + 3 * hexrow::pos(pk, m);
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int jj = 0; jj < 3; ++jj) {
+              double z = (double)blk[i][jj];
+              if constexpr (MASS != 0)
+                if (i == jj) z += hexrow::scv_shape<MASS == 2>(m) * lf;
+              unsafeAtomicAdd(at + i * L3 + jj, z);
+            }
+        });
+      } else {
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+          if (MASS == 2 && m != 0) continue;
+          double* at = myrow + 3 * hexrow::pos(pk, m);
+#pragma unroll
+          for (int i = 0; i < 3; ++i) unsafeAtomicAdd(at + i * L3 + i, hexrow::scv_shape<MASS == 2>(m) * lf);
         }
       }
     }
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-      if (rh[i] != 0.0) unsafeAtomicAdd(rseg + 3 * j + i, rh[i]);
+    for (int i = 0; i < 3; ++i) unsafeAtomicAdd(rseg + 3 * j + i, rh[i]);
   }
   __syncthreads();
   const int nr = (int)(3 * (a1 - a0));
+  double* out = vals + s0;
   if (accumulate) {
-    for (int i = threadIdx.x; i < nseg; i += blockDim.x) vals[s0 + i] += (double)seg[i];
-    for (int i = threadIdx.x; i < nr; i += blockDim.x) rhs[3 * a0 + i] += (double)rseg[i];
+    for (int i = threadIdx.x; i < nseg; i += kMomThreads) out[i] += seg[i];
+    for (int i = threadIdx.x; i < nr; i += kMomThreads) rhs[3 * a0 + i] += rseg[i];
   } else {
-    for (int i = threadIdx.x; i < nseg; i += blockDim.x) __builtin_nontemporal_store((double)seg[i], &vals[s0 + i]);
-    for (int i = threadIdx.x; i < nr; i += blockDim.x) rhs[3 * a0 + i] = (double)rseg[i];
+    for (int i = threadIdx.x; i < nseg; i += kMomThreads) __builtin_nontemporal_store(seg[i], out + i);
+    for (int i = threadIdx.x; i < nr; i += kMomThreads) rhs[3 * a0 + i] = rseg[i];
   }
-}
-
-// ---------------------------------------------------------------- momentum
-template <int LA, bool SKEW, bool SHIFT, typename R>
-__device__ __forceinline__ void momentum_row_atomic(const int32_t (&nd)[8], const R (&x)[8][3],
-                                                    const double* __restrict__ u, const double* __restrict__ mu,
-                                                    const double* __restrict__ md, double incl_divu,
-                                                    double* __restrict__ rowp, int32_t L, uint64_t pk,
-                                                    double (&rh)[3]) {
-  const hex8::Gather gt{nd};
-  const R m3[3] = {R(md[hex8::adj_ip(LA, 0)]), R(md[hex8::adj_ip(LA, 1)]), R(md[hex8::adj_ip(LA, 2)])};
-  R rr[3] = {R(0), R(0), R(0)};
-  hex8::row_momentum<LA, SKEW, SHIFT, double>(x, gt, u, mu, m3, R(incl_divu), rr, [&](int c, const R (&blk)[3][3]) {
-    const int p = (int)((pk >> (8 * c)) & 0xff);
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) unsafeAtomicAdd(rowp + 3 * i * L + 3 * p + j, (double)blk[i][j]);
-  });
-#pragma unroll
-  for (int i = 0; i < 3; ++i) rh[i] += (double)rr[i];
-}
-
-template <int LA, bool SKEW, bool SHIFT, typename R>
-__device__ __forceinline__ void momentum_body(const int32_t* __restrict__ conn, const double* __restrict__ coords,
-                                              const double* __restrict__ u, const double* __restrict__ mu,
-                                              const double* __restrict__ mdot, double incl_divu,
-                                              const int32_t* __restrict__ lid, const int32_t* __restrict__ nrp,
-                                              const uint64_t* __restrict__ elem_pos, int64_t e,
-                                              double* __restrict__ vals, double* __restrict__ rhs) {
-  int32_t nd[8];
-  load_nodes(conn, e, nd);
-  R x[8][3];
-  load_coords(coords, nd, x);
-  const int32_t nr = lid[nd[LA]];
-  const int32_t nb = nrp[nr];
-  const int32_t L = nrp[nr + 1] - nb;
-  double* rowp = vals + 9 * (int64_t)nb;
-  const uint64_t pk = elem_pos[8 * e + LA];
-  double rh[3] = {0, 0, 0};
-  momentum_row_atomic<LA, SKEW, SHIFT, R>(nd, x, u, mu, mdot + 12 * e, incl_divu, rowp, L, pk, rh);
-#pragma unroll
-  for (int i = 0; i < 3; ++i) unsafeAtomicAdd(rhs + 3 * (int64_t)nr + i, rh[i]);
 }
 
 template <bool SKEW, bool SHIFT, typename R>
 __global__ __launch_bounds__(kChunk) void k_momentum_atomic(
     const int32_t* __restrict__ conn, const double* __restrict__ coords, const double* __restrict__ u,
     const double* __restrict__ mu, const double* __restrict__ mdot, double incl_divu,
-    const int32_t* __restrict__ lid, const int32_t* __restrict__ nrp, const uint64_t* __restrict__ elem_pos,
+    const int32_t* __restrict__ lid, const int32_t* __restrict__ nrp, ElemPos elem_pos,
     int64_t nelem, double* __restrict__ vals, double* __restrict__ rhs) {
   const ChunkMap cm = chunk_map<8>(nelem);
   if (!cm.valid) return;
-  switch (cm.la) {
-#define NALU_MA(L)                                                                                          \
-  case L:                                                                                                   \
-    momentum_body<L, SKEW, SHIFT, R>(conn, coords, u, mu, mdot, incl_divu, lid, nrp, elem_pos, cm.e, vals, rhs); \
-    break;
-    NALU_MA(0) NALU_MA(1) NALU_MA(2) NALU_MA(3) NALU_MA(4) NALU_MA(5) NALU_MA(6) NALU_MA(7)
-#undef NALU_MA
-  }
+  RowElem el = row_elem(conn, cm.e, cm.la);
+  const int32_t nr = lid[el.nd[0]], nb = nrp[nr];
+  const int32_t L3 = 3 * (nrp[nr + 1] - nb);
+  double* rowp = vals + 9 * (int64_t)nb;
+  const uint64_t pk = hexrow::relative_bytes(elem_pos(cm.e, cm.la), cm.la);
+  const MomentumFields F{{{}, coords, mu}, {{}, u, nullptr}, mdot, incl_divu};
+  double x[3][8], rh[3] = {0.0, 0.0, 0.0};
+  R mn[8];
+  load4<false, true>(F.x, el.nd, x, mn);
+  momentum_row<SKEW, SHIFT, false, R>(F, el, x, mn, hexrow::handed(cm.la), rh,
+                               [&](int m, const R (&blk)[3][3]) {
+                                 double* at = rowp + 3 * hexrow::pos(pk, m);
+#pragma unroll
+                                 for (int i = 0; i < 3; ++i)
+#pragma unroll
+                                   for (int j = 0; j < 3; ++j) unsafeAtomicAdd(at + i * L3 + j, (double)blk[i][j]);
+                               });
+#pragma unroll
+  for (int i = 0; i < 3; ++i) unsafeAtomicAdd(rhs + 3 * (int64_t)nr + i, rh[i]);
 }
 
 // ---------------------------------------------------------------- mdot
@@ -560,28 +786,42 @@ __global__ __launch_bounds__(256) void k_mdot_elem(const int32_t* __restrict__ c
                                                    double* __restrict__ mdot) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= nelem) return;
-  int32_t nd[8];
-  load_nodes(conn, e, nd);
-  R x[8][3];
-  load_coords(coords, nd, x);
-  double fr[8], fp[8], fu[8][3], fg[8][3];
+  const RowElem el = row_elem(conn, e, 0);
+  double x[3][8];
+  R pn[8], W[3][8];
+  load4<false, true>(Field4<>{{}, coords, p}, el.nd, x, pn);
+  {
+    R rn[8], un[3][8], gn[3][8];
+    load4<false, true>(Field4<>{{}, u, rho}, el.nd, un, rn);
+    load3<false>(Field4<>{{}, gp, nullptr}, el.nd, gn);
 #pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const int64_t a = nd[c];
-    fr[c] = rho[a];
-    fp[c] = p[a];
+    for (int i = 0; i < 3; ++i)
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      fu[c][j] = u[3 * a + j];
-      fg[c][j] = gp[3 * a + j];
-    }
+      for (int m = 0; m < 8; ++m) W[i][m] = rn[m] * un[i][m] + R(tau) * gn[i][m];
   }
+  hexrow::Edges E;
+  hexrow::edges(x, E);
   double out[12];
-  hex8::static_for<12>([&](auto ii) {
+  static_for<12>([&](auto ii) {
+    // direction and quadrant of the scs; the area vector points to the far side
+    // along D, which is its right node's except for scs 2 and 6
     constexpr int IP = decltype(ii)::value;
-    hex8::IpGeo<double, R> G;
-    hex8::ip_geo<IP, SHIFT_POISSON>(x, G);
-    out[IP] = (double)hex8::ip_mdot_regs<IP, SHIFT_MDOT, SHIFT_POISSON>(G, fr, fp, fu, fg, R(tau));
+    constexpr int D = IP >= 8 ? 2 : (IP & 1), c = hex8::scs_left(IP);
+    constexpr int bits = hexrow::hex_of(c);
+    constexpr int QE = (bits >> (D + 1) % 3) & 1, QF = (bits >> (D + 2) % 3) & 1;
+    constexpr double sign = ((bits >> D) & 1) ? -1.0 : 1.0;
+    double A[3];
+    hexrow::Cof K;
+    hexrow::area_cofactors<D, SHIFT_POISSON, QE, QF>(E, sign, A, K);
+    R g[3], ps[3];
+    hexrow::metric<SHIFT_POISSON>(K, A, g);
+    hexrow::param_grad<D, SHIFT_POISSON, QE, QF>(pn, ps);
+    R f = -R(tau) * (ps[0] * g[0] + ps[1] * g[1] + ps[2] * g[2]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) f += hexrow::at_scs<D, SHIFT_MDOT, QE, QF>(W[i]) * R(A[i]);
+    out[IP] = (double)f;
+    pin(out[IP]);
+    pin(E);
   });
   double2* o = reinterpret_cast<double2*>(mdot + 12 * e);
 #pragma unroll
@@ -592,7 +832,7 @@ __global__ __launch_bounds__(256) void k_mdot_elem(const int32_t* __restrict__ c
 // Batched sumInto of caller-provided dense element matrices.
 __global__ void k_sum_into_batch(const int32_t* __restrict__ conn, const double* __restrict__ lhs,
                                  const double* __restrict__ rhs_e, const int32_t* __restrict__ lid,
-                                 const int32_t* __restrict__ nrp, const uint64_t* __restrict__ elem_pos,
+                                 const int32_t* __restrict__ nrp, ElemPos elem_pos,
                                  int64_t nelem, int nd, double* __restrict__ vals, double* __restrict__ rhs) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;  // (element, row node, dof)
   if (t >= nelem * 8 * nd) return;
@@ -603,7 +843,7 @@ __global__ void k_sum_into_batch(const int32_t* __restrict__ conn, const double*
   const int32_t nr = lid[conn[8 * e + a]];
   const int32_t nb = nrp[nr];
   const int32_t L = nrp[nr + 1] - nb;
-  const uint64_t pk = elem_pos[8 * e + a];
+  const uint64_t pk = elem_pos(e, a);
   const double* lrow = lhs + (e * R + (int64_t)(a * nd + d)) * R;
   double* rowp = vals + (int64_t)nd * nd * nb + (int64_t)d * nd * L;
   for (int c = 0; c < 8; ++c) {
@@ -635,44 +875,90 @@ __global__ void k_dirichlet(const int32_t* __restrict__ nodes, int64_t nbc, int6
   rhs[row] = reset_mode ? rhs_residual : bcv[(int64_t)nd * node + d] - sol[(int64_t)nd * node + d];
 }
 
-// rows (threads) per block of the row gather (128^3 continuity: 1.31 ms at
-// 256, 1.34 ms at 64, 1.40 ms at 128)
-int gather_rows() { return 256; }
+inline size_t lds_rows(const nalu_linsys* ls) {
+  return (size_t)kRowsPerBlock * ls->max_node_row_len * sizeof(double);
+}
+
+// From this many nodes on, a row pass copies its fields first (below, the copy's
+// launch costs what it saves); past 2^28 nodes the 32-bit offsets end.
+constexpr int64_t kPackNodes = 1 << 15;
+bool use_pack(const nalu_linsys* ls) { return ls->num_nodes >= kPackNodes && ls->num_nodes < ((int64_t)1 << 28); }
+
+// Copies the fields f[0..n) to 16-byte halves (on ls->stream) and points their h at them.
+void pack_fields(nalu_linsys* ls, Field4<>* const* f, int n) {
+  const int64_t N = ls->num_nodes;
+  auto* ws = reinterpret_cast<Half<double>*>(ensure_ws(ls->pack_ws, 2 * n * N * sizeof(Half<double>)));
+  PackList L{};
+  for (L.n = 0; L.n < n; ++L.n) {
+    L.vec[L.n] = f[L.n]->vec;
+    L.scal[L.n] = f[L.n]->scal;
+    f[L.n]->h[0] = ws + 2 * L.n * N;
+    f[L.n]->h[1] = ws + (2 * L.n + 1) * N;
+  }
+  hipLaunchKernelGGL(k_pack, dim3(blocks_for(N, 256)), dim3(256), 0, ls->stream, L, N, ws);
+}
 
 template <class Op>
-void launch_scalar(nalu_linsys* ls, const nalu_mesh* m, const Op& op, int mode) {
+void launch_scalar_rows(nalu_linsys* ls, const nalu_mesh* m, const Op& op) {
   hipStream_t s = ls->stream;
-  const int64_t E = m->num_elems;
-  if (mode == 0) {
-    build_node_incidence(const_cast<nalu_mesh*>(m), s);
-    const int accumulate = ls->values_pending_zero ? 0 : 1;
-    NALU_REQUIRE(ls->values_pending_zero == ls->rhs_pending_zero, NALU_ERR_STATE,
-                 "gather assembly: values/rhs zero state diverged");
-    const size_t esz = sizeof(double);
-    int B = gather_rows();
-    while (B > 32 && (size_t)B * ls->max_node_row_len * esz > 64 * 1024) B >>= 1;
-    const size_t lds = (size_t)B * ls->max_node_row_len * esz;
-    hipLaunchKernelGGL((k_scalar_gather<Op>), dim3(blocks_for(ls->nrows, B)), dim3(B), lds, s, op, m->conn.p,
-                       m->coords.p, (const int32_t*)ls->row_node.p, m->inc_ptr.p, m->inc_elem.p, ls->nrp.p,
-                       ls->elem_pos.p, ls->nrows, ls->values.p, ls->rhs.p, accumulate);
-    ls->values_pending_zero = ls->rhs_pending_zero = false;
-  } else if (mode == 2) {
-    build_node_incidence(const_cast<nalu_mesh*>(m), s);
-    NALU_REQUIRE(ls->values_pending_zero == ls->rhs_pending_zero, NALU_ERR_STATE,
-                 "tile assembly: values/rhs zero state diverged");
-    const int accumulate = ls->values_pending_zero ? 0 : 1;
-    const size_t lds = ((size_t)kTileNodes * ls->max_node_row_len + kTileNodes) * sizeof(double);
-    set_lds_limit((const void*)k_scalar_tile<Op>, lds);
-    hipLaunchKernelGGL((k_scalar_tile<Op>), dim3(blocks_for(ls->nrows, kTileNodes)), dim3(kTileThreads), lds, s, op,
-                       m->conn.p, m->coords.p, (const int32_t*)ls->row_node.p, m->inc_ptr.p, m->inc_elem.p,
-                       ls->nrp.p, ls->elem_pos.p, ls->nrows, ls->values.p, ls->rhs.p, accumulate);
-    ls->values_pending_zero = ls->rhs_pending_zero = false;
-  } else {
-    materialize_pending_zero(ls);
-    hipLaunchKernelGGL((k_scalar_atomic<Op>), dim3(chunk_blocks<8>(E)), dim3(kChunk), 0, s, op, m->conn.p,
-                       m->coords.p, ls->node_lid.p, ls->nrp.p, ls->elem_pos.p, E, ls->values.p, ls->rhs.p);
-  }
+  build_node_incidence(const_cast<nalu_mesh*>(m), s);
+  const int accumulate = ls->values_pending_zero ? 0 : 1;
+  NALU_REQUIRE(ls->values_pending_zero == ls->rhs_pending_zero, NALU_ERR_STATE,
+               "row-tile assembly: values/rhs zero state diverged");
+  const size_t lds = lds_rows(ls);
+  set_lds_limit((const void*)k_scalar_rows<Op>, lds);
+  hipLaunchKernelGGL((k_scalar_rows<Op>), dim3(blocks_for(ls->nrows, kRowsPerBlock)), dim3(kRowThreads), lds, s, op,
+                     m->conn.p, (const int32_t*)ls->row_node.p, m->inc_ptr.p, m->inc_elem.p, ls->nrp.p,
+                     elem_pos_of(ls), ls->nrows, ls->max_node_row_len, op.rhs_scale(), ls->values.p, ls->rhs.p,
+                     accumulate);
+  ls->values_pending_zero = ls->rhs_pending_zero = false;
   NALU_HIP_CHECK(hipGetLastError());
+}
+
+template <class Op>
+void launch_scalar_atomic(nalu_linsys* ls, const nalu_mesh* m, const Op& op) {
+  const int64_t E = m->num_elems;
+  materialize_pending_zero(ls);
+  hipLaunchKernelGGL((k_scalar_atomic<Op>), dim3(chunk_blocks<8>(E)), dim3(kChunk), 0, ls->stream, op, m->conn.p,
+                     ls->node_lid.p, ls->nrp.p, elem_pos_of(ls), E, op.rhs_scale(), ls->values.p, ls->rhs.p);
+  NALU_HIP_CHECK(hipGetLastError());
+}
+
+// Modes 0 ("gather") and 2 ("tile") run the row tile; mode 1 the atomic scatter.
+template <bool SHIFT, typename R>
+void scalar_diff_pass(nalu_linsys* ls, const nalu_mesh* m, const double* q, const double* k, int mode) {
+  Field4<> xk{{}, m->coords.p, k};
+  if (mode == 1) {
+    launch_scalar_atomic(ls, m, ScalarDiffOp<SHIFT, false, R>{xk, q});
+  } else if (use_pack(ls)) {
+    Field4<>* const f[] = {&xk};
+    pack_fields(ls, f, 1);
+    launch_scalar_rows(ls, m, ScalarDiffOp<SHIFT, true, R>{xk, q});
+  } else {
+    launch_scalar_rows(ls, m, ScalarDiffOp<SHIFT, false, R>{xk, q});
+  }
+}
+
+template <bool SM, bool SP, bool RED, bool MDOT, typename R>
+void continuity_pass(nalu_linsys* ls, const nalu_mesh* m, const double* rho, const double* p, const double* u,
+                     const double* gp, double tau, int mode, double* mdot) {
+  const Field4<> xp{{}, m->coords.p, p}, ur{{}, u, rho};
+  if (mode == 1) {
+    if constexpr (!MDOT)
+      launch_scalar_atomic(ls, m, ContinuityOp<SM, SP, RED, false, false, R>{xp, {}, ur, gp, tau, nullptr});
+  } else if (use_pack(ls)) {
+    const int64_t N = ls->num_nodes;
+    constexpr int nw = sizeof(R) == 8 ? 2 : 1;
+    auto* xs = reinterpret_cast<Half<double>*>(ensure_ws(ls->pack_ws, (2 + nw) * N * 16));
+    auto* W = reinterpret_cast<Half<R>*>(xs + 2 * N);
+    hipLaunchKernelGGL(k_pack_flux<R>, dim3(blocks_for(N, 256)), dim3(256), 0, ls->stream, m->coords.p, p, rho, u, gp,
+                       tau, N, xs, W);
+    const Field4<> xh{{xs, xs + N}, nullptr, nullptr};
+    const Field4<R> Wh{{W, nw == 2 ? W + N : nullptr}, nullptr, nullptr};
+    launch_scalar_rows(ls, m, ContinuityOp<SM, SP, RED, MDOT, true, R>{xh, Wh, {}, nullptr, tau, mdot});
+  } else {
+    launch_scalar_rows(ls, m, ContinuityOp<SM, SP, RED, MDOT, false, R>{xp, {}, ur, gp, tau, mdot});
+  }
 }
 
 // Systems created for the mixed-precision path assemble with FP32 arithmetic.
@@ -705,254 +991,188 @@ void check_flag(DevBuf<int>& flag, hipStream_t s, const char* msg) {
 // ---------------------------------------------------------------- kernel-input producers
 // Dual nodal volume (ComputeGeometryInteriorAlgorithm, src/ComputeGeometryInteriorAlgorithm.C:77-120)
 // and the interior Green-Gauss nodal gradient (AssembleNodalGradElemAlgorithm,
-// src/AssembleNodalGradElemAlgorithm.C:85-140), owner-computes: one thread per
-// node walks its incident elements; the node's scv (ip = its local index) and
-// its three adjacent scs (sign +1 where it is the left node) are all that
-// touch it, so every result is written once, with no atomics.
-__global__ __launch_bounds__(256) void k_dual_volume(const int32_t* __restrict__ conn,
-                                                     const double* __restrict__ coords,
-                                                     const int32_t* __restrict__ inc_ptr,
-                                                     const int32_t* __restrict__ inc_elem, int64_t nnodes,
-                                                     double* __restrict__ vol) {
-  const int64_t a = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= nnodes) return;
-  double v = 0.0;
-  for (int32_t q = inc_ptr[a]; q < inc_ptr[a + 1]; ++q) {
+// src/AssembleNodalGradElemAlgorithm.C:85-140), owner-computes: the node's scv and
+// its three adjacent scs are all that touch it.  Eight lanes per node take its
+// incident elements (as in k_scalar_rows), every result is written once.
+template <int NC, class Eval, class Store>
+__device__ __forceinline__ void node_sums(const int32_t* __restrict__ conn, const int32_t* __restrict__ inc_ptr,
+                                          const int32_t* __restrict__ inc_elem, int64_t nnodes, Eval&& eval,
+                                          Store&& store) {
+  const WaveRows w = wave_rows(nullptr, inc_ptr, nnodes);
+  double v[NC];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) v[i] = 0.0;
+  for (int32_t q = w.q; q < w.q1; q += kSlots) {
     const int32_t t = inc_elem[q];
-    int32_t nd[8];
-    load_nodes(conn, t >> 3, nd);
-    double x[8][3];
-    load_vec3(coords, nd, x);
-    switch (t & 7) {
-#define NALU_DV(Lx) \
-  case Lx: v += hex8::scv_volume<Lx>(x); break;
-      NALU_DV(0) NALU_DV(1) NALU_DV(2) NALU_DV(3) NALU_DV(4) NALU_DV(5) NALU_DV(6) NALU_DV(7)
-#undef NALU_DV
-    }
+    eval(row_elem(conn, t >> 3, t & 7), v);
   }
-  vol[a] = v;
+#pragma unroll
+  for (int i = 0; i < NC; ++i) v[i] = row_sum(v[i]);
+  if (w.slot == 0 && w.r < w.r1) store(w.r, v);
 }
 
-template <int LA, bool SHIFT>
-__device__ __forceinline__ void nodal_grad_part(const double (&x)[8][3], const int32_t (&nd)[8],
-                                                const double* __restrict__ qf, double (&g)[3]) {
-  hex8::static_for<3>([&](auto kk) {
-    constexpr int IP = hex8::adj_ip(LA, decltype(kk)::value);
-    constexpr double S = hex8::adj_sign(LA, decltype(kk)::value);
-    double A[3];
-    hex8::scs_area<IP>(x, A);
-    double qIp = 0.0;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) qIp += hex8::kScsTab.shape[SHIFT][IP][c] * qf[nd[c]];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) g[j] += S * (qIp * A[j]);
-  });
+__global__ __launch_bounds__(kRowThreads) void k_dual_volume(const int32_t* __restrict__ conn,
+                                                              const double* __restrict__ coords,
+                                                              const int32_t* __restrict__ inc_ptr,
+                                                              const int32_t* __restrict__ inc_elem, int64_t nnodes,
+                                                              double* __restrict__ vol) {
+  node_sums<1>(
+      conn, inc_ptr, inc_elem, nnodes,
+      [&](const RowElem& el, double (&v)[1]) {
+        double x[3][8];
+        load3<false>(Field4<>{{}, coords, nullptr}, el.nd, x);
+        v[0] += hexrow::scv_volume(x, hexrow::handed(el.la));
+      },
+      [&](int64_t a, const double (&v)[1]) { vol[a] = v[0]; });
 }
 
 template <bool SHIFT>
-__global__ __launch_bounds__(256) void k_nodal_grad(const int32_t* __restrict__ conn,
-                                                    const double* __restrict__ coords, const double* __restrict__ qf,
-                                                    const double* __restrict__ vol,
-                                                    const int32_t* __restrict__ inc_ptr,
-                                                    const int32_t* __restrict__ inc_elem, int64_t nnodes,
-                                                    double* __restrict__ dqdx) {
-  const int64_t a = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= nnodes) return;
-  double g[3] = {0.0, 0.0, 0.0};
-  for (int32_t q = inc_ptr[a]; q < inc_ptr[a + 1]; ++q) {
-    const int32_t t = inc_elem[q];
-    int32_t nd[8];
-    load_nodes(conn, t >> 3, nd);
-    double x[8][3];
-    load_vec3(coords, nd, x);
-    switch (t & 7) {
-#define NALU_NG(Lx) \
-  case Lx: nodal_grad_part<Lx, SHIFT>(x, nd, qf, g); break;
-      NALU_NG(0) NALU_NG(1) NALU_NG(2) NALU_NG(3) NALU_NG(4) NALU_NG(5) NALU_NG(6) NALU_NG(7)
-#undef NALU_NG
-    }
-  }
-  const double inv = 1.0 / vol[a];
+__global__ __launch_bounds__(kRowThreads) void k_nodal_grad(const int32_t* __restrict__ conn,
+                                                             const double* __restrict__ coords,
+                                                             const double* __restrict__ qf,
+                                                             const double* __restrict__ vol,
+                                                             const int32_t* __restrict__ inc_ptr,
+                                                             const int32_t* __restrict__ inc_elem, int64_t nnodes,
+                                                             double* __restrict__ dqdx) {
+  node_sums<3>(
+      conn, inc_ptr, inc_elem, nnodes,
+      [&](const RowElem& el, double (&v)[3]) {
+        double x[3][8], q[8];
+        load4<false, true>(Field4<>{{}, coords, qf}, el.nd, x, q);
+        hexrow::Edges E;
+        hexrow::edges(x, E);
+        const double h = hexrow::handed(el.la);
+        static_for<3>([&](auto dd) {
+          constexpr int D = decltype(dd)::value;
+          double A[3];
+          hexrow::area<D>(E, h, A);
+          const double qi = hexrow::at_scs<D, SHIFT>(q);
 #pragma unroll
-  for (int j = 0; j < 3; ++j) dqdx[3 * a + j] = g[j] * inv;
+          for (int i = 0; i < 3; ++i) v[i] += qi * A[i];
+        });
+      },
+      [&](int64_t a, const double (&v)[3]) {
+        const double inv = 1.0 / vol[a];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) dqdx[3 * a + i] = v[i] * inv;
+      });
 }
 
 // ---------------------------------------------------------------- segregated momentum
 // Momentum as three right-hand sides sharing one scalar matrix: the coupled
 // MomentumAdvDiffElemKernel (src/kernel/MomentumAdvDiffElemKernel.C:72-186) with
 // the transpose-gradient stress coupling kept on the rhs only (the rhs is the
-// full residual, so converged velocities are unchanged).  Owner-computes row
-// gather on a numDof 1 graph: the row segment accumulates in LDS, the three
-// residual components go to rhs3[i][row].
-template <bool SKEW, bool SHIFT, typename R, int MASS = 0>
-__global__ __launch_bounds__(256) void k_momentum_seg_gather(
-    const int32_t* __restrict__ conn, const double* __restrict__ coords, const double* __restrict__ u,
-    const double* __restrict__ mu, const double* __restrict__ mdot, double incl_divu,
+// full residual, so converged velocities are unchanged).  Row tile on a numDof 1
+// graph as k_scalar_rows, with the three residual components in rhs3[i][row].
+// ADV, MASS as in k_momentum_rows.
+template <bool ADV, bool SKEW, bool SHIFT, bool PACK, typename R, int MASS>
+__global__ __launch_bounds__(kRowThreads) void k_momentum_seg_rows(
+    MomentumFields F, MassArgs MA, const int32_t* __restrict__ conn,
     const int32_t* __restrict__ row_node, const int32_t* __restrict__ inc_ptr, const int32_t* __restrict__ inc_elem,
-    const int32_t* __restrict__ nrp, const uint64_t* __restrict__ elem_pos, int64_t nrows,
-    double* __restrict__ vals, double* __restrict__ rhs3, int accumulate, MassArgs MA) {
-  extern __shared__ double seg[];
-  const int64_t r0 = (int64_t)blockIdx.x * blockDim.x;
-  const int64_t rend = min(r0 + (int64_t)blockDim.x, nrows);
-  const int64_t r = r0 + threadIdx.x;
-  const int32_t s0 = nrp[r0], s1 = nrp[rend];
-  const int nseg = s1 - s0;
-  for (int i = threadIdx.x; i < nseg; i += blockDim.x) seg[i] = 0.0;
-  __syncthreads();
-  double rr[3] = {0.0, 0.0, 0.0};
-  if (r < nrows) {
-    const int32_t a = row_node ? row_node[r] : (int32_t)r;
-    double* myrow = seg + (nrp[r] - s0);
-    for (int32_t q = inc_ptr[a]; q < inc_ptr[a + 1]; ++q) {
+    const int32_t* __restrict__ nrp, ElemPos elem_pos, int64_t nrows, int row_len,
+    double* __restrict__ vals, double* __restrict__ rhs3, int accumulate) {
+  extern __shared__ double seg_all[];
+  double* seg = seg_all + (size_t)(threadIdx.x >> 6) * kRowsPerWave * row_len;
+  const WaveRows w = wave_rows(row_node, inc_ptr, nrows);
+  if (w.r0 >= nrows) return;
+  const int32_t s0 = nrp[w.r0];
+  const int nseg = nrp[w.r1] - s0;
+  for (int i = w.lane; i < nseg; i += 64) seg[i] = 0.0;
+  wave_sync();
+  double rh[3] = {0.0, 0.0, 0.0};
+  if (w.q < w.q1) {
+    double* myrow = seg + (nrp[w.r] - s0);
+    for (int32_t q = w.q; q < w.q1; q += kSlots) {
       const int32_t t = inc_elem[q];
-      const int64_t e = t >> 3;
-      int32_t nd[8];
-      load_nodes(conn, e, nd);
-      R x[8][3];
-      load_coords(coords, nd, x);
-      const uint64_t pk = elem_pos[t];
-      const double* md = mdot + 12 * e;
-      const hex8::Gather gt{nd};
-      auto emit = [&](int c, const R (&blk)[3][3]) { myrow[(int)((pk >> (8 * c)) & 0xff)] += (double)blk[0][0]; };
-      R rl[3] = {R(0), R(0), R(0)};
-      switch (t & 7) {
-#define NALU_SG(Lx)                                                                                           \
-  case Lx: {                                                                                                  \
-    const R m3[3] = {R(md[hex8::adj_ip(Lx, 0)]), R(md[hex8::adj_ip(Lx, 1)]), R(md[hex8::adj_ip(Lx, 2)])};    \
-    hex8::row_momentum<Lx, SKEW, SHIFT, double, true>(x, gt, u, mu, m3, R(incl_divu), rl, emit);              \
-  } break;
-        NALU_SG(0) NALU_SG(1) NALU_SG(2) NALU_SG(3) NALU_SG(4) NALU_SG(5) NALU_SG(6) NALU_SG(7)
-#undef NALU_SG
+      RowElem el = row_elem(conn, t >> 3, t & 7);
+      const uint64_t pk = hexrow::relative_bytes(elem_pos(t >> 3, t & 7), t & 7);
+      const double h = hexrow::handed(t & 7);
+      double x[3][8], v[8], lf = 0.0;
+      R mn[8];
+      load4<PACK, ADV>(F.x, el.nd, x, mn);
+      if constexpr (MASS != 0) lf = momentum_mass_row<MASS == 2, PACK>(MA, el.nd, x, h, rh);
+      if constexpr (ADV) {
+        R am[8];
+        momentum_row_seg<SKEW, SHIFT, PACK, R>(F, el, x, mn, h, am, rh);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) v[m] = (double)am[m];
+      } else {
+#pragma unroll
+        for (int m = 0; m < 8; ++m) v[m] = 0.0;
+      }
+      if constexpr (MASS != 0) {
+#pragma unroll
+        for (int m = 0; m < 8; ++m) v[m] += hexrow::scv_shape<MASS == 2>(m) * lf;
       }
 #pragma unroll
-      for (int i = 0; i < 3; ++i) rr[i] += (double)rl[i];
-      if (MASS) {  // the momentum mass kernel of the same element and scv (MASS 1 consistent, 2 lumped)
-        double xd[8][3];
-        load_vec3(coords, nd, xd);
-        switch (t & 7) {
-#define NALU_SM(Lx) \
-  case Lx: mass_row<Lx, true, MASS == 2, true>(MA, nd, xd, pk, myrow, 0, rr); break;
-          NALU_SM(0) NALU_SM(1) NALU_SM(2) NALU_SM(3) NALU_SM(4) NALU_SM(5) NALU_SM(6) NALU_SM(7)
-#undef NALU_SM
-        }
-      }
+      for (int m = 0; m < 8; ++m) unsafeAtomicAdd(myrow + hexrow::pos(pk, m), v[m]);
     }
   }
-  __syncthreads();
-  if (accumulate) {
-    for (int i = threadIdx.x; i < nseg; i += blockDim.x) vals[s0 + i] += seg[i];
-  } else {
-    for (int i = threadIdx.x; i < nseg; i += blockDim.x) __builtin_nontemporal_store(seg[i], &vals[s0 + i]);
-  }
-  if (r < nrows) {
 #pragma unroll
-    for (int i = 0; i < 3; ++i) rhs3[i * nrows + r] += rr[i];
+  for (int i = 0; i < 3; ++i) rh[i] = row_sum(rh[i]);
+  wave_sync();
+  double* out = vals + s0;
+  if (accumulate) {
+    for (int i = w.lane; i < nseg; i += 64) out[i] += seg[i];
+  } else {
+    for (int i = w.lane; i < nseg; i += 64) __builtin_nontemporal_store(seg[i], out + i);
   }
+  // lanes 0, 1, 2 of a row add its three residual components
+  const double rr = w.slot == 0 ? rh[0] : w.slot == 1 ? rh[1] : rh[2];
+  if (w.slot < 3 && w.r < w.r1) rhs3[w.slot * nrows + w.r] += rr;
 }
 
-template <bool MOM, bool LUMPED, bool SEG>
+// ContinuityMassElemKernel (rhs only), and the momentum mass of numDof 3 rows too
+// long for a row tile (added to the matrix in place): one thread per row.
+template <bool MOM, bool LUMPED>
 __global__ __launch_bounds__(256) void k_mass_gather(MassArgs A, const int32_t* __restrict__ conn,
                                                      const double* __restrict__ coords,
                                                      const int32_t* __restrict__ row_node,
                                                      const int32_t* __restrict__ inc_ptr,
                                                      const int32_t* __restrict__ inc_elem,
                                                      const int32_t* __restrict__ nrp,
-                                                     const uint64_t* __restrict__ elem_pos, int64_t nnodes,
+                                                     ElemPos elem_pos, int64_t nnodes,
                                                      double* __restrict__ vals, double* __restrict__ rhs) {
   const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= nnodes) return;
   const int32_t a = row_node ? row_node[r] : (int32_t)r;
-  const int32_t L = nrp[r + 1] - nrp[r];
-  double* row = vals + (MOM && !SEG ? 9 : 1) * (int64_t)nrp[r];
+  const int32_t q1 = inc_ptr[a + 1];
   double rh[3] = {0.0, 0.0, 0.0};
-  for (int32_t q = inc_ptr[a]; q < inc_ptr[a + 1]; ++q) {
+  for (int32_t q = inc_ptr[a]; q < q1; ++q) {
     const int32_t t = inc_elem[q];
-    const int64_t e = t >> 3;
-    int32_t nd[8];
-    load_nodes(conn, e, nd);
-    double x[8][3];
-    load_vec3(coords, nd, x);
-    const uint64_t pk = elem_pos[t];
-    switch (t & 7) {
-#define NALU_MS(Lx) \
-  case Lx: mass_row<Lx, MOM, LUMPED, SEG>(A, nd, x, pk, row, L, rh); break;
-      NALU_MS(0) NALU_MS(1) NALU_MS(2) NALU_MS(3) NALU_MS(4) NALU_MS(5) NALU_MS(6) NALU_MS(7)
-#undef NALU_MS
+    const RowElem el = row_elem(conn, t >> 3, t & 7);
+    const double h = hexrow::handed(t & 7);
+    double x[3][8];
+    load3<false>(Field4<>{{}, coords, nullptr}, el.nd, x);
+    if constexpr (MOM) {
+      const uint64_t pk = hexrow::relative_bytes(elem_pos(t >> 3, t & 7), t & 7);
+      const int32_t L3 = 3 * (nrp[r + 1] - nrp[r]);
+      double* row = vals + 9 * (int64_t)nrp[r];
+      const double lf = momentum_mass_row<LUMPED, false>(A, el.nd, x, h, rh);
+#pragma unroll
+      for (int m = 0; m < 8; ++m) {
+        if (LUMPED && m != 0) continue;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) row[i * L3 + 3 * hexrow::pos(pk, m) + i] += hexrow::scv_shape<LUMPED>(m) * lf;
+      }
+    } else {
+      double s = 0.0;
+      const double g[3] = {A.g3, A.g2, A.g1};
+#pragma unroll
+      for (int st = 0; st < 3; ++st) {
+        double f[8];
+        load1<false>(A.s[st].scal, el.nd, f);
+        s += g[st] * hexrow::at_scv<LUMPED>(f);
+      }
+      const double proj_time_scale = A.dt / A.g1;
+      rh[0] -= s * hexrow::scv_volume(x, h) / A.dt / proj_time_scale;
     }
   }
-  if (MOM && SEG) {
+  if (MOM) {
 #pragma unroll
-    for (int j = 0; j < 3; ++j) rhs[j * nnodes + r] += rh[j];
-  } else if (MOM) {
-#pragma unroll
-    for (int j = 0; j < 3; ++j) rhs[3 * r + j] += rh[j];
+    for (int i = 0; i < 3; ++i) rhs[3 * r + i] += rh[i];
   } else {
     rhs[r] += rh[0];
-  }
-}
-
-// Momentum mass (numDof 3) as a node tile, the structure of k_momentum_tile:
-// a block owns kTileNodes consecutive rows; thread (node j, slot s) adds the
-// sub-control volume of local node s of each element in which node j has local
-// index s (the 3x3 blocks' diagonal entries, LDS atomics: the 8 slots share
-// the row), and the block adds its LDS segment to the matrix in one coalesced
-// pass -- or stores it, folding a pending zeroSystem.  Replaces the
-// thread-per-row form, whose scattered read-modify-writes of 81 diagonal
-// entries per row went to HBM one 8-byte value at a time.
-template <bool LUMPED>
-__global__ __launch_bounds__(kTileThreads) void k_mass_tile3(MassArgs A, const int32_t* __restrict__ conn,
-                                                             const double* __restrict__ coords,
-                                                             const int32_t* __restrict__ row_node,
-                                                             const int32_t* __restrict__ inc_ptr,
-                                                             const int32_t* __restrict__ inc_elem,
-                                                             const int32_t* __restrict__ nrp,
-                                                             const uint64_t* __restrict__ elem_pos, int64_t nnodes,
-                                                             double* __restrict__ vals, double* __restrict__ rhs,
-                                                             int accumulate) {
-  extern __shared__ double seg[];
-  const int64_t a0 = (int64_t)blockIdx.x * kTileNodes;
-  const int64_t a1 = min(a0 + (int64_t)kTileNodes, nnodes);
-  const int64_t s0 = 9 * (int64_t)nrp[a0], s1 = 9 * (int64_t)nrp[a1];
-  const int nseg = (int)(s1 - s0);
-  double* rseg = seg + nseg;
-  for (int i = threadIdx.x; i < nseg + 3 * kTileNodes; i += blockDim.x) seg[i] = 0.0;
-  __syncthreads();
-  const int slot = __builtin_amdgcn_readfirstlane(threadIdx.x / kTileNodes);
-  const int j = threadIdx.x % kTileNodes;
-  const int64_t r = a0 + j;
-  if (r < a1) {
-    const int32_t a = row_node ? row_node[r] : (int32_t)r;
-    const int32_t L = nrp[r + 1] - nrp[r];
-    double* myrow = seg + (9 * (int64_t)nrp[r] - s0);
-    double rh[3] = {0.0, 0.0, 0.0};
-    for (int32_t q = inc_ptr[a]; q < inc_ptr[a + 1]; ++q) {
-      const int32_t t = inc_elem[q];
-      if ((t & 7) != slot) continue;
-      const int64_t e = t >> 3;
-      int32_t nd[8];
-      load_nodes(conn, e, nd);
-      double x[8][3];
-      load_vec3(coords, nd, x);
-      const uint64_t pk = elem_pos[t];
-      switch (slot) {
-#define NALU_MS(Lx) \
-  case Lx: mass_row<Lx, true, LUMPED, false, true>(A, nd, x, pk, myrow, L, rh); break;
-        NALU_MS(0) NALU_MS(1) NALU_MS(2) NALU_MS(3) NALU_MS(4) NALU_MS(5) NALU_MS(6) NALU_MS(7)
-#undef NALU_MS
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-      if (rh[i] != 0.0) unsafeAtomicAdd(rseg + 3 * j + i, rh[i]);
-  }
-  __syncthreads();
-  const int nr = (int)(3 * (a1 - a0));
-  if (accumulate) {
-    for (int i = threadIdx.x; i < nseg; i += blockDim.x) vals[s0 + i] += seg[i];
-    for (int i = threadIdx.x; i < nr; i += blockDim.x) rhs[3 * a0 + i] += rseg[i];
-  } else {
-    for (int i = threadIdx.x; i < nseg; i += blockDim.x) __builtin_nontemporal_store(seg[i], &vals[s0 + i]);
-    for (int i = threadIdx.x; i < nr; i += blockDim.x) rhs[3 * a0 + i] = rseg[i];
   }
 }
 
@@ -1002,11 +1222,9 @@ extern "C" int nalu_assemble_scalar_diff(nalu_linsys* ls, const nalu_mesh* m, co
     if (mode == 3) {
       etile_scalar_diff(ls, m, q, k, shifted != 0, fp32_assembly(ls));
     } else if (fp32_assembly(ls)) {
-      if (shifted) launch_scalar(ls, m, ScalarDiffOp<true, float>{q, k}, mode);
-      else launch_scalar(ls, m, ScalarDiffOp<false, float>{q, k}, mode);
+      shifted ? scalar_diff_pass<true, float>(ls, m, q, k, mode) : scalar_diff_pass<false, float>(ls, m, q, k, mode);
     } else {
-      if (shifted) launch_scalar(ls, m, ScalarDiffOp<true>{q, k}, mode);
-      else launch_scalar(ls, m, ScalarDiffOp<false>{q, k}, mode);
+      shifted ? scalar_diff_pass<true, double>(ls, m, q, k, mode) : scalar_diff_pass<false, double>(ls, m, q, k, mode);
     }
     return NALU_OK;
   });
@@ -1027,10 +1245,10 @@ extern "C" int nalu_assemble_continuity(nalu_linsys* ls, const nalu_mesh* m, con
       return NALU_OK;
     }
     switch (key) {
-#define NALU_CT(K, A, B, C)                                                          \
-  case K:                                                                            \
-    if (fp32_assembly(ls)) launch_scalar(ls, m, ContinuityOp<A, B, C, float>{rho, p, u, gp, tau}, mode); \
-    else launch_scalar(ls, m, ContinuityOp<A, B, C>{rho, p, u, gp, tau}, mode);       \
+#define NALU_CT(K, A, B, C)                                                                              \
+  case K:                                                                                                \
+    fp32_assembly(ls) ? continuity_pass<A, B, C, false, float>(ls, m, rho, p, u, gp, tau, mode, nullptr)  \
+                      : continuity_pass<A, B, C, false, double>(ls, m, rho, p, u, gp, tau, mode, nullptr); \
     break;
       NALU_CT(0, false, false, false)
       NALU_CT(1, false, false, true)
@@ -1056,10 +1274,10 @@ extern "C" int nalu_assemble_continuity_mdot(nalu_linsys* ls, const nalu_mesh* m
     PhaseTimer t(ls, PH_ASSEMBLE);
     const int key = (shift_mdot ? 4 : 0) | (shift_poisson ? 2 : 0) | (reduced_sens ? 1 : 0);
     switch (key) {
-#define NALU_CM(K, A, B, C)                                                                              \
-  case K:                                                                                                \
-    if (fp32_assembly(ls)) launch_scalar(ls, m, ContinuityOp<A, B, C, float>{rho, p, u, gp, tau, mdot}, 0); \
-    else launch_scalar(ls, m, ContinuityOp<A, B, C>{rho, p, u, gp, tau, mdot}, 0);                        \
+#define NALU_CM(K, A, B, C)                                                                       \
+  case K:                                                                                         \
+    fp32_assembly(ls) ? continuity_pass<A, B, C, true, float>(ls, m, rho, p, u, gp, tau, 0, mdot)  \
+                      : continuity_pass<A, B, C, true, double>(ls, m, rho, p, u, gp, tau, 0, mdot); \
     break;
       NALU_CM(0, false, false, false)
       NALU_CM(1, false, false, true)
@@ -1098,37 +1316,76 @@ extern "C" int nalu_compute_mdot_f32(const nalu_mesh* m, const double* rho, cons
 }
 
 namespace {
-// The node-tile momentum pass; ma != nullptr adds the momentum mass kernel in
-// the same pass.
-void launch_momentum_tile(nalu_linsys* ls, const nalu_mesh* m, const double* u, const double* mu, const double* mdot,
-                          double include_divu, bool skew, bool shifted, const MassArgs* ma, bool lumped) {
+// The longest node rows that the numDof 3 row tiles take: 64 of them (and their
+// rhs) fit the LDS of a CU (35 columns).
+bool numdof3_rows_fit(const nalu_linsys* ls) {
+  return (64 * (size_t)ls->max_node_row_len * 9 + 3 * 64) * sizeof(double) <= kMaxLds;
+}
+
+// Fields of a momentum pass as its kernels read them, copied to records for larger
+// systems; a velocity state that is the advected field itself is copied once.
+struct MomentumPass {
+  MomentumFields F;
+  MassArgs A{};
+  MomentumPass(nalu_linsys* ls, const nalu_mesh* m, bool adv, const double* u, const double* mu, const double* mdot,
+               double include_divu, const MassArgs* ma)
+      : F{{{}, m->coords.p, mu}, {{}, u, nullptr}, mdot, include_divu} {
+    if (ma) A = *ma;
+    if (!use_pack(ls)) return;
+    const bool same = adv && ma && A.s[2].vec == u;
+    if (same) F.u.scal = A.s[2].scal;
+    Field4<>* f[6];
+    int n = 0;
+    f[n++] = &F.x;
+    if (adv) f[n++] = &F.u;
+    if (ma) {
+      f[n++] = &A.s[0];
+      f[n++] = &A.s[1];
+      if (!same) f[n++] = &A.s[2];
+      f[n++] = &A.gjp;
+    }
+    pack_fields(ls, f, n);
+    if (same) A.s[2] = F.u;
+  }
+};
+
+// The numDof 3 row-tile pass: advection-diffusion (adv), momentum mass (ma), or both.
+void launch_momentum_rows(nalu_linsys* ls, const nalu_mesh* m, bool adv, const double* u, const double* mu,
+                          const double* mdot, double include_divu, bool skew, bool shifted, const MassArgs* ma,
+                          bool lumped) {
   build_node_incidence(const_cast<nalu_mesh*>(m), ls->stream);
   NALU_REQUIRE(ls->values_pending_zero == ls->rhs_pending_zero, NALU_ERR_STATE,
                "tile assembly: values/rhs zero state diverged");
+  NALU_REQUIRE(numdof3_rows_fit(ls), NALU_ERR_UNSUPPORTED, "momentum row tile: node rows are too long");
   const int accumulate = ls->values_pending_zero ? 0 : 1;
-  const size_t lds = ((size_t)kTileNodes * ls->max_node_row_len * 9 + 3 * kTileNodes) * sizeof(double);
-  const MassArgs none{};
-  const MassArgs& A = ma ? *ma : none;
+  const size_t lds = (size_t)kMomRows * (ls->max_node_row_len * 9 + 3) * sizeof(double);
+  MomentumPass P(ls, m, adv, u, mu, mdot, include_divu, ma);
   auto go = [&](auto kern) {
     set_lds_limit((const void*)kern, lds);
-    hipLaunchKernelGGL(kern, dim3(blocks_for(ls->num_nodes, kTileNodes)), dim3(kTileThreads), lds, ls->stream,
-                       m->conn.p, m->coords.p, u, mu, mdot, include_divu, (const int32_t*)ls->row_node.p,
-                       m->inc_ptr.p, m->inc_elem.p, ls->nrp.p, ls->elem_pos.p, ls->num_nodes, ls->values.p,
-                       ls->rhs.p, accumulate, A);
+    hipLaunchKernelGGL(kern, dim3(blocks_for(ls->num_nodes, kMomRows)), dim3(kMomThreads), lds, ls->stream, P.F, P.A,
+                       m->conn.p, (const int32_t*)ls->row_node.p, m->inc_ptr.p, m->inc_elem.p, ls->nrp.p,
+                       elem_pos_of(ls), ls->num_nodes, ls->values.p, ls->rhs.p, accumulate);
   };
+  // the mass part is FP64 arithmetic at either precision of the advection-diffusion part
   const bool f32 = fp32_assembly(ls);
-  if (ma) {  // the mass part is FP64 arithmetic at either precision of the momentum part
-    // one-pass forms for the default advection options only (compile time)
-    NALU_REQUIRE(!skew && !shifted, NALU_ERR_UNSUPPORTED, "momentum tile: one pass with mass needs skew = shifted = 0");
-    if (lumped) f32 ? go(k_momentum_tile<false, false, float, 2>) : go(k_momentum_tile<false, false, double, 2>);
-    else f32 ? go(k_momentum_tile<false, false, float, 1>) : go(k_momentum_tile<false, false, double, 1>);
-  } else {
-    if (skew && shifted) f32 ? go(k_momentum_tile<true, true, float>) : go(k_momentum_tile<true, true, double>);
-    else if (skew) f32 ? go(k_momentum_tile<true, false, float>) : go(k_momentum_tile<true, false, double>);
-    else if (shifted) f32 ? go(k_momentum_tile<false, true, float>) : go(k_momentum_tile<false, true, double>);
-    else f32 ? go(k_momentum_tile<false, false, float>) : go(k_momentum_tile<false, false, double>);
-  }
+  auto pick = [&](auto pack) {
+    constexpr bool S = decltype(pack)::value;
+    if (!adv) {
+      lumped ? go(k_momentum_rows<false, false, false, S, double, 2>) : go(k_momentum_rows<false, false, false, S, double, 1>);
+    } else if (ma) {  // one-pass forms for the default advection options only (compile time)
+      NALU_REQUIRE(!skew && !shifted, NALU_ERR_UNSUPPORTED, "momentum tile: one pass with mass needs skew = shifted = 0");
+      if (lumped) f32 ? go(k_momentum_rows<true, false, false, S, float, 2>) : go(k_momentum_rows<true, false, false, S, double, 2>);
+      else f32 ? go(k_momentum_rows<true, false, false, S, float, 1>) : go(k_momentum_rows<true, false, false, S, double, 1>);
+    } else {
+      if (skew && shifted) f32 ? go(k_momentum_rows<true, true, true, S, float, 0>) : go(k_momentum_rows<true, true, true, S, double, 0>);
+      else if (skew) f32 ? go(k_momentum_rows<true, true, false, S, float, 0>) : go(k_momentum_rows<true, true, false, S, double, 0>);
+      else if (shifted) f32 ? go(k_momentum_rows<true, false, true, S, float, 0>) : go(k_momentum_rows<true, false, true, S, double, 0>);
+      else f32 ? go(k_momentum_rows<true, false, false, S, float, 0>) : go(k_momentum_rows<true, false, false, S, double, 0>);
+    }
+  };
+  use_pack(ls) ? pick(std::true_type{}) : pick(std::false_type{});
   ls->values_pending_zero = ls->rhs_pending_zero = false;
+  NALU_HIP_CHECK(hipGetLastError());
 }
 }  // namespace
 
@@ -1146,13 +1403,13 @@ extern "C" int nalu_assemble_momentum(nalu_linsys* ls, const nalu_mesh* m, const
       build_node_incidence(const_cast<nalu_mesh*>(m), ls->stream);
       etile_momentum(ls, m, u, mu, mdot, include_divu, skew != 0, shifted != 0, fp32_assembly(ls));
     } else if (mode == 2) {
-      launch_momentum_tile(ls, m, u, mu, mdot, include_divu, skew != 0, shifted != 0, nullptr, false);
+      launch_momentum_rows(ls, m, true, u, mu, mdot, include_divu, skew != 0, shifted != 0, nullptr, false);
     } else {
       materialize_pending_zero(ls);
       const dim3 g(chunk_blocks<8>(E)), b(kChunk);
       auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, g, b, 0, ls->stream, m->conn.p, m->coords.p, u, mu, mdot, include_divu,
-                           ls->node_lid.p, ls->nrp.p, ls->elem_pos.p, E, ls->values.p, ls->rhs.p);
+                           ls->node_lid.p, ls->nrp.p, elem_pos_of(ls), E, ls->values.p, ls->rhs.p);
       };
       const bool f32 = fp32_assembly(ls);
       if (skew && shifted) f32 ? go(k_momentum_atomic<true, true, float>) : go(k_momentum_atomic<true, true, double>);
@@ -1179,7 +1436,7 @@ extern "C" int nalu_linsys_sum_into_batch(nalu_linsys* ls, int64_t nelem, const 
                  "sum_into_batch: conn must be the graph mesh's connectivity (nalu_mesh_device_ptrs)");
     const int64_t n = nelem * 8 * ls->num_dof;
     hipLaunchKernelGGL(k_sum_into_batch, dim3(blocks_for(n, 256)), dim3(256), 0, ls->stream, conn, lhs, rhs_e,
-                       ls->node_lid.p, ls->nrp.p, ls->elem_pos.p, nelem, ls->num_dof, ls->values.p, ls->rhs.p);
+                       ls->node_lid.p, ls->nrp.p, elem_pos_of(ls), nelem, ls->num_dof, ls->values.p, ls->rhs.p);
     NALU_HIP_CHECK(hipGetLastError());
     return NALU_OK;
   });
@@ -1228,34 +1485,16 @@ extern "C" int nalu_linsys_reset_rows(nalu_linsys* ls, int64_t nn, const int32_t
 }
 
 namespace {
-void launch_mass(nalu_linsys* ls, const nalu_mesh* m, const MassArgs& A, bool mom, bool lumped,
-                 double* rhs3 = nullptr) {
+template <bool MOM>
+void launch_mass_gather(nalu_linsys* ls, const nalu_mesh* m, const MassArgs& A, bool lumped) {
   build_node_incidence(const_cast<nalu_mesh*>(m), ls->stream);
-  const size_t lds3 = ((size_t)kTileNodes * ls->max_node_row_len * 9 + 3 * kTileNodes) * sizeof(double);
-  if (mom && !rhs3 && lds3 <= kMaxLds && ls->values_pending_zero == ls->rhs_pending_zero) {
-    // numDof 3: node tile with the row segments in LDS
-    const int accumulate = ls->values_pending_zero ? 0 : 1;
-    auto go3 = [&](auto kern) {
-      set_lds_limit((const void*)kern, lds3);
-      hipLaunchKernelGGL(kern, dim3(blocks_for(ls->num_nodes, kTileNodes)), dim3(kTileThreads), lds3, ls->stream, A,
-                         m->conn.p, m->coords.p, (const int32_t*)ls->row_node.p, m->inc_ptr.p, m->inc_elem.p,
-                         ls->nrp.p, ls->elem_pos.p, ls->num_nodes, ls->values.p, ls->rhs.p, accumulate);
-    };
-    lumped ? go3(k_mass_tile3<true>) : go3(k_mass_tile3<false>);
-    ls->values_pending_zero = ls->rhs_pending_zero = false;
-    NALU_HIP_CHECK(hipGetLastError());
-    return;
-  }
   materialize_pending_zero(ls);
-  const dim3 g(blocks_for(ls->num_nodes, 256)), b(256);
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, g, b, 0, ls->stream, A, m->conn.p, m->coords.p, (const int32_t*)ls->row_node.p,
-                       m->inc_ptr.p, m->inc_elem.p, ls->nrp.p, ls->elem_pos.p, ls->num_nodes, ls->values.p,
-                       rhs3 ? rhs3 : ls->rhs.p);
+    hipLaunchKernelGGL(kern, dim3(blocks_for(ls->num_nodes, 256)), dim3(256), 0, ls->stream, A, m->conn.p,
+                       m->coords.p, (const int32_t*)ls->row_node.p, m->inc_ptr.p, m->inc_elem.p, ls->nrp.p,
+                       elem_pos_of(ls), ls->num_nodes, ls->values.p, ls->rhs.p);
   };
-  if (rhs3) lumped ? go(k_mass_gather<true, true, true>) : go(k_mass_gather<true, false, true>);
-  else if (mom) lumped ? go(k_mass_gather<true, true, false>) : go(k_mass_gather<true, false, false>);
-  else lumped ? go(k_mass_gather<false, true, false>) : go(k_mass_gather<false, false, false>);
+  lumped ? go(k_mass_gather<MOM, true>) : go(k_mass_gather<MOM, false>);
   NALU_HIP_CHECK(hipGetLastError());
 }
 
@@ -1277,9 +1516,11 @@ extern "C" int nalu_assemble_momentum_mass(nalu_linsys* ls, const nalu_mesh* m, 
     NALU_REQUIRE(rho_nm1 && rho_n && rho_np1 && u_nm1 && u_n && u_np1 && gjp, NALU_ERR_ARG,
                  "momentum_mass: null field");
     PhaseTimer t(ls, PH_ASSEMBLE);
-    const MassArgs A{{rho_nm1, rho_n, rho_np1}, {u_nm1, u_n, u_np1}, gjp, dt, gamma[0], gamma[1], gamma[2],
+    const MassArgs A{{{{}, u_nm1, rho_nm1}, {{}, u_n, rho_n}, {{}, u_np1, rho_np1}}, {{}, gjp, nullptr}, dt, gamma[0], gamma[1], gamma[2],
                      balanced_force ? 1 : 0};
-    launch_mass(ls, m, A, true, lumped != 0);
+    if (numdof3_rows_fit(ls) && ls->values_pending_zero == ls->rhs_pending_zero)
+      launch_momentum_rows(ls, m, false, nullptr, nullptr, nullptr, 0.0, false, false, &A, lumped != 0);
+    else launch_mass_gather<true>(ls, m, A, lumped != 0);
     return NALU_OK;
   });
 }
@@ -1296,19 +1537,19 @@ extern "C" int nalu_assemble_momentum_with_mass(nalu_linsys* ls, const nalu_mesh
     NALU_REQUIRE(u && mu && mdot, NALU_ERR_ARG, "momentum_with_mass: null advection-diffusion field");
     NALU_REQUIRE(rho_nm1 && rho_n && rho_np1 && u_nm1 && u_n && u_np1 && gjp, NALU_ERR_ARG,
                  "momentum_with_mass: null mass field");
-    const size_t lds = ((size_t)kTileNodes * ls->max_node_row_len * 9 + 3 * kTileNodes) * sizeof(double);
-    // the two passes one after the other: rows too long for a node tile, or the
+    const bool tile = numdof3_rows_fit(ls);
+    // the two passes one after the other: rows too long for a row tile, or the
     // skew-symmetric / shifted advection options (one-pass forms exist for the defaults)
-    if (lds > kMaxLds || skew || shifted) {
-      int rc = nalu_assemble_momentum(ls, m, u, mu, mdot, include_divu, skew, shifted, lds > kMaxLds ? 1 : 2);
+    if (!tile || skew || shifted) {
+      int rc = nalu_assemble_momentum(ls, m, u, mu, mdot, include_divu, skew, shifted, tile ? 2 : 1);
       if (rc != NALU_OK) return rc;
       return nalu_assemble_momentum_mass(ls, m, rho_nm1, rho_n, rho_np1, u_nm1, u_n, u_np1, gjp, dt, gamma, lumped,
                                          balanced_force);
     }
     PhaseTimer t(ls, PH_ASSEMBLE);
-    const MassArgs A{{rho_nm1, rho_n, rho_np1}, {u_nm1, u_n, u_np1}, gjp, dt, gamma[0], gamma[1], gamma[2],
+    const MassArgs A{{{{}, u_nm1, rho_nm1}, {{}, u_n, rho_n}, {{}, u_np1, rho_np1}}, {{}, gjp, nullptr}, dt, gamma[0], gamma[1], gamma[2],
                      balanced_force ? 1 : 0};
-    launch_momentum_tile(ls, m, u, mu, mdot, include_divu, skew != 0, shifted != 0, &A, lumped != 0);
+    launch_momentum_rows(ls, m, true, u, mu, mdot, include_divu, skew != 0, shifted != 0, &A, lumped != 0);
     NALU_HIP_CHECK(hipGetLastError());
     return NALU_OK;
   });
@@ -1322,45 +1563,50 @@ extern "C" int nalu_assemble_continuity_mass(nalu_linsys* ls, const nalu_mesh* m
     check_mass_args(dt, gamma);
     NALU_REQUIRE(rho_nm1 && rho_n && rho_np1, NALU_ERR_ARG, "continuity_mass: null field");
     PhaseTimer t(ls, PH_ASSEMBLE);
-    const MassArgs A{{rho_nm1, rho_n, rho_np1}, {nullptr, nullptr, nullptr}, nullptr, dt, gamma[0], gamma[1],
+    const MassArgs A{{{{}, nullptr, rho_nm1}, {{}, nullptr, rho_n}, {{}, nullptr, rho_np1}}, {}, dt, gamma[0], gamma[1],
                      gamma[2], 0};
-    launch_mass(ls, m, A, false, lumped != 0);
+    launch_mass_gather<false>(ls, m, A, lumped != 0);
     return NALU_OK;
   });
 }
 
 namespace {
-// The segregated momentum row gather; ma != nullptr adds the momentum mass
-// kernel in the same pass.
-void launch_momentum_seg(nalu_linsys* ls, const nalu_mesh* m, const double* u, const double* mu, const double* mdot,
-                         double include_divu, bool skew, bool shifted, double* rhs3, const MassArgs* ma, bool lumped) {
+// The segregated momentum row tile: advection-diffusion (adv), momentum mass (ma), or both.
+void launch_momentum_seg(nalu_linsys* ls, const nalu_mesh* m, bool adv, const double* u, const double* mu,
+                         const double* mdot, double include_divu, bool skew, bool shifted, double* rhs3,
+                         const MassArgs* ma, bool lumped) {
   build_node_incidence(const_cast<nalu_mesh*>(m), ls->stream);
   if (ls->rhs_pending_zero) NALU_HIP_CHECK(hipMemsetAsync(ls->rhs.p, 0, ls->rhs.bytes(), ls->stream));
   ls->rhs_pending_zero = false;
   const int accumulate = ls->values_pending_zero ? 0 : 1;
-  constexpr int B = 256;
-  const size_t lds = (size_t)B * ls->max_node_row_len * sizeof(double);
-  const MassArgs none{};
-  const MassArgs& A = ma ? *ma : none;
+  const size_t lds = lds_rows(ls);
+  MomentumPass P(ls, m, adv, u, mu, mdot, include_divu, ma);
   auto go = [&](auto kern) {
     set_lds_limit((const void*)kern, lds);
-    hipLaunchKernelGGL(kern, dim3(blocks_for(ls->nrows, B)), dim3(B), lds, ls->stream, m->conn.p, m->coords.p, u, mu,
-                       mdot, include_divu, (const int32_t*)ls->row_node.p, m->inc_ptr.p, m->inc_elem.p, ls->nrp.p,
-                       ls->elem_pos.p, ls->nrows, ls->values.p, rhs3, accumulate, A);
+    hipLaunchKernelGGL(kern, dim3(blocks_for(ls->nrows, kRowsPerBlock)), dim3(kRowThreads), lds, ls->stream, P.F, P.A,
+                       m->conn.p, (const int32_t*)ls->row_node.p, m->inc_ptr.p, m->inc_elem.p, ls->nrp.p,
+                       elem_pos_of(ls), ls->nrows, ls->max_node_row_len, ls->values.p, rhs3, accumulate);
   };
+  // the mass part is FP64 arithmetic at either precision of the advection-diffusion part
   const bool f32 = fp32_assembly(ls);
-  if (ma) {  // the mass part is FP64 arithmetic at either precision of the momentum part
-    // one-pass forms for the default advection options only (compile time)
-    NALU_REQUIRE(!skew && !shifted, NALU_ERR_UNSUPPORTED,
-                 "momentum gather: one pass with mass needs skew = shifted = 0");
-    if (lumped) f32 ? go(k_momentum_seg_gather<false, false, float, 2>) : go(k_momentum_seg_gather<false, false, double, 2>);
-    else f32 ? go(k_momentum_seg_gather<false, false, float, 1>) : go(k_momentum_seg_gather<false, false, double, 1>);
-  } else {
-    if (skew && shifted) f32 ? go(k_momentum_seg_gather<true, true, float>) : go(k_momentum_seg_gather<true, true, double>);
-    else if (skew) f32 ? go(k_momentum_seg_gather<true, false, float>) : go(k_momentum_seg_gather<true, false, double>);
-    else if (shifted) f32 ? go(k_momentum_seg_gather<false, true, float>) : go(k_momentum_seg_gather<false, true, double>);
-    else f32 ? go(k_momentum_seg_gather<false, false, float>) : go(k_momentum_seg_gather<false, false, double>);
-  }
+  auto pick = [&](auto pack) {
+    constexpr bool S = decltype(pack)::value;
+    if (!adv) {
+      lumped ? go(k_momentum_seg_rows<false, false, false, S, double, 2>)
+             : go(k_momentum_seg_rows<false, false, false, S, double, 1>);
+    } else if (ma) {  // one-pass forms for the default advection options only (compile time)
+      NALU_REQUIRE(!skew && !shifted, NALU_ERR_UNSUPPORTED,
+                   "momentum rows: one pass with mass needs skew = shifted = 0");
+      if (lumped) f32 ? go(k_momentum_seg_rows<true, false, false, S, float, 2>) : go(k_momentum_seg_rows<true, false, false, S, double, 2>);
+      else f32 ? go(k_momentum_seg_rows<true, false, false, S, float, 1>) : go(k_momentum_seg_rows<true, false, false, S, double, 1>);
+    } else {
+      if (skew && shifted) f32 ? go(k_momentum_seg_rows<true, true, true, S, float, 0>) : go(k_momentum_seg_rows<true, true, true, S, double, 0>);
+      else if (skew) f32 ? go(k_momentum_seg_rows<true, true, false, S, float, 0>) : go(k_momentum_seg_rows<true, true, false, S, double, 0>);
+      else if (shifted) f32 ? go(k_momentum_seg_rows<true, false, true, S, float, 0>) : go(k_momentum_seg_rows<true, false, true, S, double, 0>);
+      else f32 ? go(k_momentum_seg_rows<true, false, false, S, float, 0>) : go(k_momentum_seg_rows<true, false, false, S, double, 0>);
+    }
+  };
+  use_pack(ls) ? pick(std::true_type{}) : pick(std::false_type{});
   ls->values_pending_zero = false;
   NALU_HIP_CHECK(hipGetLastError());
 }
@@ -1373,7 +1619,7 @@ extern "C" int nalu_assemble_momentum_segregated(nalu_linsys* ls, const nalu_mes
     check_assembly_args(ls, m, 1);
     NALU_REQUIRE(u && mu && mdot && rhs3, NALU_ERR_ARG, "momentum_segregated: null field");
     PhaseTimer t(ls, PH_ASSEMBLE);
-    launch_momentum_seg(ls, m, u, mu, mdot, include_divu, skew != 0, shifted != 0, rhs3, nullptr, false);
+    launch_momentum_seg(ls, m, true, u, mu, mdot, include_divu, skew != 0, shifted != 0, rhs3, nullptr, false);
     return NALU_OK;
   });
 }
@@ -1389,9 +1635,9 @@ extern "C" int nalu_assemble_momentum_mass_segregated(nalu_linsys* ls, const nal
     NALU_REQUIRE(rho_nm1 && rho_n && rho_np1 && u_nm1 && u_n && u_np1 && gjp && rhs3, NALU_ERR_ARG,
                  "momentum_mass_segregated: null field");
     PhaseTimer t(ls, PH_ASSEMBLE);
-    const MassArgs A{{rho_nm1, rho_n, rho_np1}, {u_nm1, u_n, u_np1}, gjp, dt, gamma[0], gamma[1], gamma[2],
+    const MassArgs A{{{{}, u_nm1, rho_nm1}, {{}, u_n, rho_n}, {{}, u_np1, rho_np1}}, {{}, gjp, nullptr}, dt, gamma[0], gamma[1], gamma[2],
                      balanced_force ? 1 : 0};
-    launch_mass(ls, m, A, true, lumped != 0, rhs3);
+    launch_momentum_seg(ls, m, false, nullptr, nullptr, nullptr, 0.0, false, false, rhs3, &A, lumped != 0);
     return NALU_OK;
   });
 }
@@ -1414,9 +1660,9 @@ extern "C" int nalu_assemble_momentum_with_mass_segregated(
                                                     lumped, balanced_force, rhs3);
     }
     PhaseTimer t(ls, PH_ASSEMBLE);
-    const MassArgs A{{rho_nm1, rho_n, rho_np1}, {u_nm1, u_n, u_np1}, gjp, dt, gamma[0], gamma[1], gamma[2],
+    const MassArgs A{{{{}, u_nm1, rho_nm1}, {{}, u_n, rho_n}, {{}, u_np1, rho_np1}}, {{}, gjp, nullptr}, dt, gamma[0], gamma[1], gamma[2],
                      balanced_force ? 1 : 0};
-    launch_momentum_seg(ls, m, u, mu, mdot, include_divu, false, false, rhs3, &A, lumped != 0);
+    launch_momentum_seg(ls, m, true, u, mu, mdot, include_divu, false, false, rhs3, &A, lumped != 0);
     return NALU_OK;
   });
 }
@@ -1426,7 +1672,7 @@ extern "C" int nalu_compute_dual_volume(const nalu_mesh* m, double* dual_vol, vo
     NALU_REQUIRE(m && dual_vol, NALU_ERR_ARG, "dual_volume: null argument");
     hipStream_t s = (hipStream_t)stream;
     build_node_incidence(const_cast<nalu_mesh*>(m), s);
-    hipLaunchKernelGGL(k_dual_volume, dim3(blocks_for(m->num_nodes, 256)), dim3(256), 0, s, m->conn.p, m->coords.p,
+    hipLaunchKernelGGL(k_dual_volume, dim3(blocks_for(m->num_nodes, kRowsPerBlock)), dim3(kRowThreads), 0, s, m->conn.p, m->coords.p,
                        m->inc_ptr.p, m->inc_elem.p, m->num_nodes, dual_vol);
     NALU_HIP_CHECK(hipGetLastError());
     return NALU_OK;
@@ -1438,7 +1684,7 @@ void nodal_grad_interior(const nalu_mesh* m, const double* q, const double* dual
                          hipStream_t s) {
   build_node_incidence(const_cast<nalu_mesh*>(m), s);
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(blocks_for(m->num_nodes, 256)), dim3(256), 0, s, m->conn.p, m->coords.p, q,
+    hipLaunchKernelGGL(kern, dim3(blocks_for(m->num_nodes, kRowsPerBlock)), dim3(kRowThreads), 0, s, m->conn.p, m->coords.p, q,
                        dual_vol, m->inc_ptr.p, m->inc_elem.p, m->num_nodes, dqdx);
   };
   if (shifted) go(k_nodal_grad<true>);

@@ -130,7 +130,7 @@ __device__ __forceinline__ int col_pos(const Visit& v, int k, int c) {
 
 template <int CLS>
 __device__ __forceinline__ void load_visit(Visit& v, int64_t e, uint32_t perm, const int32_t* __restrict__ conn,
-                                           const int32_t* __restrict__ lid, const uint64_t* __restrict__ elem_pos,
+                                           const int32_t* __restrict__ lid, ElemPos elem_pos,
                                            int32_t a0, int32_t a1) {
   v.e = e;
   v.perm = perm;
@@ -144,7 +144,7 @@ __device__ __forceinline__ void load_visit(Visit& v, int64_t e, uint32_t perm, c
     if ((kClassNodes[CLS] >> k) & 1u) {
       v.row[k] = lid[v.nd[k]];
       v.own[k] = v.row[k] >= a0 && v.row[k] < a1;
-      if (v.own[k]) v.pk[k] = elem_pos[8 * e + phys(perm, k)];
+      if (v.own[k]) v.pk[k] = elem_pos(e, phys(perm, k));
     }
   }
 }
@@ -277,7 +277,7 @@ __device__ __forceinline__ int wave_max(int v) {
 template <int CLS, class Op>
 __device__ __forceinline__ void scalar_visit(const Op& op, int64_t e, uint32_t perm, const int32_t* __restrict__ conn,
                                              const double* __restrict__ coords, const int32_t* __restrict__ lid,
-                                             const int32_t* __restrict__ nrp, const uint64_t* __restrict__ elem_pos,
+                                             const int32_t* __restrict__ nrp, ElemPos elem_pos,
                                              int32_t a0, int32_t a1, int32_t s0, double* seg, double* rseg) {
   Visit v;
   load_visit<CLS>(v, e, perm, conn, lid, elem_pos, a0, a1);
@@ -344,7 +344,7 @@ __global__ __launch_bounds__(256) void k_scalar_etile(Op op, const int32_t* __re
                                                       const double* __restrict__ coords,
                                                       const int32_t* __restrict__ lid,
                                                       const int32_t* __restrict__ nrp,
-                                                      const uint64_t* __restrict__ elem_pos,
+                                                      ElemPos elem_pos,
                                                       const int32_t* __restrict__ vptr,
                                                       const int32_t* __restrict__ velem,
                                                       const uint8_t* __restrict__ vcode,
@@ -445,7 +445,7 @@ __device__ __forceinline__ void momentum_visit(int64_t e, int code, const int32_
                                                const double* __restrict__ mu, const double* __restrict__ mdot,
                                                double incl_divu, const int32_t* __restrict__ lid,
                                                const int32_t* __restrict__ nrp,
-                                               const uint64_t* __restrict__ elem_pos, int32_t a0, int32_t a1,
+                                               ElemPos elem_pos, int32_t a0, int32_t a1,
                                                int32_t s0, double* seg, double* rseg) {
   Visit v;
   const uint32_t perm = kSym.perm[code & 31];
@@ -518,7 +518,7 @@ __global__ __launch_bounds__(128) void k_momentum_etile(const int32_t* __restric
                                                         const double* __restrict__ mdot, double incl_divu,
                                                         const int32_t* __restrict__ lid,
                                                         const int32_t* __restrict__ nrp,
-                                                        const uint64_t* __restrict__ elem_pos,
+                                                        ElemPos elem_pos,
                                                         const int32_t* __restrict__ vptr,
                                                         const int32_t* __restrict__ velem,
                                                         const uint8_t* __restrict__ vcode,
@@ -577,7 +577,7 @@ __host__ __device__ constexpr int item_ip(int slot) {
 template <int IP, class Op>
 __device__ __forceinline__ void scalar_item(const Op& op, int64_t e, uint32_t perm, const int32_t* __restrict__ conn,
                                             const double* __restrict__ coords, const int32_t* __restrict__ lid,
-                                            const int32_t* __restrict__ nrp, const uint64_t* __restrict__ elem_pos,
+                                            const int32_t* __restrict__ nrp, ElemPos elem_pos,
                                             int32_t a0, int32_t a1, int32_t s0, double* seg, double* rseg) {
   constexpr int il = scs_left(IP), ir = scs_right(IP);
   constexpr bool Lc = (kClassNodes[kClassB] >> il) & 1u, Rc = (kClassNodes[kClassB] >> ir) & 1u;
@@ -600,7 +600,7 @@ __device__ __forceinline__ void scalar_item(const Op& op, int64_t e, uint32_t pe
 template <class Op>
 __global__ __launch_bounds__(64 * kItemSlots) void k_scalar_items(
     Op op, const int32_t* __restrict__ conn, const double* __restrict__ coords, const int32_t* __restrict__ lid,
-    const int32_t* __restrict__ nrp, const uint64_t* __restrict__ elem_pos, const int32_t* __restrict__ vptr,
+    const int32_t* __restrict__ nrp, ElemPos elem_pos, const int32_t* __restrict__ vptr,
     const int32_t* __restrict__ velem, const uint8_t* __restrict__ vcode, const int32_t* __restrict__ tiles,
     int64_t ntl, int T, int64_t nrows, double* __restrict__ vals, double* __restrict__ rhs, int accumulate) {
   extern __shared__ double seg[];
@@ -643,7 +643,7 @@ __device__ __forceinline__ void momentum_item(int64_t e, int code, const int32_t
                                               const double* __restrict__ mu, const double* __restrict__ mdot,
                                               double incl_divu, const int32_t* __restrict__ lid,
                                               const int32_t* __restrict__ nrp,
-                                              const uint64_t* __restrict__ elem_pos, int32_t a0, int32_t a1,
+                                              ElemPos elem_pos, int32_t a0, int32_t a1,
                                               int32_t s0, double* seg, double* rseg) {
   constexpr int il = scs_left(IP), ir = scs_right(IP);
   constexpr bool Lc = (kClassNodes[kClassB] >> il) & 1u, Rc = (kClassNodes[kClassB] >> ir) & 1u;
@@ -703,7 +703,7 @@ template <bool SKEW, bool SHIFT, typename R>
 __global__ __launch_bounds__(64 * kItemSlots) void k_momentum_items(
     const int32_t* __restrict__ conn, const double* __restrict__ coords, const double* __restrict__ u,
     const double* __restrict__ mu, const double* __restrict__ mdot, double incl_divu, const int32_t* __restrict__ lid,
-    const int32_t* __restrict__ nrp, const uint64_t* __restrict__ elem_pos, const int32_t* __restrict__ vptr,
+    const int32_t* __restrict__ nrp, ElemPos elem_pos, const int32_t* __restrict__ vptr,
     const int32_t* __restrict__ velem, const uint8_t* __restrict__ vcode, const int32_t* __restrict__ tiles,
     int64_t ntl, int T, int64_t nnodes, double* __restrict__ vals, double* __restrict__ rhs, int accumulate) {
   extern __shared__ double seg[];
@@ -932,13 +932,13 @@ void etile_scalar(nalu_linsys* ls, const nalu_mesh* m, const Op& op) {
     if (ntl == 0) return;
     set_lds_limit((const void*)kern, lds);
     hipLaunchKernelGGL(kern, dim3((unsigned)xcd_grid(ntl)), dim3(256), lds, ls->stream, op, m->conn.p, m->coords.p,
-                       ls->node_lid.p, ls->nrp.p, ls->elem_pos.p, P.vptr.p, P.velem.p, P.vcode.p, tiles, ntl, P.T,
+                       ls->node_lid.p, ls->nrp.p, elem_pos_of(ls), P.vptr.p, P.velem.p, P.vcode.p, tiles, ntl, P.T,
                        ls->num_nodes, ls->values.p, ls->rhs.p, accumulate);
   };
   if (P.nfast) {
     set_lds_limit((const void*)k_scalar_items<Op>, lds);
     hipLaunchKernelGGL(k_scalar_items<Op>, dim3((unsigned)xcd_grid(P.nfast)), dim3(64 * kItemSlots), lds, ls->stream,
-                       op, m->conn.p, m->coords.p, ls->node_lid.p, ls->nrp.p, ls->elem_pos.p, P.vptr.p, P.velem.p,
+                       op, m->conn.p, m->coords.p, ls->node_lid.p, ls->nrp.p, elem_pos_of(ls), P.vptr.p, P.velem.p,
                        P.vcode.p, P.fast_tiles.p, P.nfast, P.T, ls->num_nodes, ls->values.p, ls->rhs.p, accumulate);
   }
   go(k_scalar_etile<Op, false>, P.other_tiles.p, P.nother);
@@ -988,14 +988,14 @@ void etile_momentum(nalu_linsys* ls, const nalu_mesh* m, const double* u, const 
     if (ntl == 0) return;
     set_lds_limit((const void*)kern, lds);
     hipLaunchKernelGGL(kern, dim3((unsigned)xcd_grid(ntl)), dim3(128), lds, ls->stream, m->conn.p, m->coords.p, u,
-                       mu, mdot, include_divu, ls->node_lid.p, ls->nrp.p, ls->elem_pos.p, P.vptr.p, P.velem.p,
+                       mu, mdot, include_divu, ls->node_lid.p, ls->nrp.p, elem_pos_of(ls), P.vptr.p, P.velem.p,
                        P.vcode.p, tiles, ntl, P.T, ls->num_nodes, ls->values.p, ls->rhs.p, accumulate);
   };
   auto go = [&](auto fast, auto other) {
     if (P.nfast) {
       set_lds_limit((const void*)fast, lds);
       hipLaunchKernelGGL(fast, dim3((unsigned)xcd_grid(P.nfast)), dim3(64 * kItemSlots), lds, ls->stream, m->conn.p,
-                         m->coords.p, u, mu, mdot, include_divu, ls->node_lid.p, ls->nrp.p, ls->elem_pos.p, P.vptr.p,
+                         m->coords.p, u, mu, mdot, include_divu, ls->node_lid.p, ls->nrp.p, elem_pos_of(ls), P.vptr.p,
                          P.velem.p, P.vcode.p, P.fast_tiles.p, P.nfast, P.T, ls->num_nodes, ls->values.p, ls->rhs.p,
                          accumulate);
     }

@@ -81,14 +81,15 @@ __device__ inline int find_in_row(const int32_t* __restrict__ cols, int len, int
   return lo;
 }
 
-// Element scatter table: for (e, a), byte c = position of node c in node-row a.
+// Element scatter table, one array of elements per local node a: byte c of
+// pos[a][e] = position of node c in the node-row of a.
 __global__ void k_elem_pos(const int32_t* __restrict__ conn, const int32_t* __restrict__ lid,
                            const int32_t* __restrict__ nrp, const int32_t* __restrict__ nci,
                            int64_t nelem, uint64_t* __restrict__ pos, int* __restrict__ bad) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nelem * 8) return;
-  const int64_t e = t >> 3;
-  const int a = (int)(t & 7);
+  const int a = (int)(t / nelem);
+  const int64_t e = t - a * nelem;
   const int32_t row = lid[conn[8 * e + a]];
   const int32_t b0 = nrp[row];
   const int len = nrp[row + 1] - b0;

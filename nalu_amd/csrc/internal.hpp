@@ -164,9 +164,12 @@ struct nalu_linsys {
   nalu::DevBuf<int32_t> node_lid;  // [N] rank of node id (row of dof 0 = num_dof*lid)
   nalu::DevBuf<int32_t> nrp;       // node graph row_ptr [N+1]
   nalu::DevBuf<int32_t> nci;       // node graph col idx (node lids) [P]
-  // element scatter table: for element e, local row node a: 8 bytes, byte c =
-  // position of column node c in node-row of node a.
-  nalu::DevBuf<uint64_t> elem_pos; // [E][8]
+  // element scatter table: for local row node a of element e: 8 bytes, byte c =
+  // position of column node c in node-row of node a.  One array per local node, so
+  // that lanes on consecutive elements read consecutive entries.
+  nalu::DevBuf<uint64_t> elem_pos; // [8][E]
+  // packed nodal fields of a row-assembly pass (assemble.hip)
+  nalu::DevBuf<unsigned char> pack_ws;
 
   // expanded CSR (numDof rows interleaved, src/TpetraLinearSystem.C:1227-1246)
   nalu::DevBuf<int32_t> row_ptr;   // [nrows+1]
@@ -270,6 +273,16 @@ struct PhaseTimer {
   ~PhaseTimer();
 };
 void flush_timers(nalu_linsys* ls);
+
+// The element scatter table as kernels read it.
+struct ElemPos {
+  const uint64_t* p;
+  int64_t nelem;
+  __device__ __forceinline__ uint64_t operator()(int64_t e, int a) const { return p[a * nelem + e]; }
+};
+inline ElemPos elem_pos_of(const nalu_linsys* ls) {
+  return {ls->elem_pos.p, (int64_t)(ls->elem_pos.n / 8)};
+}
 
 // One chunk of the SELL-64 solver copy: rows [row0, row0 + nrows) of one color;
 // L entry k of row row0 + r at loff + 64 k + r (lw entries), U likewise.

@@ -1,0 +1,206 @@
+"""Row-tile assembly against the oracle where its indexing can go wrong: nodes with
+more incident elements than a row has lanes (fan meshes), element axes that differ
+from element to element (every local node as the row node, both handednesses),
+row counts around the tile sizes, explicit node ids, and systems on both sides of
+the size from which the nodal fields are packed first (32768 nodes).
+
+Bar: 1e-12 of the row's (rhs: of the vector's) largest entry.  Entries are sums of
+at most 24 products of coordinate differences (about 1e2 eps), and the meshes have
+cells no smaller than 1/33 of their coordinates (a further factor of 1e2)."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import nalu_amd as na  # noqa: E402
+from tests.fixtures import rel_err_rowwise  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+TOL = 1e-12
+# the 24 orientation-preserving relabelings of the reference hexahedron's nodes
+SIGN = np.array([[-1, -1, -1], [1, -1, -1], [1, 1, -1], [-1, 1, -1], [-1, -1, 1], [1, -1, 1], [1, 1, 1], [-1, 1, 1]])
+
+
+def rotations():
+    out = []
+    for p in ((0, 1, 2), (1, 2, 0), (2, 0, 1), (0, 2, 1), (2, 1, 0), (1, 0, 2)):
+        for s in np.ndindex(2, 2, 2):
+            R = np.zeros((3, 3))
+            for i in range(3):
+                R[i, p[i]] = 1 - 2 * s[i]
+            if np.linalg.det(R) > 0:
+                T = SIGN @ R.T
+                out.append([int(np.nonzero((SIGN == t).all(1))[0][0]) for t in T])
+    return out
+
+
+def dev(a):
+    return torch.as_tensor(np.ascontiguousarray(a), dtype=torch.float64, device=DEV)
+
+
+def fan(sectors, layers, rng):
+    """Quadrilaterals around an axis, extruded: an axis node inside has 2 sectors incident elements."""
+    th = 2 * np.pi * np.arange(sectors) / sectors
+    half = np.pi / sectors
+    ring = [[0.0, 0.0]]
+    for t in th:
+        ring += [[np.cos(t), np.sin(t)], [1.4 * np.cos(t + half), 1.4 * np.sin(t + half)]]
+    n2 = len(ring)
+    X = np.array([[x, y, 0.7 * k] for k in range(layers + 1) for x, y in ring])
+    X += 0.05 * rng.uniform(-1, 1, X.shape)
+    conn = []
+    for k in range(layers):
+        for s in range(sectors):
+            q = [0, 1 + 2 * s, 2 + 2 * s, 1 + 2 * ((s + 1) % sectors)]
+            conn.append([k * n2 + a for a in q] + [(k + 1) * n2 + a for a in q])
+    return X, np.array(conn, dtype=np.int32)
+
+
+def brick(nx, ny, nz, rng):
+    i, j, k = np.meshgrid(np.arange(nx + 1), np.arange(ny + 1), np.arange(nz + 1), indexing="ij")
+    at = (i + (nx + 1) * (j + (ny + 1) * k))
+    X = np.zeros((at.size, 3))
+    X[at.ravel()] = np.stack([i.ravel() / nx, j.ravel() / ny, k.ravel() / nz], 1)
+    X += rng.uniform(-0.1, 0.1, X.shape) / np.array([nx, ny, nz])
+    c = lambda a, b, d: at[a:nx + a, b:ny + b, d:nz + d].transpose(2, 1, 0).ravel()  # noqa: E731
+    conn = np.stack([c(0, 0, 0), c(1, 0, 0), c(1, 1, 0), c(0, 1, 0), c(0, 0, 1), c(1, 0, 1), c(1, 1, 1), c(0, 1, 1)], 1)
+    return X, conn.astype(np.int32)
+
+
+MESHES = {
+    "fan5": lambda r: fan(5, 3, r),            # valence 10
+    "fan9": lambda r: fan(9, 2, r),            # valence 18: three passes over a row's elements
+    "brick1": lambda r: brick(1, 1, 1, r),     # 8 rows
+    "brick-odd": lambda r: brick(5, 2, 4, r),  # 90 rows
+    "below-pack": lambda r: brick(31, 31, 30, r),
+    "pack": lambda r: brick(31, 31, 31, r),    # 32768 nodes
+    "pack-odd": lambda r: brick(30, 37, 28, r),
+}
+
+
+def problem(name, seed):
+    rng = np.random.default_rng(seed)
+    X, conn = MESHES[name](rng)
+    rot = rotations()
+    conn = np.stack([c[rot[k]] for c, k in zip(conn, rng.integers(0, len(rot), conn.shape[0]))]).astype(np.int32)
+    N, E = X.shape[0], conn.shape[0]
+    f = {"rho": rng.uniform(0.5, 2, (3, N)), "p": rng.normal(size=N), "u": rng.normal(size=(3, N, 3)),
+         "gp": rng.normal(size=(N, 3)), "mu": rng.uniform(0.1, 2, N), "mdot": rng.normal(size=(E, 12))}
+    return X, conn, f, rng
+
+
+def check(what, v, r, ov, orhs, row_ptr):
+    e1 = rel_err_rowwise(v, ov, row_ptr) if v is not None else 0.0
+    e2 = np.abs(r - orhs).max() / np.abs(orhs).max()
+    print("  %s: matrix %.2e rhs %.2e" % (what, e1, e2), flush=True)
+    assert e1 <= TOL and e2 <= TOL, what
+
+
+@pytest.mark.parametrize("name", list(MESHES))
+@pytest.mark.parametrize("ids", [False, True])
+def test_rows(oracle, name, ids):
+    print("case: row tiles on", name, "ids" if ids else "", flush=True)
+    X, conn, f, rng = problem(name, 3)
+    N, E = X.shape[0], conn.shape[0]
+    gid = (rng.permutation(N) + 1).astype(np.int64) if ids else None
+    mesh = na.Mesh(X, conn, gid)
+    ls = na.LinearSystem(1)
+    ls.buildElemToNodeGraph(mesh)
+    ls.finalizeLinearSystem()
+    g = oracle.graph_build(N, conn, node_ids=gid)
+    d = {k: dev(v) for k, v in f.items()}
+    rho, u = [d["rho"][i].contiguous() for i in range(3)], [d["u"][i].contiguous() for i in range(3)]
+    big = N > 4000
+    for shifted in (False, True):
+        for mode in ("gather", "tile", "atomic"):
+            ls.zeroSystem()
+            na.assemble_scalar_diff(ls, mesh, d["p"], d["mu"], shifted=shifted, mode=mode)
+            _, _, v, r = ls.csr()
+            check("diffusion shifted=%d %s" % (shifted, mode), v, r,
+                  *oracle.assemble_scalar_diff(g, conn, X, f["p"], f["mu"], shifted=shifted), g.row_ptr)
+    mdot = torch.zeros((E, 12), dtype=torch.float64, device=DEV)
+    for sm, sp, red in ((0, 0, 0), (0, 0, 1), (1, 1, 0)) if big else np.ndindex(2, 2, 2):
+        ls.zeroSystem()
+        na.assemble_continuity(ls, mesh, rho[2], d["p"], u[2], d["gp"], tau=0.7, shift_mdot=sm, shift_poisson=sp,
+                               reduced_sens=red, mode="gather", mdot_out=mdot)
+        _, _, v, r = ls.csr()
+        ov, orhs = oracle.assemble_continuity(g, conn, X, f["rho"][2], f["p"], f["u"][2], f["gp"], 0.7, sm, sp, red)
+        check("continuity %d%d%d" % (sm, sp, red), v, r, ov, orhs, g.row_ptr)
+        om = oracle.compute_mdot(conn, X, f["rho"][2], f["p"], f["u"][2], f["gp"], 0.7, sm, sp)
+        assert np.abs(mdot.cpu().numpy() - om.reshape(E, 12)).max() <= TOL * np.abs(om).max()
+        na.compute_mdot(mesh, rho[2], d["p"], u[2], d["gp"], mdot, tau=0.7, shift_mdot=sm, shift_poisson=sp)
+        assert np.abs(mdot.cpu().numpy() - om.reshape(E, 12)).max() <= TOL * np.abs(om).max()
+    # a second pass onto the assembled system accumulates
+    na.assemble_continuity(ls, mesh, rho[2], d["p"], u[2], d["gp"], tau=0.7, shift_mdot=sm, shift_poisson=sp,
+                           reduced_sens=red, mode="tile")
+    _, _, v, r = ls.csr()
+    check("accumulate", v, r, 2 * ov, 2 * orhs, g.row_ptr)
+    vol, grad = torch.zeros(N, dtype=torch.float64, device=DEV), torch.zeros((N, 3), dtype=torch.float64, device=DEV)
+    na.compute_dual_volume(mesh, vol)
+    ovol = oracle.dual_nodal_volume(conn, X)
+    assert np.abs(vol.cpu().numpy() - ovol).max() <= TOL * ovol.max()
+    na.compute_nodal_gradient(mesh, d["p"], vol, grad)
+    og = oracle.nodal_grad(conn, X, f["p"], ovol)
+    assert np.abs(grad.cpu().numpy() - og).max() <= TOL * np.abs(og).max()
+
+
+@pytest.mark.parametrize("name", list(MESHES))
+def test_momentum_rows(oracle, name):
+    print("case: momentum row tiles on", name, flush=True)
+    X, conn, f, rng = problem(name, 4)
+    N = X.shape[0]
+    mesh = na.Mesh(X, conn)
+    d = {k: dev(v) for k, v in f.items()}
+    rho, u = [d["rho"][i].contiguous() for i in range(3)], [d["u"][i].contiguous() for i in range(3)]
+    g1, g3 = oracle.graph_build(N, conn), oracle.graph_build(N, conn, num_dof=3)
+    gam, dt = (1.5, -2.0, 0.5), 0.3
+    l1, l3 = na.LinearSystem(1), na.LinearSystem(3)
+    for ls in (l1, l3):
+        ls.buildElemToNodeGraph(mesh)
+        ls.finalizeLinearSystem()
+    fits = np.diff(g1.row_ptr).max() <= 35  # longer rows run the atomic form
+    big = N > 4000
+    for skew, shifted, divu in ((0, 0, 0.0), (0, 0, 1.0)) if big else ((0, 0, 0.0), (0, 0, 1.0), (1, 0, 0.0), (1, 1, 1.0)):
+        a3 = oracle.assemble_momentum(g3, conn, X, f["u"][2], f["mu"], f["mdot"], divu, skew, shifted)
+        a1 = oracle.momentum_segregated(g1, g3, conn, X, f["u"][2], f["mu"], f["mdot"], divu, skew, shifted)
+        args = (mesh, u[2], d["mu"], d["mdot"])
+        kw = dict(include_divu=divu, skew=bool(skew), shifted=bool(shifted))
+        for mode in ("tile", "atomic") if fits else ("atomic",):
+            l3.zeroSystem()
+            na.assemble_momentum(l3, *args, mode=mode, **kw)
+            _, _, v, r = l3.csr()
+            check("coupled %s %d%d %g" % (mode, skew, shifted, divu), v, r, *a3, g3.row_ptr)
+        rhs3 = torch.zeros((3, N), dtype=torch.float64, device=DEV)
+        l1.zeroSystem()
+        na.assemble_momentum_segregated(l1, *args, rhs3, **kw)
+        _, _, v, _ = l1.csr()
+        check("segregated %d%d %g" % (skew, shifted, divu), v, rhs3.cpu().numpy().ravel(), a1[0], a1[1].ravel(),
+              g1.row_ptr)
+        for lumped, balanced in ((False, False), (True, True)):
+            m3 = oracle.assemble_momentum_mass(g3, conn, X, f["rho"], f["u"], f["gp"], dt, gam, lumped, balanced)
+            for states in (u, [u[0], u[1], u[2].clone()]):  # the Np1 state is the advected field, or another array
+                l3.zeroSystem()
+                na.assemble_momentum_with_mass(l3, *args, rho, states, d["gp"], dt, gamma=gam, lumped=lumped,
+                                               balanced_force=balanced, **kw)
+                _, _, v, r = l3.csr()
+                check("coupled + mass lumped=%d" % lumped, v, r, a3[0] + m3[0], a3[1] + m3[1], g3.row_ptr)
+            rhs3.zero_()
+            l1.zeroSystem()
+            na.assemble_momentum_with_mass_segregated(l1, *args, rho, u, d["gp"], dt, rhs3, gamma=gam, lumped=lumped,
+                                                      balanced_force=balanced, **kw)
+            _, _, v1, _ = l1.csr()
+            r1 = rhs3.cpu().numpy().copy()
+            rhs3.zero_()
+            l1.zeroSystem()
+            na.assemble_momentum_segregated(l1, *args, rhs3, **kw)
+            na.assemble_momentum_mass_segregated(l1, mesh, rho, u, d["gp"], dt, rhs3, gamma=gam, lumped=lumped,
+                                                 balanced_force=balanced)
+            _, _, v, _ = l1.csr()
+            check("segregated + mass, one pass and two", v, r1.ravel(), v1, rhs3.cpu().numpy().ravel(), g1.row_ptr)
+            check("segregated + mass rhs", None, r1.T.ravel(), None, a3[1] + m3[1], None)
+            l3.zeroSystem()
+            na.assemble_momentum_mass(l3, mesh, rho, u, d["gp"], dt, gamma=gam, lumped=lumped, balanced_force=balanced)
+            _, _, v, r = l3.csr()
+            check("mass alone lumped=%d" % lumped, v, r, *m3, g3.row_ptr)
