@@ -88,8 +88,8 @@ __global__ void k_elem_pos(const int32_t* __restrict__ conn, const int32_t* __re
                            int64_t nelem, uint64_t* __restrict__ pos, int* __restrict__ bad) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nelem * 8) return;
-  const int a = (int)(t / nelem);
-  const int64_t e = t - a * nelem;
+  const int64_t e = t >> 3;
+  const int a = (int)(t & 7);
   const int32_t row = lid[conn[8 * e + a]];
   const int32_t b0 = nrp[row];
   const int len = nrp[row + 1] - b0;
@@ -101,7 +101,7 @@ __global__ void k_elem_pos(const int32_t* __restrict__ conn, const int32_t* __re
     if (p >= len || p > 255 || nci[b0 + p] != key) atomicOr(bad, 1);
     packed |= (uint64_t)(p & 0xff) << (8 * c);
   }
-  pos[t] = packed;
+  pos[a * nelem + e] = packed;
 }
 
 // Expanded CSR for numDof > 1: row (a*nd+d) = node-row a with each column

@@ -116,115 +116,154 @@ struct V16<double> {
   }
 };
 
-// Coefficients part[j * gridDim.x + blk] = V_j . w over the chunks blk, blk + G,
-// ... of R rows (j < cnt), plus w . w as row cnt when with_self; w's chunk is
-// staged in LDS, one wavefront per basis vector, per-block sums kept in LDS.
+// sum over the lanes of a wave: DPP within each 16 lanes, two shuffles across them
+// (a sixth of the latency of six shuffles through LDS)
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_sum_dpp(double v) {
+  v += dpp_move<0xB1>(v);   // quad_perm 1 0 3 2
+  v += dpp_move<0x4E>(v);   // quad_perm 2 3 0 1
+  v += dpp_move<0x141>(v);  // row_half_mirror
+  v += dpp_move<0x140>(v);  // row_mirror
+  v += __shfl_xor(v, 16);
+  return v + __shfl_xor(v, 32);
+}
+
+// Coefficients part[j * gridDim.x + blockIdx.x] = V_j . w over the chunks
+// blockIdx.x, blockIdx.x + gridDim.x, ... of kDotRows rows (j < cnt), plus w . w as
+// row cnt when with_self.  A wave holds its part of w's chunk in registers and
+// takes the vectors j = 4 blockIdx.y + wave, + 4 gridDim.y, ...  Large systems run
+// one block to a chunk (w read four times, V once); small ones spread the vectors
+// over gridDim.y, because a chunk count far below the CU count leaves the chip
+// waiting on one block's serial walk over the basis (32^3, 25 vectors: 24.6 us with
+// 18 blocks).
+constexpr int kDotRows = 1024;
 template <typename TV>
 __global__ __launch_bounds__(kThreads) void k_gs_dots(const TV* __restrict__ V, int64_t ldv, int cnt, int with_self,
-                                                      const TV* __restrict__ w, int64_t n, int R,
+                                                      const TV* __restrict__ w, int64_t n,
                                                       double* __restrict__ part) {
-  extern __shared__ unsigned char smem_raw[];
-  TV* ws = reinterpret_cast<TV*>(smem_raw);         // [R]
-  double* acc = reinterpret_cast<double*>(ws + R);  // [cnt + 1]
-  constexpr int VN = V16<TV>::N;
+  extern __shared__ double acc[];  // [rows]; each row is one wave's
+  constexpr int VN = V16<TV>::N, U = kDotRows / 64 / VN;
   const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const int rows = cnt + (with_self ? 1 : 0);
-  for (int j = threadIdx.x; j < rows; j += blockDim.x) acc[j] = 0.0;
-  const int64_t nch = (n + R - 1) / R;
+  const int rows = cnt + (with_self ? 1 : 0), j0 = 4 * (int)blockIdx.y + wv, dj = 4 * (int)gridDim.y;
+  const int64_t nch = (n + kDotRows - 1) / kDotRows;
   for (int64_t c = blockIdx.x; c < nch; c += gridDim.x) {
-    const int64_t r0 = c * R;
-    const int m = (int)min<int64_t>(R, n - r0);
-    __syncthreads();
-    for (int t = threadIdx.x; t < m; t += blockDim.x) ws[t] = w[r0 + t];
-    __syncthreads();
-    const int mv = m / VN * VN;
-    for (int j = wv; j < rows; j += kThreads / 64) {
-      const TV* v = (j < cnt ? V + (int64_t)j * ldv : w) + r0;
-      double sj = 0.0;
-      for (int t = l * VN; t < mv; t += 64 * VN) {
-        double a[VN];
-        V16<TV>::load(v + t, a);
+    const int64_t r0 = c * kDotRows + l * VN;
+    const bool first = c == (int64_t)blockIdx.x, full = (c + 1) * kDotRows <= n;
+    double wr[U][VN];
 #pragma unroll
-        for (int u = 0; u < VN; ++u) sj += a[u] * (double)ws[t + u];
+    for (int u = 0; u < U; ++u) {
+      const int64_t i = r0 + u * 64 * VN;
+      if (full) {
+        V16<TV>::load(w + i, wr[u]);
+      } else {
+#pragma unroll
+        for (int k = 0; k < VN; ++k) wr[u][k] = i + k < n ? (double)w[i + k] : 0.0;
       }
-      for (int t = mv + l; t < m; t += 64) sj += (double)v[t] * (double)ws[t];
-      sj = wave_sum(sj);
-      if (l == 0) acc[j] += sj;
+    }
+    for (int j = j0; j < rows; j += dj) {
+      const TV* v = (j < cnt ? V + (int64_t)j * ldv : w) + r0;
+      double sj[2] = {0.0, 0.0};
+      if (full) {
+        double a[U][VN];
+#pragma unroll
+        for (int u = 0; u < U; ++u) V16<TV>::load(v + u * 64 * VN, a[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int k = 0; k < VN; ++k) sj[k & 1] += a[u][k] * wr[u][k];
+      } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int k = 0; k < VN; ++k)
+            if (r0 + u * 64 * VN + k < n) sj[k & 1] += (double)v[u * 64 * VN + k] * wr[u][k];
+      }
+      const double sum = wave_sum_dpp(sj[0] + sj[1]);
+      if (l == 0) acc[j] = first ? sum : acc[j] + sum;
     }
   }
   __syncthreads();
-  for (int j = threadIdx.x; j < rows; j += blockDim.x) part[(int64_t)j * gridDim.x + blockIdx.x] = acc[j];
+  for (int j = j0; j < rows; j += dj)
+    if (l == 0) part[(int64_t)j * gridDim.x + blockIdx.x] = acc[j];
 }
 
-// w -= V h (FP64 accumulation); each thread owns VN consecutive rows
-template <typename TV>
+// w -= V h (FP64 accumulation); NORM: part[blk] = ||w||^2 (partial).  A wave owns
+// 64 VN consecutive rows at a time.  JS = 4: the block's waves take the vectors in
+// turns for the same rows and meet in LDS, which gives small systems four times the
+// waves and a quarter of the serial chain (32^3, 25 vectors on average: 12 us with
+// JS = 1, 4.7 us so).
+template <typename TV, bool NORM, int JS>
 __global__ __launch_bounds__(kThreads) void k_gs_update(const TV* __restrict__ V, int64_t ldv, int cnt,
-                                                        const double* __restrict__ h, TV* __restrict__ w, int64_t n) {
+                                                        const double* __restrict__ h, TV* __restrict__ w, int64_t n,
+                                                        double* __restrict__ part) {
   constexpr int VN = V16<TV>::N;
+  __shared__ double meet[JS > 1 ? JS - 1 : 1][64][VN];
+  const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, jw = JS > 1 ? wv : 0;
   const int64_t ng = (n + VN - 1) / VN;
-  for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < ng; g += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t i0 = g * VN;
-    if (i0 + VN <= n) {
-      double a[VN];
-      V16<TV>::load(w + i0, a);
-      for (int j = 0; j < cnt; ++j) {
-        double v[VN];
-        V16<TV>::load(V + (int64_t)j * ldv + i0, v);
-        const double hj = h[j];
-#pragma unroll
-        for (int u = 0; u < VN; ++u) a[u] -= hj * v[u];
-      }
-#pragma unroll
-      for (int u = 0; u < VN; ++u) w[i0 + u] = (TV)a[u];
-    } else {
-      for (int64_t i = i0; i < n; ++i) {
-        double t = (double)w[i];
-        for (int j = 0; j < cnt; ++j) t -= h[j] * (double)V[(int64_t)j * ldv + i];
-        w[i] = (TV)t;
-      }
-    }
-  }
-}
-
-// pass-2 update with the norm of the result: w -= V h, part[blk] = ||w||^2 (partial);
-// each thread owns VN consecutive rows
-template <typename TV>
-__global__ __launch_bounds__(kThreads) void k_gs_update_norm(const TV* __restrict__ V, int64_t ldv, int cnt,
-                                                             const double* __restrict__ h, TV* __restrict__ w,
-                                                             int64_t n, double* __restrict__ part) {
-  constexpr int VN = V16<TV>::N;
   double s2 = 0.0;
-  const int64_t ng = (n + VN - 1) / VN;
-  for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < ng; g += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t i0 = g * VN;
+  for (int64_t g0 = (int64_t)blockIdx.x * (JS > 1 ? 64 : kThreads); g0 < ng;
+       g0 += (int64_t)gridDim.x * (JS > 1 ? 64 : kThreads)) {
+    const int64_t i0 = (g0 + (JS > 1 ? l : (int)threadIdx.x)) * VN;
+    const bool full = i0 + VN <= n;
     double a[VN];
-    if (i0 + VN <= n) {
-      V16<TV>::load(w + i0, a);
-      for (int j = 0; j < cnt; ++j) {
+#pragma unroll
+    for (int u = 0; u < VN; ++u) a[u] = 0.0;
+    if (full) {
+      int j = jw;
+      for (; j + 3 * JS < cnt; j += 4 * JS) {
+        double v[4][VN];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) V16<TV>::load(V + (int64_t)(j + k * JS) * ldv + i0, v[k]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int u = 0; u < VN; ++u) a[u] += h[j + k * JS] * v[k][u];
+      }
+      for (; j < cnt; j += JS) {
         double v[VN];
         V16<TV>::load(V + (int64_t)j * ldv + i0, v);
-        const double hj = h[j];
 #pragma unroll
-        for (int u = 0; u < VN; ++u) a[u] -= hj * v[u];
+        for (int u = 0; u < VN; ++u) a[u] += h[j] * v[u];
       }
+    } else if (i0 < n) {
+      for (int j = jw; j < cnt; j += JS)
 #pragma unroll
-      for (int u = 0; u < VN; ++u) {
-        const TV t = (TV)a[u];
-        w[i0 + u] = t;
-        s2 += (double)t * (double)t;
+        for (int u = 0; u < VN; ++u)
+          if (i0 + u < n) a[u] += h[j] * (double)V[(int64_t)j * ldv + i0 + u];
+    }
+    if (JS > 1) {
+      __syncthreads();  // the last turn's readers are done
+      if (wv > 0) {
+#pragma unroll
+        for (int u = 0; u < VN; ++u) meet[wv - 1][l][u] = a[u];
       }
-    } else {
-      for (int64_t i = i0; i < n; ++i) {
-        double t = (double)w[i];
-        for (int j = 0; j < cnt; ++j) t -= h[j] * (double)V[(int64_t)j * ldv + i];
-        const TV tv = (TV)t;
-        w[i] = tv;
-        s2 += (double)tv * (double)tv;
+      __syncthreads();
+      if (wv == 0) {
+#pragma unroll
+        for (int k = 0; k < JS - 1; ++k)
+#pragma unroll
+          for (int u = 0; u < VN; ++u) a[u] += meet[k][l][u];
       }
     }
+    if (jw == 0) {
+#pragma unroll
+      for (int u = 0; u < VN; ++u)
+        if (i0 + u < n) {
+          const TV t = (TV)((double)w[i0 + u] - a[u]);
+          w[i0 + u] = t;
+          s2 += (double)t * (double)t;
+        }
+    }
   }
-  s2 = block_sum(s2);
-  if (threadIdx.x == 0) part[blockIdx.x] = s2;
+  if (NORM) {
+    s2 = block_sum(s2);
+    if (threadIdx.x == 0) part[blockIdx.x] = s2;
+  }
 }
 
 // ------------------------------------------------------------ SpMV (CSR-stream)
@@ -750,180 +789,206 @@ __global__ void k_take_sell(const int32_t* __restrict__ src, const double* __res
   if (q < n) out[q] = src[q] >= 0 ? (T)v[src[q]] : T(0);
 }
 
+// Part `part` of P of a chunk row's products: entries part, part + P, ... of w.
+// P = 1, 2: the plain loop (measured best where the launch fills the chip); the
+// entries stream through once, so they are loaded non-temporally.  More: a few
+// entries to a lane, all columns and values loaded before the first gather, so that
+// a launch with few waves takes three memory round trips, not a chain of them, and
+// cached, because such a matrix stays in the L2s from one sweep to the next.
+template <typename T, int P>
+__device__ __forceinline__ T sell_part(const T* __restrict__ val, const int32_t* __restrict__ cs, int64_t o, int w,
+                                       int lane, int part, const T* __restrict__ x) {
+  T s = T(0);
+  if constexpr (P <= 2) {
+#pragma unroll NALU_SPARSE_UNROLL
+    for (int q = part; q < w; q += P)
+      s += __builtin_nontemporal_load(&val[o + lane + q * 64]) * x[__builtin_nontemporal_load(&cs[o + lane + q * 64])];
+  } else {
+    for (int q0 = part; q0 < w; q0 += 4 * P) {
+      int32_t c[4];
+      T v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int64_t at = o + lane + (int64_t)min(q0 + i * P, w - 1) * 64;
+        c[i] = cs[at];
+        v[i] = val[at];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (q0 + i * P < w) s += v[i] * x[c[i]];
+    }
+  }
+  return s;
+}
+
+// The row products of the P waves of one chunk, in wave order, in the first wave.
+template <typename T, int P>
+__device__ __forceinline__ T sell_meet(T (*meet)[64], int part, int lane, T s) {
+  if (part > 0) meet[part - 1][lane] = s;
+  __syncthreads();
+  if (part == 0) {
+#pragma unroll
+    for (int k = 0; k < P - 1; ++k) s += meet[k][lane];
+  }
+  return s;
+}
+// blocks of a launch with P waves to a chunk: max(1, 4 / P) chunks each
+template <int P>
+struct SellBlock {
+  static constexpr int threads = P <= 4 ? kThreads : 64 * P;
+  static constexpr int chunks = P <= 4 ? 4 / P : 1;
+};
+
 // y = (D + L + U) x  (mode 0)  or  y = b - (D + L + U) x  (mode 1); the matrix
 // entries stream through once (non-temporal loads), the gathered x stays cached
-template <typename T, typename TY>
-__global__ __launch_bounds__(kThreads) void k_sell_spmv(const SellChunk* __restrict__ ch, int64_t nch,
-                                                        const int32_t* __restrict__ lcs, const T* __restrict__ lval,
-                                                        const int32_t* __restrict__ ucs, const T* __restrict__ uval,
-                                                        const T* __restrict__ dv, const T* __restrict__ x,
-                                                        TY* __restrict__ y, const TY* __restrict__ b, int mode) {
-  const int64_t c = (int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (c >= nch) return;
-  const SellChunk k = ch[c];
+template <typename T, typename TY, int P>
+__global__ __launch_bounds__(SellBlock<P>::threads) void k_sell_spmv(
+    const SellChunk* __restrict__ ch, int64_t nch, const int32_t* __restrict__ lcs, const T* __restrict__ lval,
+    const int32_t* __restrict__ ucs, const T* __restrict__ uval, const T* __restrict__ dv, const T* __restrict__ x,
+    TY* __restrict__ y, const TY* __restrict__ b, int mode) {
+  __shared__ T meet[SellBlock<P>::chunks][P > 1 ? P - 1 : 1][64];
+  // wave-uniform, so that the chunk header is a scalar load
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, part = wave % P,
+            mine = wave / P;
+  const int64_t c = (int64_t)blockIdx.x * SellBlock<P>::chunks + mine;
+  if (P == 1 && c >= nch) return;
+  SellChunk k{};
+  if (c < nch) k = ch[c];
   const bool act = lane < k.nrows;
   const int row = k.row0 + (act ? lane : 0);
-  T s = dv[row] * x[row];
-#pragma unroll NALU_SPARSE_UNROLL
-  for (int q = 0; q < k.lw; ++q) {
-    s += __builtin_nontemporal_load(&lval[k.loff + lane + q * 64]) *
-         x[__builtin_nontemporal_load(&lcs[k.loff + lane + q * 64])];
-  }
-#pragma unroll NALU_SPARSE_UNROLL
-  for (int q = 0; q < k.uw; ++q) {
-    s += __builtin_nontemporal_load(&uval[k.uoff + lane + q * 64]) *
-         x[__builtin_nontemporal_load(&ucs[k.uoff + lane + q * 64])];
-  }
-  if (act) y[row] = mode ? (TY)((T)b[row] - s) : (TY)s;
+  T s = T(0);
+  if (part == 0 && (P == 1 || c < nch)) s = dv[row] * x[row];
+  s += sell_part<T, P>(lval, lcs, k.loff, k.lw, lane, part, x);
+  s += sell_part<T, P>(uval, ucs, k.uoff, k.uw, lane, part, x);
+  if constexpr (P > 1) s = sell_meet<T, P>(meet[mine], part, lane, s);
+  if (act && part == 0) y[row] = mode ? (TY)((T)b[row] - s) : (TY)s;
 }
 
-// forward sweep over the chunks [c0, c1) of one color: z = (r - L z) / d.
-// Two lanes per row (128 threads per 64-row chunk, even / odd entries, the
-// halves combined through LDS) double the loads in flight per chunk; the matrix
-// entries are read once per sweep, so they are loaded non-temporally and the
-// gathered z entries keep the cache.  Each XCD sweeps a contiguous range of the
-// color's chunks, so neighbouring rows gather z through the same L2.
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_sell_fwd(const SellChunk* __restrict__ ch, int64_t c0, int64_t c1,
-                                                       const int32_t* __restrict__ lcs, const T* __restrict__ lval,
-                                                       const T* __restrict__ invd, const T* __restrict__ r,
-                                                       T* __restrict__ z) {
-  __shared__ T part[kThreads / 2];
-  const int64_t nb = (c1 - c0 + 1) / 2;  // blocks of two chunks, XCD-contiguous ranges
-  const int64_t pos = xcd_block(blockIdx.x, nb);
-  const int64_t c = pos < 0 ? c1 : c0 + pos * (kThreads / 128) + (threadIdx.x >> 7);
-  const int lane = threadIdx.x & 63;
-  const int half = (threadIdx.x >> 6) & 1;
-  const int slot = (threadIdx.x >> 7) * 64 + lane;
-  const bool ok = c < c1;
+// Sweeps over the chunks [c0, c1) of one color: forward z = (r - L z) / d, backward
+// in place z = z - (U z) / d.  Several waves to a chunk double (P = 2) the loads in
+// flight; the matrix entries are read once per sweep, so they are loaded
+// non-temporally and the gathered z entries keep the cache.  Each XCD sweeps a
+// contiguous range of the color's chunks, so neighbouring rows gather z through the
+// same L2.
+template <typename T, bool UPPER, int P>
+__global__ __launch_bounds__(SellBlock<P>::threads) void k_sell_sweep(
+    const SellChunk* __restrict__ ch, int64_t c0, int64_t c1, const int32_t* __restrict__ cs,
+    const T* __restrict__ val, const T* __restrict__ invd, const T* __restrict__ r, T* __restrict__ z) {
+  __shared__ T meet[SellBlock<P>::chunks][P - 1][64];
+  constexpr int C = SellBlock<P>::chunks;
+  const int64_t pos = xcd_block(blockIdx.x, (c1 - c0 + C - 1) / C);
+  // wave-uniform, so that the chunk header is a scalar load
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, part = wave % P,
+            mine = wave / P;
+  const int64_t c = pos < 0 ? c1 : c0 + pos * C + mine;
   SellChunk k{};
-  if (ok) k = ch[c];
-  const bool act = ok && lane < k.nrows;
-  T s = T(0);
-  if (act) {
-#pragma unroll NALU_SPARSE_UNROLL
-    for (int q = half; q < k.lw; q += 2)
-      s += __builtin_nontemporal_load(&lval[k.loff + lane + q * 64]) *
-           z[__builtin_nontemporal_load(&lcs[k.loff + lane + q * 64])];
+  if (c < c1) k = ch[c];
+  const bool act = lane < k.nrows;
+  const int row = k.row0 + (act ? lane : 0);
+  T d = T(0), rr = T(0);  // loaded early: they do not depend on the products
+  if (act && part == 0) {
+    d = invd[row];
+    rr = UPPER ? z[row] : r[row];
   }
-  if (half == 1) part[slot] = s;
-  __syncthreads();
-  if (!act || half == 1) return;
-  const int row = k.row0 + lane;
-  s += part[slot];
-  z[row] = (r[row] - s) * invd[row];
-}
-
-// backward sweep over the chunks of one color, in place: z = y - (U z) / d
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_sell_bwd(const SellChunk* __restrict__ ch, int64_t c0, int64_t c1,
-                                                       const int32_t* __restrict__ ucs, const T* __restrict__ uval,
-                                                       const T* __restrict__ invd, T* __restrict__ z) {
-  __shared__ T part[kThreads / 2];
-  const int64_t nb = (c1 - c0 + 1) / 2;  // blocks of two chunks, XCD-contiguous ranges
-  const int64_t pos = xcd_block(blockIdx.x, nb);
-  const int64_t c = pos < 0 ? c1 : c0 + pos * (kThreads / 128) + (threadIdx.x >> 7);
-  const int lane = threadIdx.x & 63;
-  const int half = (threadIdx.x >> 6) & 1;
-  const int slot = (threadIdx.x >> 7) * 64 + lane;
-  const bool ok = c < c1;
-  SellChunk k{};
-  if (ok) k = ch[c];
-  const bool act = ok && lane < k.nrows;
-  T s = T(0);
-  if (act) {
-#pragma unroll NALU_SPARSE_UNROLL
-    for (int q = half; q < k.uw; q += 2)
-      s += __builtin_nontemporal_load(&uval[k.uoff + lane + q * 64]) *
-           z[__builtin_nontemporal_load(&ucs[k.uoff + lane + q * 64])];
-  }
-  if (half == 1) part[slot] = s;
-  __syncthreads();
-  if (!act || half == 1) return;
-  const int row = k.row0 + lane;
-  s += part[slot];
-  z[row] = z[row] - s * invd[row];
+  T s = sell_part<T, P>(val, cs, UPPER ? k.uoff : k.loff, UPPER ? k.uw : k.lw, lane, part, z);
+  s = sell_meet<T, P>(meet[mine], part, lane, s);
+  if (act && part == 0) z[row] = UPPER ? rr - s * d : (rr - s) * d;
 }
 
 // q = A p (SELL copy); per-block partials of p.q
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_sell_spmv_dot(const SellChunk* __restrict__ ch, int64_t nch,
-                                                            const int32_t* __restrict__ lcs, const T* __restrict__ lval,
-                                                            const int32_t* __restrict__ ucs, const T* __restrict__ uval,
-                                                            const T* __restrict__ dv, const T* __restrict__ x,
-                                                            T* __restrict__ y, double* __restrict__ part,
-                                                            const CgState* __restrict__ st) {
+template <typename T, int P>
+__global__ __launch_bounds__(SellBlock<P>::threads) void k_sell_spmv_dot(
+    const SellChunk* __restrict__ ch, int64_t nch, const int32_t* __restrict__ lcs, const T* __restrict__ lval,
+    const int32_t* __restrict__ ucs, const T* __restrict__ uval, const T* __restrict__ dv, const T* __restrict__ x,
+    T* __restrict__ y, double* __restrict__ part_out, const CgState* __restrict__ st) {
+  __shared__ T meet[SellBlock<P>::chunks][P > 1 ? P - 1 : 1][64];
   if (st->done) return;
-  const int64_t c = (int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  double d = 0.0;
-  if (c < nch) {
-    const SellChunk k = ch[c];
-    const bool act = lane < k.nrows;
-    const int row = k.row0 + (act ? lane : 0);
-    T s = dv[row] * x[row];
-#pragma unroll NALU_SPARSE_UNROLL
-    for (int q = 0; q < k.lw; ++q) {
-      s += __builtin_nontemporal_load(&lval[k.loff + lane + q * 64]) *
-           x[__builtin_nontemporal_load(&lcs[k.loff + lane + q * 64])];
-    }
-#pragma unroll NALU_SPARSE_UNROLL
-    for (int q = 0; q < k.uw; ++q) {
-      s += __builtin_nontemporal_load(&uval[k.uoff + lane + q * 64]) *
-           x[__builtin_nontemporal_load(&ucs[k.uoff + lane + q * 64])];
-    }
-    if (act) {
-      y[row] = s;
-      d = (double)s * (double)x[row];
-    }
+  // wave-uniform, so that the chunk header is a scalar load
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, part = wave % P,
+            mine = wave / P;
+  const int64_t c = (int64_t)blockIdx.x * SellBlock<P>::chunks + mine;
+  SellChunk k{};
+  if (c < nch) k = ch[c];
+  const bool act = lane < k.nrows;
+  const int row = k.row0 + (act ? lane : 0);
+  T s = T(0), xr = T(0);
+  if (act && part == 0) {
+    xr = x[row];
+    s = dv[row] * xr;
   }
-  d = block_sum(d);
-  if (threadIdx.x == 0) part[blockIdx.x] = d;
+  s += sell_part<T, P>(lval, lcs, k.loff, k.lw, lane, part, x);
+  s += sell_part<T, P>(uval, ucs, k.uoff, k.uw, lane, part, x);
+  if constexpr (P > 1) s = sell_meet<T, P>(meet[mine], part, lane, s);
+  double d = 0.0;
+  if (act && part == 0) {
+    y[row] = s;
+    d = (double)s * (double)xr;
+  }
+  if constexpr (SellBlock<P>::chunks == 1) {
+    if (part > 0) return;
+    d = wave_sum_dpp(d);
+  } else {
+    d = block_sum(d);
+  }
+  if (threadIdx.x == 0) part_out[blockIdx.x] = d;
 }
 
-// Sweeps of the fused CG: as k_sell_fwd / k_sell_bwd, plus the partial sums
-// r.z of the rows they finalize (the forward sweep of the last color, every
-// backward sweep) in part[off + block].  All return at once after convergence.
-template <typename T, bool UPPER>
-__global__ __launch_bounds__(kThreads) void k_sell_sweep_dot(const SellChunk* __restrict__ ch, int64_t c0,
-                                                             int64_t c1, const int32_t* __restrict__ cs, const T* __restrict__ val,
-                                                             const T* __restrict__ invd, const T* __restrict__ r,
-                                                             T* __restrict__ z, int dot, double* __restrict__ part,
-                                                             int off, const CgState* __restrict__ st) {
-  __shared__ T hpart[kThreads / 2];
+// Sweeps of the fused CG: as k_sell_sweep, plus the partial sums r.z of the rows
+// they finalize (the forward sweep of the last color, every backward sweep) in
+// part[off + block].  All return at once after convergence.
+template <typename T, bool UPPER, int P>
+__global__ __launch_bounds__(SellBlock<P>::threads) void k_sell_sweep_dot(
+    const SellChunk* __restrict__ ch, int64_t c0, int64_t c1, const int32_t* __restrict__ cs,
+    const T* __restrict__ val, const T* __restrict__ invd, const T* __restrict__ r, T* __restrict__ z, int dot,
+    double* __restrict__ part_out, int off, const CgState* __restrict__ st) {
+  __shared__ T meet[SellBlock<P>::chunks][P - 1][64];
   if (st->done) return;
-  const int64_t nb = (c1 - c0 + 1) / 2;
-  const int64_t pos = xcd_block(blockIdx.x, nb);
-  const int64_t c = pos < 0 ? c1 : c0 + pos * (kThreads / 128) + (threadIdx.x >> 7);
-  const int lane = threadIdx.x & 63;
-  const int half = (threadIdx.x >> 6) & 1;
-  const int hslot = (threadIdx.x >> 7) * 64 + lane;
-  const bool ok = c < c1;
+  constexpr int C = SellBlock<P>::chunks;
+  const int64_t pos = xcd_block(blockIdx.x, (c1 - c0 + C - 1) / C);
+  // wave-uniform, so that the chunk header is a scalar load
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, part = wave % P,
+            mine = wave / P;
+  const int64_t c = pos < 0 ? c1 : c0 + pos * C + mine;
   SellChunk k{};
-  if (ok) k = ch[c];
-  const bool act = ok && lane < k.nrows;
-  T s = T(0);
-  if (act) {
-    const int w = UPPER ? k.uw : k.lw;
-    const int64_t o = UPPER ? k.uoff : k.loff;
-#pragma unroll NALU_SPARSE_UNROLL
-    for (int q = half; q < w; q += 2)
-      s += __builtin_nontemporal_load(&val[o + lane + q * 64]) * z[__builtin_nontemporal_load(&cs[o + lane + q * 64])];
+  if (c < c1) k = ch[c];
+  const bool act = lane < k.nrows;
+  const int row = k.row0 + (act ? lane : 0);
+  T d = T(0), rr = T(0), zr = T(0);
+  if (act && part == 0) {
+    d = invd[row];
+    rr = r[row];
+    if (UPPER) zr = z[row];
   }
-  if (half == 1) hpart[hslot] = s;
-  __syncthreads();
-  double d = 0.0;
-  if (act && half == 0) {
-    const int row = k.row0 + lane;
-    s += hpart[hslot];
-    const T zr = UPPER ? z[row] - s * invd[row] : (r[row] - s) * invd[row];
+  T s = sell_part<T, P>(val, cs, UPPER ? k.uoff : k.loff, UPPER ? k.uw : k.lw, lane, part, z);
+  s = sell_meet<T, P>(meet[mine], part, lane, s);
+  double rz = 0.0;
+  if (act && part == 0) {
+    zr = UPPER ? zr - s * d : (rr - s) * d;
     z[row] = zr;
-    if (dot) d = (double)r[row] * (double)zr;
+    if (dot) rz = (double)rr * (double)zr;
   }
   if (!dot) return;  // grid-uniform
-  d = block_sum(d);
-  if (threadIdx.x == 0) part[off + blockIdx.x] = d;
+  if constexpr (C == 1) {
+    if (part > 0) return;
+    rz = wave_sum_dpp(rz);
+  } else {
+    rz = block_sum(rz);
+  }
+  if (threadIdx.x == 0) part_out[off + blockIdx.x] = rz;
+}
+
+// Waves to a chunk by the chunks of the launch: below these counts a launch does
+// not fill the chip and its time is one wave's chain plus the launch (about 2 us).
+// Sweeps, forward / backward: 74 chunks (32^3) 4.4 / 4.4 us with two waves, 3.3 / 3.3
+// with eight; 536 chunks (64^3, with r.z) 5.2 / 6.0 and 5.0 / 5.4; 4194 chunks (128^3)
+// four waves were already slower than two.  Product: 562 chunks (32^3) 9.2 us with
+// one wave, 6.2 with four; 4292 chunks (64^3) run at 4.9 TB/s with one.
+constexpr int64_t kFewSweepChunks = 1024, kFewSpmvChunks = 2048;
+inline bool few_sweep(int64_t nch) { return nch <= kFewSweepChunks; }
+inline bool few_spmv(int64_t nch) { return nch <= kFewSpmvChunks; }
+template <int P>
+inline unsigned sell_grid(int64_t nch) {
+  return (unsigned)std::max<int64_t>(1, (nch + SellBlock<P>::chunks - 1) / SellBlock<P>::chunks);
 }
 
 // Batched forms for NR right-hand sides interleaved [n][NR] (one matrix read
@@ -1178,9 +1243,13 @@ void pspmv(nalu_linsys* ls, const T* x, TY* y, const TY* b, int mode) {
   const int kc = sparse_kernel_choice();
   if (kc == 64) {
     const int64_t nch = ls->sell_nchunks;
-    hipLaunchKernelGGL((k_sell_spmv<T, TY>), dim3((unsigned)std::max<int64_t>(1, (nch + 3) / 4)), dim3(kThreads), 0,
-                       ls->stream, reinterpret_cast<const SellChunk*>(ls->sell_chunks.p), nch, sell_cols(ls, false),
-                       sell_vals<T>(ls, false), sell_cols(ls, true), sell_vals<T>(ls, true), A.dv, x, y, b, mode);
+    auto go = [&](auto kern, unsigned grid, int threads) {
+      hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), 0, ls->stream,
+                         reinterpret_cast<const SellChunk*>(ls->sell_chunks.p), nch, sell_cols(ls, false),
+                         sell_vals<T>(ls, false), sell_cols(ls, true), sell_vals<T>(ls, true), A.dv, x, y, b, mode);
+    };
+    if (few_spmv(nch)) go(k_sell_spmv<T, TY, 4>, sell_grid<4>(nch), SellBlock<4>::threads);
+    else go(k_sell_spmv<T, TY, 1>, sell_grid<1>(nch), SellBlock<1>::threads);
     return;
   }
   if (kc == 8 || kc == 4) {
@@ -1212,18 +1281,19 @@ void psgs(nalu_linsys* ls, const T* r, T* z) {
   if (kc == 64) {
     const SellChunk* ch = reinterpret_cast<const SellChunk*>(ls->sell_chunks.p);
     const auto& ccp = ls->sell_color_ptr;
-    for (int c = 0; c < ls->num_colors; ++c) {
+    auto sweep = [&](int c, auto upper) {
+      constexpr bool UP = decltype(upper)::value;
       const int64_t c0 = ccp[c], c1 = ccp[c + 1];
-      if (c1 > c0)
-        hipLaunchKernelGGL(k_sell_fwd<T>, dim3((unsigned)xcd_grid((c1 - c0 + 1) / 2)), dim3(kThreads), 0, s, ch,
-                           c0, c1, sell_cols(ls, false), sell_vals<T>(ls, false), A.invd, r, z);
-    }
-    for (int c = ls->num_colors - 2; c >= 0; --c) {  // the last color has no U entries
-      const int64_t c0 = ccp[c], c1 = ccp[c + 1];
-      if (c1 > c0)
-        hipLaunchKernelGGL(k_sell_bwd<T>, dim3((unsigned)xcd_grid((c1 - c0 + 1) / 2)), dim3(kThreads), 0, s, ch,
-                           c0, c1, sell_cols(ls, true), sell_vals<T>(ls, true), A.invd, z);
-    }
+      if (c1 <= c0) return;
+      auto go = [&](auto kern, unsigned grid, int threads) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)xcd_grid(grid)), dim3(threads), 0, s, ch, c0, c1, sell_cols(ls, UP),
+                           sell_vals<T>(ls, UP), A.invd, r, z);
+      };
+      if (few_sweep(c1 - c0)) go(k_sell_sweep<T, UP, 8>, sell_grid<8>(c1 - c0), SellBlock<8>::threads);
+      else go(k_sell_sweep<T, UP, 2>, sell_grid<2>(c1 - c0), SellBlock<2>::threads);
+    };
+    for (int c = 0; c < ls->num_colors; ++c) sweep(c, std::false_type{});
+    for (int c = ls->num_colors - 2; c >= 0; --c) sweep(c, std::true_type{});  // the last color has no U entries
     return;
   }
   if (kc == 8 || kc == 4) {
@@ -1437,10 +1507,25 @@ int gmres_t(nalu_linsys* ls, const double* b, double* x, int m, int maxit, doubl
   // solve only computes a correction, the FP64 outer residual decides).
   constexpr int kGsBlocks = 2048;
   const bool always2 = std::is_same<TV, double>::value;
-  const int R_dots = 2048;
-  const unsigned nb_dots = (unsigned)std::min<int64_t>(kGsBlocks, (n + R_dots - 1) / R_dots);
-  const size_t lds_dots = (size_t)R_dots * sizeof(TV) + (size_t)(m + 2) * 8;
-  const unsigned nb_upd = red_blocks((n + 3) / 4);
+  // dots: one block to a chunk of rows, the vectors spread over as many more as
+  // make about 1024 blocks
+  const unsigned nb_dots = (unsigned)std::min<int64_t>(kGsBlocks, (n + kDotRows - 1) / kDotRows);
+  const size_t lds_dots = (size_t)(m + 2) * 8;
+  auto dots_grid = [&](int rows) {
+    return dim3(nb_dots, (unsigned)std::max<int64_t>(1, std::min<int64_t>((rows + 3) / 4, 1024 / nb_dots)));
+  };
+  // updates: the vectors split over a block's waves while that still leaves few
+  // enough blocks (partial norms)
+  const int64_t wave_rows = 64 * V16<TV>::N;
+  const bool split_upd = (n + wave_rows - 1) / wave_rows <= kGsBlocks;
+  const unsigned nb_upd = split_upd ? (unsigned)((n + wave_rows - 1) / wave_rows) : red_blocks((n + 3) / 4);
+  auto update = [&](int cnt, const double* h, TV* w, bool norm) {
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(nb_upd), dim3(kThreads), 0, s, V, ldv, cnt, h, w, n, ls->red.p);
+    };
+    if (split_upd) norm ? go(k_gs_update<TV, true, 4>) : go(k_gs_update<TV, false, 4>);
+    else norm ? go(k_gs_update<TV, true, 1>) : go(k_gs_update<TV, false, 1>);
+  };
   NALU_REQUIRE((size_t)(m + 2) * kGsBlocks <= ls->red.n, NALU_ERR_STATE, "gmres: reduction workspace too small");
   // hA: pass-1 coefficients (+ ||w||^2 at k+1), hB: pass-2 coefficients, nrm: ||w_new||^2
   double* hA = hbuf;
@@ -1453,6 +1538,15 @@ int gmres_t(nalu_linsys* ls, const double* b, double* x, int m, int maxit, doubl
   std::vector<double> hcol(m + 2), y;
   (void)xt;
 
+  // The host decides from each column's norm whether to go on.  The next column's
+  // preconditioner and product are enqueued before it waits for that norm, so the
+  // device does not idle for the read (about 20 us of a 100 us iteration at 32^3);
+  // the last column of a cycle leaves one such product unused.
+  struct Event {
+    hipEvent_t e = nullptr;
+    Event() { NALU_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming)); }
+    ~Event() { (void)hipEventDestroy(e); }
+  } col_read;
   int iters = 0;
   double r0 = -1.0, rel = 1.0;
   while (iters < maxit) {
@@ -1471,50 +1565,60 @@ int gmres_t(nalu_linsys* ls, const double* b, double* x, int m, int maxit, doubl
     int k = 0;
     bool done = false;
     const bool learned_cycle = watch && learned_active(ls);
+    auto product = [&](int c) {  // V_{c+1} = A M^-1 V_c
+      TV* zc = flexible ? Z + (size_t)ldv * c : Z;
+      prec_m<TV>(ls, nrhs, V + (size_t)ldv * c, zc);
+      spmv_m<TV, TV>(ls, nrhs, zc, V + (size_t)ldv * (c + 1), (const TV*)nullptr, 0);
+    };
+    bool ahead = false;  // product(k) is already enqueued
     for (; k < m && iters < maxit; ++k) {
       ++iters;
-      TV* vk = V + (size_t)ldv * k;
       TV* vk1 = V + (size_t)ldv * (k + 1);
-      TV* zk = flexible ? Z + (size_t)ldv * k : Z;
-      prec_m<TV>(ls, nrhs, vk, zk);
-      spmv_m<TV, TV>(ls, nrhs, zk, vk1, (const TV*)nullptr, 0);
+      if (!ahead) product(k);
       const int cnt = k + 1;
       const size_t hbytes = sizeof(double) * (2 * (m + 2) + 1);
-      hipLaunchKernelGGL(k_gs_dots<TV>, dim3(nb_dots), dim3(kThreads), lds_dots, s, V, ldv, cnt, always2 ? 0 : 1, vk1,
-                         n, R_dots, ls->red.p);
+      hipLaunchKernelGGL(k_gs_dots<TV>, dots_grid(cnt + 1), dim3(kThreads), lds_dots, s, V, ldv, cnt, always2 ? 0 : 1,
+                         vk1, n, ls->red.p);
       hipLaunchKernelGGL(k_reduce_rows, dim3(always2 ? cnt : cnt + 1), dim3(kThreads), 0, s, ls->red.p, (int)nb_dots,
                          hA, 0);
       auto second_pass = [&]() {
-        hipLaunchKernelGGL(k_gs_dots<TV>, dim3(nb_dots), dim3(kThreads), lds_dots, s, V, ldv, cnt, 0, vk1, n, R_dots,
+        hipLaunchKernelGGL(k_gs_dots<TV>, dots_grid(cnt), dim3(kThreads), lds_dots, s, V, ldv, cnt, 0, vk1, n,
                            ls->red.p);
         hipLaunchKernelGGL(k_reduce_rows, dim3(cnt), dim3(kThreads), 0, s, ls->red.p, (int)nb_dots, hB, 0);
-        hipLaunchKernelGGL(k_gs_update_norm<TV>, dim3(nb_upd), dim3(kThreads), 0, s, V, ldv, cnt, hB, vk1, n,
-                           ls->red.p);
+        update(cnt, hB, vk1, true);
         hipLaunchKernelGGL(k_reduce_rows, dim3(1), dim3(kThreads), 0, s, ls->red.p, (int)nb_upd, nrm, 0);
       };
       if (always2) {
-        hipLaunchKernelGGL(k_gs_update<TV>, dim3(nb_upd), dim3(kThreads), 0, s, V, ldv, cnt, hA, vk1, n);
+        update(cnt, hA, vk1, false);
         second_pass();
       } else {
-        hipLaunchKernelGGL(k_gs_update_norm<TV>, dim3(nb_upd), dim3(kThreads), 0, s, V, ldv, cnt, hA, vk1, n,
-                           ls->red.p);
+        update(cnt, hA, vk1, true);
         hipLaunchKernelGGL(k_reduce_rows, dim3(1), dim3(kThreads), 0, s, ls->red.p, (int)nb_upd, nrm, 0);
       }
       NALU_HIP_CHECK(hipMemcpyAsync(hpin, hbuf, hbytes, hipMemcpyDeviceToHost, s));
-      NALU_HIP_CHECK(hipStreamSynchronize(s));
-      bool two = always2;
-      if (!always2) {
-        const double w2 = hpin[cnt], n2 = hpin[2 * (m + 2)];
-        if (!(n2 >= 0.01 * w2)) {  // severe cancellation (or NaN): reorthogonalize once
-          second_pass();
-          NALU_HIP_CHECK(hipMemcpyAsync(hpin, hbuf, hbytes, hipMemcpyDeviceToHost, s));
-          NALU_HIP_CHECK(hipStreamSynchronize(s));
-          two = true;
-        }
-      }
-      for (int i = 0; i <= k; ++i) hcol[i] = hpin[i] + (two ? hpin[(m + 2) + i] : 0.0);
+      NALU_HIP_CHECK(hipEventRecord(col_read.e, s));
+      auto normalize = [&]() {
+        hipLaunchKernelGGL(k_scale_invnorm<TV>, dim3(nblocks(n)), dim3(kThreads), 0, s, vk1, n, nrm);
+      };
+      normalize();
+      ahead = k + 1 < m && iters < maxit;
+      if (ahead) product(k + 1);
+      NALU_HIP_CHECK(hipEventSynchronize(col_read.e));
+      for (int i = 0; i <= k; ++i) hcol[i] = hpin[i] + (always2 ? hpin[(m + 2) + i] : 0.0);
       hcol[k + 1] = std::sqrt(hpin[2 * (m + 2)]);
-      hipLaunchKernelGGL(k_scale_invnorm<TV>, dim3(nblocks(n)), dim3(kThreads), 0, s, vk1, n, nrm);
+      // FP32: severe cancellation (or NaN) reorthogonalizes once, on the vector
+      // already scaled by its norm n1, so the new coefficients and norm count n1
+      // times (a zero vector needs none)
+      if (!always2 && hcol[k + 1] != 0.0 && !(hpin[2 * (m + 2)] >= 0.01 * hpin[cnt])) {
+        const double n1 = hcol[k + 1];
+        second_pass();
+        NALU_HIP_CHECK(hipMemcpyAsync(hpin, hbuf, hbytes, hipMemcpyDeviceToHost, s));
+        normalize();
+        NALU_HIP_CHECK(hipStreamSynchronize(s));
+        for (int i = 0; i <= k; ++i) hcol[i] += n1 * hpin[(m + 2) + i];
+        hcol[k + 1] = n1 * std::sqrt(hpin[2 * (m + 2)]);
+        ahead = false;
+      }
       if (learned_cycle && !std::isfinite(hcol[k + 1])) {
         learned_set_fallback(ls, true);  // drop this direction, finish the cycle with k columns
         break;
@@ -1565,12 +1669,15 @@ int cg_fused(nalu_linsys* ls, const double* b, double* x, int maxit, double tol)
   const int nc = ls->num_colors;
   const auto& ccp = ls->sell_color_ptr;
   const SellChunk* ch = reinterpret_cast<const SellChunk*>(ls->sell_chunks.p);
-  const unsigned g_spmv = (unsigned)std::max<int64_t>(1, (nch + 3) / 4);
+  const unsigned g_spmv = few_spmv(nch) ? sell_grid<4>(nch) : sell_grid<1>(nch);
   const unsigned g_upd = red_blocks(n);
   // partial-sum slots of the sweeps that finalize z: forward of the last color, every backward
   std::vector<int> off(nc + 1, 0);
   int total = 0;
-  auto sweep_grid = [&](int c) { return (unsigned)xcd_grid(std::max<int64_t>(1, (ccp[c + 1] - ccp[c] + 1) / 2)); };
+  auto sweep_grid = [&](int c) {
+    const int64_t k = ccp[c + 1] - ccp[c];
+    return (unsigned)xcd_grid(few_sweep(k) ? sell_grid<8>(k) : sell_grid<2>(k));
+  };
   const int cl = nc - 1;
   off[cl] = total;
   total += (int)sweep_grid(cl);
@@ -1612,20 +1719,28 @@ int cg_fused(nalu_linsys* ls, const double* b, double* x, int maxit, double tol)
   bool stop = false;
   while (!stop && it < maxit) {
     ++it;
-    hipLaunchKernelGGL(k_sell_spmv_dot<double>, dim3(g_spmv), dim3(kThreads), 0, s, ch, nch, lcs, lval, ucs, uval,
-                       split_of<double>(ls).dv, (const double*)p, q, part, (const CgState*)st);
+    auto spmv_dot = [&](auto kern, int threads) {
+      hipLaunchKernelGGL(kern, dim3(g_spmv), dim3(threads), 0, s, ch, nch, lcs, lval, ucs, uval,
+                         split_of<double>(ls).dv, (const double*)p, q, part, (const CgState*)st);
+    };
+    if (few_spmv(nch)) spmv_dot(k_sell_spmv_dot<double, 4>, SellBlock<4>::threads);
+    else spmv_dot(k_sell_spmv_dot<double, 1>, SellBlock<1>::threads);
     hipLaunchKernelGGL(k_cg_reduce, dim3(1), dim3(kReduceThreads), 0, s, (const double*)part, (int)g_spmv, 0, 0, it, st);
     hipLaunchKernelGGL(k_cg_update_f, dim3(g_upd), dim3(kThreads), 0, s, x, r, (const double*)p,
                        (const double*)q, n, cur, part, (const CgState*)st);
     hipLaunchKernelGGL(k_cg_reduce, dim3(1), dim3(kReduceThreads), 0, s, (const double*)part, (int)g_upd, 1, 0, it, st);
     const int nxt = 1 - cur;
-    for (int c = 0; c < nc; ++c)
-      hipLaunchKernelGGL((k_sell_sweep_dot<double, false>), dim3(sweep_grid(c)), dim3(kThreads), 0, s, ch, ccp[c],
-                         ccp[c + 1], lcs, lval, invd, (const double*)r, z, c == cl ? 1 : 0, part, off[c],
-                         (const CgState*)st);
-    for (int c = nc - 2; c >= 0; --c)
-      hipLaunchKernelGGL((k_sell_sweep_dot<double, true>), dim3(sweep_grid(c)), dim3(kThreads), 0, s, ch, ccp[c],
-                         ccp[c + 1], ucs, uval, invd, (const double*)r, z, 1, part, off[c], (const CgState*)st);
+    auto sweep = [&](int c, auto upper, int dot) {
+      constexpr bool UP = decltype(upper)::value;
+      auto go = [&](auto kern, int threads) {
+        hipLaunchKernelGGL(kern, dim3(sweep_grid(c)), dim3(threads), 0, s, ch, ccp[c], ccp[c + 1], UP ? ucs : lcs,
+                           UP ? uval : lval, invd, (const double*)r, z, dot, part, off[c], (const CgState*)st);
+      };
+      if (few_sweep(ccp[c + 1] - ccp[c])) go(k_sell_sweep_dot<double, UP, 8>, SellBlock<8>::threads);
+      else go(k_sell_sweep_dot<double, UP, 2>, SellBlock<2>::threads);
+    };
+    for (int c = 0; c < nc; ++c) sweep(c, std::false_type{}, c == cl ? 1 : 0);
+    for (int c = nc - 2; c >= 0; --c) sweep(c, std::true_type{}, 1);
     hipLaunchKernelGGL(k_cg_reduce, dim3(1), dim3(kReduceThreads), 0, s, (const double*)part, total, 2, nxt, it, st);
     hipLaunchKernelGGL(k_cg_p_f, dim3(nblocks(n)), dim3(kThreads), 0, s, p, (const double*)z, n, nxt, cur,
                        (const CgState*)st);
