@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <cstring>
+#include <map>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -49,27 +50,116 @@ int guarded(F&& f) {
 }
 
 // -------------------------------------------------------- device buffers
+// Device memory that a handle keeps between calls: buffers allocated in a
+// PoolScope return to the handle's pool instead of to the runtime (every hipFree
+// synchronizes the device; an AMG set-up at 96^3 makes about a hundred).  All work of
+// a handle runs in order on its stream, so a returned block can be taken again at
+// once; a scope on another stream than the last one waits for the device first.
+// One handle is used by one thread at a time, and so is its pool.  Idle memory is
+// bounded and goes back with the handle; blocks past the bound, and all idle ones
+// when an allocation fails, are freed.
+class DevPool {
+ public:
+  DevPool() = default;
+  DevPool(const DevPool&) = delete;
+  DevPool& operator=(const DevPool&) = delete;
+  ~DevPool() { trim(); }
+  void on_stream(hipStream_t s) {
+    if (used_ && s != stream_) NALU_HIP_CHECK(hipDeviceSynchronize());
+    used_ = true;
+    stream_ = s;
+  }
+  void* get(size_t bytes, size_t* cap) {
+    // sizes recur from one set-up to the next but for a few per cent: round up to an
+    // eighth of the power of two below
+    size_t step = 512;
+    while (step * 16 <= bytes) step <<= 1;
+    bytes = (bytes + step - 1) / step * step;
+    const auto it = idle_.lower_bound(bytes);
+    if (it != idle_.end() && it->first <= bytes + bytes / 4) {
+      void* q = it->second;
+      *cap = it->first;
+      idle_bytes_ -= it->first;
+      idle_.erase(it);
+      return q;
+    }
+    void* q = nullptr;
+    if (hipMalloc(&q, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      trim();
+      NALU_HIP_CHECK(hipMalloc(&q, bytes));
+    }
+    *cap = bytes;
+    return q;
+  }
+  void put(void* q, size_t cap) {
+    if (idle_bytes_ + cap > kMaxIdle) {
+      (void)hipFree(q);
+      return;
+    }
+    idle_.emplace(cap, q);
+    idle_bytes_ += cap;
+  }
+  static DevPool*& current() {
+    static thread_local DevPool* p = nullptr;
+    return p;
+  }
+
+ private:
+  static constexpr size_t kMaxIdle = (size_t)4 << 30;
+  void trim() {
+    for (auto& b : idle_) (void)hipFree(b.second);
+    idle_.clear();
+    idle_bytes_ = 0;
+  }
+  std::multimap<size_t, void*> idle_;
+  size_t idle_bytes_ = 0;
+  hipStream_t stream_ = nullptr;
+  bool used_ = false;
+};
+// Buffers allocated while it lives come from the pool.  Only for buffers that die
+// with the pool's handle or before it.
+struct PoolScope {
+  DevPool* prev;
+  PoolScope(DevPool& p, hipStream_t s) : prev(DevPool::current()) {
+    p.on_stream(s);
+    DevPool::current() = &p;
+  }
+  PoolScope(const PoolScope&) = delete;
+  PoolScope& operator=(const PoolScope&) = delete;
+  ~PoolScope() { DevPool::current() = prev; }
+};
+
 template <class T>
 struct DevBuf {
   T* p = nullptr;
   size_t n = 0;
+  DevPool* pool = nullptr;  // where p goes back to (null: the runtime)
+  size_t cap = 0;           // its size there
   DevBuf() = default;
   explicit DevBuf(size_t count) { alloc(count); }
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
-  DevBuf(DevBuf&& o) noexcept : p(o.p), n(o.n) { o.p = nullptr; o.n = 0; }
+  DevBuf(DevBuf&& o) noexcept : p(o.p), n(o.n), pool(o.pool), cap(o.cap) { o.p = nullptr; o.n = 0; }
   DevBuf& operator=(DevBuf&& o) noexcept {
-    if (this != &o) { release(); p = o.p; n = o.n; o.p = nullptr; o.n = 0; }
+    if (this != &o) {
+      release();
+      p = o.p; n = o.n; pool = o.pool; cap = o.cap;
+      o.p = nullptr; o.n = 0;
+    }
     return *this;
   }
   ~DevBuf() { release(); }
   void alloc(size_t count) {
     release();
-    if (count) NALU_HIP_CHECK(hipMalloc((void**)&p, count * sizeof(T)));
+    pool = DevPool::current();
+    if (count && pool) p = static_cast<T*>(pool->get(count * sizeof(T), &cap));
+    else if (count) NALU_HIP_CHECK(hipMalloc((void**)&p, count * sizeof(T)));
     n = count;
   }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p && pool) pool->put(p, cap);
+    else if (p) (void)hipFree(p);
     p = nullptr;
     n = 0;
   }
@@ -146,6 +236,7 @@ struct nalu_mesh {
 
 // ---------------------------------------------------------- linear system
 struct nalu_linsys {
+  nalu::DevPool pool;  // first member: outlives every buffer of the handle
   int num_dof = 1;
   nalu_solver_config cfg{};
   hipStream_t stream = nullptr;

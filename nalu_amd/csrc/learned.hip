@@ -1743,7 +1743,10 @@ extern "C" int nalu_gnn_loss_grad(nalu_gnn* g, nalu_linsys* ls, int batch, const
     const int64_t n = ls->nrows, T = n * batch;
     hipStream_t s = ls->stream;
     nalu::Work w;
-    w.alloc(n, batch, g->L);
+    {
+      nalu::PoolScope scope(ls->pool, s);
+      w.alloc(n, batch, g->L);
+    }
     hipLaunchKernelGGL((nalu::k_gather_perm<float, float>), dim3(nalu::nblocks(T)), dim3(nalu::kThreads), 0, s, r_dev,
                        ls->perm.p, n, batch, w.R.p);
     hipLaunchKernelGGL((nalu::k_gather_perm<float, float>), dim3(nalu::nblocks(T)), dim3(nalu::kThreads), 0, s, e_dev,

@@ -1,0 +1,105 @@
+"""The memory a handle keeps between calls (AMG set-ups, batches of the learned
+preconditioner, Dirichlet flags): repeated use gives what a new handle gives, also
+on another stream and from several threads with a handle each, and destroying the
+handle gives the memory back.
+
+Bar: solutions of two solves to 1e-12 on the same matrix within 1e-8 of each other
+(condition number below 1e4)."""
+import gc
+import threading
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import nalu_amd as na  # noqa: E402
+from nalu_amd.problems import lowmach_problem  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def dev(a):
+    return torch.as_tensor(np.ascontiguousarray(a), dtype=torch.float64, device=DEV)
+
+
+class Problem:
+    def __init__(self, n, seed):
+        P = lowmach_problem(n, seed=seed, rho_sigma=0.3)
+        self.mesh = na.Mesh(P["coords"], P["conn"])
+        self.f = [dev(P[k]) for k in ("rho", "p", "u", "gpdx")]
+
+    def handle(self, stream=None):
+        ls = na.LinearSystem(1, na.SolverConfig("cg", "muelu", tolerance=1e-12, max_iterations=400))
+        ls.set_muelu_params(na.MueLuParams(max_coarse_size=60))
+        ls.buildElemToNodeGraph(self.mesh)
+        ls.finalizeLinearSystem()
+        if stream is not None:
+            ls.set_stream(stream.cuda_stream)
+        return ls
+
+    def solve(self, ls, scale=1.0):
+        f = [self.f[0]] + [a * scale for a in self.f[1:]]
+        x = torch.zeros(self.f[1].shape[0], dtype=torch.float64, device=DEV)
+        torch.cuda.synchronize()  # x and the scaled fields come from torch's stream
+        ls.zeroSystem()
+        na.assemble_continuity(ls, self.mesh, *f)
+        ls.loadComplete()
+        ls.removeRhsMean()
+        assert ls.solve(x) == 0  # returns after the handle's stream is done
+        return x - x.mean()
+
+
+def close(a, b):
+    return float((a - b).norm() / b.norm()) <= 1e-8
+
+
+def test_repeated_setups_and_streams():
+    P = Problem(13, 3)
+    ref = P.solve(P.handle())
+    ls = P.handle()
+    for k in range(4):
+        print("case: repeated AMG set-up", k, flush=True)
+        if k == 2:
+            st = torch.cuda.Stream()
+            ls.set_stream(st.cuda_stream)
+        x = P.solve(ls, 1.0 + k)
+        assert close(x / (1.0 + k), ref)
+
+
+def test_threads_with_a_handle_each():
+    probs = [Problem(10 + k, 5 + k) for k in range(3)]
+    refs = [P.solve(P.handle()) for P in probs]
+    bad = []
+
+    def work(P, ref):
+        st = torch.cuda.Stream()
+        ls = P.handle(st)
+        for _ in range(3):
+            if not close(P.solve(ls), ref):
+                bad.append(P)
+
+    print("case: three threads", flush=True)
+    ts = [threading.Thread(target=work, args=a) for a in zip(probs, refs)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert not bad
+
+
+def test_destroying_the_handle_gives_the_memory_back():
+    P = Problem(32, 9)
+    P.solve(P.handle())
+    gc.collect()
+    torch.cuda.synchronize()
+    free0 = torch.cuda.mem_get_info()[0]
+    ls = P.handle()
+    P.solve(ls)
+    held = free0 - torch.cuda.mem_get_info()[0]
+    del ls
+    gc.collect()
+    torch.cuda.synchronize()
+    left = free0 - torch.cuda.mem_get_info()[0]
+    print("case: held %.1f MB, left %.1f MB" % (held / 1e6, left / 1e6), flush=True)
+    assert left <= 8 << 20
