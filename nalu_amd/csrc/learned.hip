@@ -672,20 +672,34 @@ __global__ __launch_bounds__(kThreads) void k_aop(const int32_t* __restrict__ gp
   __shared__ double sh[2][kThreads / 64];
   const int64_t off = (int64_t)blockIdx.y * n;
   const float* xb = x + off;
+  // eight lanes to a row: its entries are read coalesced, and the chain of gathers
+  // is an eighth (48^3, batch 4: 478 us with a lane per row, below 70 us so)
+  const int q = threadIdx.x & 7;
   double sp = 0.0, sq = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+  for (int64_t i0 = (int64_t)blockIdx.x * (kThreads / 8); i0 < n; i0 += (int64_t)gridDim.x * (kThreads / 8)) {
+    const int64_t i = i0 + (threadIdx.x >> 3);
     float wx = 0.f, wtdx = 0.f;
-    for (int p = gptr[i]; p < gptr[i + 1]; ++p) {
-      const int j = gcol[p];
-      const float xj = xb[j];
-      wx = fmaf(gw[p], xj, wx);
-      wtdx = fmaf(gwt[p], dF[j] * xj, wtdx);
+    if (i < n) {
+      const int p1 = gptr[i + 1];
+      for (int p = gptr[i] + q; p < p1; p += 8) {
+        const int j = gcol[p];
+        const float xj = xb[j];
+        wx = fmaf(gw[p], xj, wx);
+        wtdx = fmaf(gwt[p], dF[j] * xj, wtdx);
+      }
     }
-    const float d = dF[i], xi = xb[i];
-    const float ax = d * (xi - wx);
-    sym[off + i] = 2.f * d * xi - d * wx - wtdx;
-    sp += (double)xi * (double)r[off + i];
-    sq += (double)xi * (double)ax;
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) {
+      wx += __shfl_xor(wx, o, 8);
+      wtdx += __shfl_xor(wtdx, o, 8);
+    }
+    if (i < n && q == 0) {
+      const float d = dF[i], xi = xb[i];
+      const float ax = d * (xi - wx);
+      sym[off + i] = 2.f * d * xi - d * wx - wtdx;
+      sp += (double)xi * (double)r[off + i];
+      sq += (double)xi * (double)ax;
+    }
   }
   sp = wave_sum(sp);
   sq = wave_sum(sq);
@@ -791,6 +805,9 @@ __global__ __launch_bounds__(kThreads) void k_output_bwd(const float* __restrict
 //   dW_l += delta^T [h ; m],  db_l += sum delta   (per-wavefront partials)
 // Blocks stride over tile groups so every wavefront of a block runs the same
 // number of iterations (the LDS tiles are per wavefront, the barriers per block).
+// Bound by its 240 B per node and feature row of streams: 16-byte loads and four
+// blocks to a CU, their waves' dW summed in LDS first (48^3, batch 4: 74 us; 171 us
+// with 4-byte loads and one block to a CU).
 __global__ __launch_bounds__(kThreads) void k_layer_bwd(int64_t total, const float* __restrict__ G,
                                                         const uint32_t* __restrict__ mask,
                                                         const uint16_t* __restrict__ h, const uint16_t* __restrict__ mst,
@@ -808,25 +825,45 @@ __global__ __launch_bounds__(kThreads) void k_layer_bwd(int64_t total, const flo
 #pragma unroll
       for (int t = 0; t < 8; ++t) wb[ks][nt][t] = wl[(ks * 16 + 8 * half + t) * 2 * kH + nt * kH + f];
   f32x16 dw0 = {}, dw1 = {};
-  float db = 0.f;
+  float db[4] = {0.f, 0.f, 0.f, 0.f};  // features 4 (lane & 7) ..
   const int64_t ntiles = (total + kTile - 1) / kTile;
   for (int64_t grp = blockIdx.x; grp * kWaves < ntiles; grp += gridDim.x) {
     const int64_t tile0 = (grp * kWaves + wv) * kTile;
-    for (int p = 0; p < kTile / 2; ++p) {
-      const int nl = 2 * p + half;
-      const int64_t node = tile0 + nl;
-      float dl = 0.f;
-      uint16_t hh = 0, mm = 0;
+    // 16-byte loads: four features of G, eight of h and m to a lane
+    float4 gv[kTile / 8];
+    uint32_t mk[kTile / 8];
+#pragma unroll
+    for (int p = 0; p < kTile / 8; ++p) {
+      const int64_t node = tile0 + 8 * p + (lane >> 3);
+      gv[p] = make_float4(0.f, 0.f, 0.f, 0.f);
+      mk[p] = 0u;
       if (node < total) {
-        const float gv = G[node * kH + f];
-        dl = ((mask[node] >> f) & 1u) ? gv : 0.f;
-        hh = h[node * kH + f];
-        mm = mst[node * kH + f];
+        gv[p] = *reinterpret_cast<const float4*>(G + node * kH + 4 * (lane & 7));
+        mk[p] = mask[node] >> (4 * (lane & 7));
       }
-      db += dl;
-      Ds[wv][nl][f] = f2bf(dl);
-      As[wv][nl][f] = hh;
-      As[wv][nl][kH + f] = mm;
+    }
+#pragma unroll
+    for (int p = 0; p < kTile / 16; ++p) {
+      const int nl = 16 * p + (lane >> 2), c = 8 * (lane & 3);
+      const int64_t node = tile0 + nl;
+      u16x8 hh = {}, mm = {};
+      if (node < total) {
+        hh = *reinterpret_cast<const u16x8*>(h + node * kH + c);
+        mm = *reinterpret_cast<const u16x8*>(mst + node * kH + c);
+      }
+      *reinterpret_cast<u16x8*>(&As[wv][nl][c]) = hh;
+      *reinterpret_cast<u16x8*>(&As[wv][nl][kH + c]) = mm;
+    }
+#pragma unroll
+    for (int p = 0; p < kTile / 8; ++p) {
+      const int nl = 8 * p + (lane >> 3), c = 4 * (lane & 7);
+      const float dl[4] = {(mk[p] & 1u) ? gv[p].x : 0.f, (mk[p] & 2u) ? gv[p].y : 0.f, (mk[p] & 4u) ? gv[p].z : 0.f,
+                           (mk[p] & 8u) ? gv[p].w : 0.f};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        db[k] += dl[k];
+        Ds[wv][nl][c + k] = f2bf(dl[k]);
+      }
     }
     __syncthreads();
     f32x16 ch = {}, cm = {};
@@ -859,15 +896,32 @@ __global__ __launch_bounds__(kThreads) void k_layer_bwd(int64_t total, const flo
     }
     __syncthreads();
   }
-  float* pw = part + ((int64_t)blockIdx.x * kWaves + wv) * kLayerParams;
+  // the four waves' sums meet in LDS, in wave order
+  float* sum = reinterpret_cast<float*>(&As[0][0][0]);
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int o = acc_row(r, half);
-    pw[o * 2 * kH + f] = dw0[r];
-    pw[o * 2 * kH + kH + f] = dw1[r];
+  for (int o = 8; o < 64; o <<= 1)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) db[k] += __shfl_xor(db[k], o);
+  for (int w = 0; w < kWaves; ++w) {
+    if (wv == w) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int o = acc_row(r, half);
+        sum[o * 2 * kH + f] = dw0[r] + (w ? sum[o * 2 * kH + f] : 0.f);
+        sum[o * 2 * kH + kH + f] = dw1[r] + (w ? sum[o * 2 * kH + kH + f] : 0.f);
+      }
+      if (lane < 8) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          float* q = sum + 2 * kH * kH + 4 * lane + k;
+          *q = db[k] + (w ? *q : 0.f);
+        }
+      }
+    }
+    __syncthreads();
   }
-  db += __shfl_xor(db, 32);
-  if (half == 0) pw[2 * kH * kH + f] = db;
+  float* pw = part + (int64_t)blockIdx.x * kLayerParams;
+  for (int k = threadIdx.x; k < kLayerParams; k += kThreads) pw[k] = sum[k];
 }
 
 // G_j = Gp_j + sum_{i in N(j)} w_ij DM_i  (transposed aggregation; FP32);
@@ -1427,6 +1481,12 @@ void apply_perm(nalu_linsys* ls, Learned* st, const nalu_gnn* g, const float* r,
 }
 
 // ---------------------------------------------------------------- batch work
+// Grids of the reducing backward kernels: partial parameter gradients per block.
+// The streaming ones need eight blocks to a CU to keep loads in flight (48^3, batch
+// 4, output / encoder: 125 / 100 us with one block to a CU).
+constexpr int kBwdBlocks = 1024;
+constexpr int kStreamBlocks = 2048;
+
 struct Work {
   int64_t n = 0;
   int B = 0, L = 0;
@@ -1465,12 +1525,11 @@ struct Work {
     pq.alloc(2 * B);
     dpart.alloc((size_t)kRedBlocks * B * 2);
     loss.alloc(1);
-    fpart.alloc((size_t)256 * kWaves * kLayerParams);
+    fpart.alloc((size_t)kBwdBlocks * kLayerParams);
     ftmp.alloc((size_t)64 * kLayerParams);
   }
 };
 
-constexpr int kBwdBlocks = 256;  // grid of the reducing backward kernels
 constexpr int kColChunk = 64;
 
 // g[0..cols) = column sums of part[rows][cols]
@@ -1514,7 +1573,7 @@ void fwd_bwd(nalu_linsys* ls, Learned* st, nalu_gnn* g, Work& w, double* loss_sl
   hipLaunchKernelGGL(k_loss, dim3(1), dim3(64), 0, s, w.pq.p, w.S.p, B, loss_slot, 0);
   hipLaunchKernelGGL(k_gout, dim3(nblocks(T)), dim3(kThreads), 0, s, w.R.p, w.sym.p, w.pq.p, w.S.p, n, B, w.gout.p);
   // backward
-  const unsigned nbo = std::min<unsigned>(kBwdBlocks, nblocks(T * kH));
+  const unsigned nbo = std::min<unsigned>(kStreamBlocks, nblocks(T * kH));
   hipLaunchKernelGGL(k_output_bwd, dim3(nbo), dim3(kThreads), 0, s, w.gout.p, w.h[g->L].p, w.F.p,
                      g->wbf.p + lay.w_out(), T, w.G.p, w.fpart.p);
   col_sum(s, w.fpart.p, (int)nbo, 34, g->grad.p + lay.w_out(), w);
@@ -1523,11 +1582,11 @@ void fwd_bwd(nalu_linsys* ls, Learned* st, nalu_gnn* g, Work& w, double* loss_sl
   for (int l = g->L - 1; l >= 0; --l) {
     hipLaunchKernelGGL(k_layer_bwd, dim3(nbl), dim3(kThreads), 0, s, T, w.G.p, w.mask[l].p, w.h[l].p, w.mst[l].p,
                        g->wbf.p + lay.w(l), w.Gp.p, w.DM.p, w.fpart.p);
-    col_sum(s, w.fpart.p, (int)nbl * kWaves, kLayerParams, g->grad.p + lay.w(l), w);
+    col_sum(s, w.fpart.p, (int)nbl, kLayerParams, g->grad.p + lay.w(l), w);
     hipLaunchKernelGGL(k_agg_t, dim3(nblocks(T * 8)), dim3(kThreads), 0, s, st->gptr.p, st->gcol.p, st->gwt.p, n, T,
                        w.Gp.p, w.DM.p, w.G.p);
   }
-  const unsigned nbe = std::min<unsigned>(kBwdBlocks, nblocks(T * kH));
+  const unsigned nbe = std::min<unsigned>(kStreamBlocks, nblocks(T * kH));
   hipLaunchKernelGGL(k_encode_bwd, dim3(nbe), dim3(kThreads), 0, s, w.G.p, w.F.p, st->delta.p, n, T, w.fpart.p);
   col_sum(s, w.fpart.p, (int)nbe, 128, g->grad.p, w);
 }
