@@ -21,7 +21,7 @@
 //        A_f is A with the weak entries lumped into the diagonal (rows with no
 //        strong entry keep their tentative row);
 //     6. R = P^T (device radix sort), A_c = R (A P) with a hash SpGEMM
-//        (one wave per row, hash table in LDS);
+//        (32 lanes per row, hash table in LDS);
 //   until the operator has at most max_coarse rows, whose dense inverse is
 //   formed by Gauss-Jordan elimination with partial pivoting; pivots below
 //   1e-10 of the scale max(max|a_ii|, max|a_ii of the level above| x
@@ -352,38 +352,68 @@ __device__ __forceinline__ uint64_t mis_key(int st, uint32_t i) {
   return (cls << 62) | ((uint64_t)prio_hash(i) << 31) | (uint64_t)i;
 }
 
-__global__ void k_mis_keys(const int8_t* __restrict__ state, int64_t n, uint64_t* __restrict__ key) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) key[i] = mis_key(state[i], (uint32_t)i);
-}
-
-__global__ void k_mis_max(const int32_t* __restrict__ rp, const int32_t* __restrict__ ci,
-                          const uint8_t* __restrict__ strong, const uint64_t* __restrict__ in, int64_t n,
-                          uint64_t* __restrict__ out) {
+// One round of the synchronous MIS-2, two passes of kL lanes per row.  Near: m1[i] =
+// largest key of i and its strong neighbours.  Once none of those is undecided the
+// value is final (live[i] = 0) and later rounds skip the row; after a few rounds that
+// is nearly all of them (96^3 set-up: 29 and 22 us a pass here and below on average,
+// 85 us on the finest level for every row).
+__global__ void k_mis_near(const int32_t* __restrict__ rp, const int32_t* __restrict__ ci,
+                           const uint8_t* __restrict__ strong, const int8_t* __restrict__ state, int64_t n,
+                           int8_t* __restrict__ live, uint64_t* __restrict__ m1) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t i = t / kL;
   const int lane = (int)(t % kL);
+  const bool mine = i < n && live[i] != 0;
   uint64_t m = 0;
-  if (i < n) {
-    if (lane == 0) m = in[i];
+  int open = 0;
+  if (mine) {
+    if (lane == 0) {
+      const int st = state[i];
+      m = mis_key(st, (uint32_t)i);
+      open = st == 0;
+    }
     for (int32_t q = rp[i] + lane; q < rp[i + 1]; q += kL)
-      if (strong[q]) m = max(m, in[ci[q]]);
+      if (strong[q]) {
+        const int32_t j = ci[q];
+        const int st = state[j];
+        m = max(m, mis_key(st, (uint32_t)j));
+        open |= st == 0;
+      }
+  }
+#pragma unroll
+  for (int o = kL / 2; o > 0; o >>= 1) {
+    m = max(m, (uint64_t)__shfl_xor((unsigned long long)m, o, kL));
+    open |= __shfl_xor(open, o, kL);
+  }
+  if (mine && lane == 0) {
+    m1[i] = m;
+    live[i] = (int8_t)open;
+  }
+}
+
+// Far: an undecided row becomes a root when it holds the largest key of its
+// 2-neighbourhood (the largest m1 of itself and its neighbours), covered when a root
+// lies within two steps; *undecided is set to 1 (one store per wave) while rows
+// remain undecided.
+__global__ void k_mis_far(const int32_t* __restrict__ rp, const int32_t* __restrict__ ci,
+                          const uint8_t* __restrict__ strong, const uint64_t* __restrict__ m1, int64_t n,
+                          int8_t* __restrict__ state, int* __restrict__ undecided) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t i = t / kL;
+  const int lane = (int)(t % kL);
+  const bool mine = i < n && state[i] == 0;
+  uint64_t m = 0;
+  if (mine) {
+    if (lane == 0) m = m1[i];
+    for (int32_t q = rp[i] + lane; q < rp[i + 1]; q += kL)
+      if (strong[q]) m = max(m, m1[ci[q]]);
   }
 #pragma unroll
   for (int o = kL / 2; o > 0; o >>= 1) m = max(m, (uint64_t)__shfl_xor((unsigned long long)m, o, kL));
-  if (i < n && lane == 0) out[i] = m;
-}
-
-// undecided row: root when it holds the largest key of its 2-neighbourhood,
-// covered when a root lies within two steps; *undecided is set to 1 (one
-// store per wave) while rows remain undecided
-__global__ void k_mis_update(const uint64_t* __restrict__ key, const uint64_t* __restrict__ m2, int64_t n,
-                             int8_t* __restrict__ state, int* __restrict__ undecided) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   bool left = false;
-  if (i < n && state[i] == 0) {
-    if (m2[i] == key[i]) state[i] = 1;
-    else if ((m2[i] >> 62) == 3u) state[i] = 2;
+  if (mine && lane == 0) {
+    if (m == mis_key(0, (uint32_t)i)) state[i] = 1;
+    else if ((m >> 62) == 3u) state[i] = 2;
     else left = true;
   }
   if (__ballot(left) != 0 && (threadIdx.x % 64) == 0) *undecided = 1;
@@ -503,68 +533,80 @@ __global__ void k_tentative(const int32_t* __restrict__ agg, const double* __res
 }
 
 // ------------------------------------------------------------------ SpGEMM
-// C = A B, one 64-lane block per row (grid-stride), open-addressing hash of H
-// (power of two) slots in LDS.  Phase 0 counts each row's distinct columns;
-// phase 1 writes them (unsorted) at C.rp[i].  Zero entries of A or B add
-// nothing.  A row with more than H distinct columns sets *overflow.
-__device__ __forceinline__ uint32_t slot_hash(int32_t c) { return (uint32_t)c * 0x9e3779b1u; }
+// C = A B, 32 lanes per row (grid-stride), each row's open-addressing hash of H (power
+// of two) slots in LDS.  Phase 0 counts each row's distinct columns; phase 1 writes
+// them (unsorted) at C.rp[i].  Zero entries of A or B add nothing.  A row with more
+// than H distinct columns sets *overflow.  The lanes take the entries of A's row, as
+// B's rows are short in both products of a level (about 10 entries).  Bound by LDS:
+// clearing and scanning the table costs as much as the inserts, so the fill phase
+// takes the smallest table that is at least half empty and the count phase starts
+// with 256 slots of keys only.  The 96^3 pressure solve with its set-up went from
+// 23.4 to 20.8 ms with this and the MIS passes above, against one wave and 1024 slots
+// to a row and MIS passes over every row.
+constexpr int kGemmLanes = 32;
+__device__ __forceinline__ uint32_t slot_hash(int32_t c, int shift) { return ((uint32_t)c * 0x9e3779b1u) >> shift; }
 
 template <int PHASE>
-__global__ __launch_bounds__(64) void k_spgemm(const int32_t* __restrict__ arp, const int32_t* __restrict__ aci,
+__global__ __launch_bounds__(kT) void k_spgemm(const int32_t* __restrict__ arp, const int32_t* __restrict__ aci,
                                                const double* __restrict__ av, const int32_t* __restrict__ brp,
                                                const int32_t* __restrict__ bci, const double* __restrict__ bv,
-                                               int64_t n, int H, const int32_t* __restrict__ crp,
+                                               int64_t n, int H, int shift, const int32_t* __restrict__ crp,
                                                int32_t* __restrict__ cnt, int32_t* __restrict__ cci,
                                                double* __restrict__ cv, int* __restrict__ overflow) {
-  extern __shared__ unsigned char smem[];
-  double* hv = reinterpret_cast<double*>(smem);
-  int32_t* hk = reinterpret_cast<int32_t*>(hv + H);
-  const int lane = threadIdx.x;
+  extern __shared__ double smem[];
+  const int rows = blockDim.x / kGemmLanes, group = threadIdx.x / kGemmLanes, lane = threadIdx.x % kGemmLanes;
+  double* hv = smem + (size_t)group * H;
+  int32_t* hk = reinterpret_cast<int32_t*>(smem + (PHASE == 1 ? (size_t)rows * H : 0)) + (size_t)group * H;
   const uint32_t mask = (uint32_t)H - 1;
-  for (int64_t i = blockIdx.x; i < n; i += gridDim.x) {
-    for (int s = lane; s < H; s += 64) {
+  auto sync = [] {  // a group is half a wave: order its LDS accesses, no block barrier
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  auto insert = [&](int32_t c, double ab) {
+    uint32_t h = slot_hash(c, shift) & mask;
+    for (int probe = 0; probe < H; ++probe) {
+      const int32_t old = atomicCAS(&hk[h], -1, c);
+      if (old == -1 || old == c) {
+        if (PHASE == 1) atomicAdd(&hv[h], ab);
+        return;
+      }
+      h = (h + 1) & mask;
+    }
+    atomicOr(overflow, 1);
+  };
+  for (int64_t i0 = (int64_t)blockIdx.x * rows; i0 < n; i0 += (int64_t)gridDim.x * rows) {
+    const int64_t i = i0 + group;
+    for (int s = lane; s < H; s += kGemmLanes) {
       hk[s] = -1;
-      hv[s] = 0.0;
+      if (PHASE == 1) hv[s] = 0.0;
     }
-    __syncthreads();
-    for (int32_t q = arp[i] + lane; q < arp[i + 1]; q += 64) {
-      const double a = av[q];
-      if (a == 0.0) continue;
-      const int32_t k = aci[q];
-      for (int32_t t = brp[k]; t < brp[k + 1]; ++t) {
-        const double b = bv[t];
-        if (b == 0.0) continue;
-        const int32_t c = bci[t];
-        uint32_t h = slot_hash(c) & mask;
-        int probe = 0;
-        for (; probe < H; ++probe) {
-          const int32_t old = atomicCAS(&hk[h], -1, c);
-          if (old == -1 || old == c) break;
-          h = (h + 1) & mask;
+    sync();
+    if (i < n) {
+      for (int32_t q = arp[i] + lane; q < arp[i + 1]; q += kGemmLanes) {
+        const double a = av[q];
+        if (a == 0.0) continue;
+        const int32_t k = aci[q];
+        for (int32_t t = brp[k]; t < brp[k + 1]; ++t) {
+          const double b = bv[t];
+          if (b != 0.0) insert(bci[t], a * b);
         }
-        if (probe == H) {
-          atomicOr(overflow, 1);
-          continue;
-        }
-        if (PHASE == 1) atomicAdd(&hv[h], a * b);
       }
     }
-    __syncthreads();
+    sync();
     int base = 0;
-    for (int s0 = 0; s0 < H; s0 += 64) {
-      const int s = s0 + lane;
-      const bool occ = s < H && hk[s] != -1;
-      const uint64_t bal = __ballot(occ);
-      if (PHASE == 1 && occ) {
-        const int off = __popcll(bal & ((1ull << lane) - 1ull));
-        const int64_t o = (int64_t)crp[i] + base + off;
-        cci[o] = hk[s];
-        cv[o] = hv[s];
+    for (int s0 = 0; s0 < H; s0 += kGemmLanes) {
+      const int32_t c = hk[s0 + lane];
+      const uint32_t bal = (uint32_t)(__ballot(c != -1) >> ((threadIdx.x & 32) ? 32 : 0));
+      if (PHASE == 1 && c != -1 && i < n) {
+        const int64_t o = (int64_t)crp[i] + base + __popc(bal & ((1u << lane) - 1u));
+        cci[o] = c;
+        cv[o] = hv[s0 + lane];
       }
-      base += __popcll(bal);
+      base += __popc(bal);
     }
-    if (PHASE == 0 && lane == 0) cnt[i] = base;
-    __syncthreads();
+    if (PHASE == 0 && lane == 0 && i < n) cnt[i] = base;
+    sync();
   }
 }
 
@@ -583,19 +625,6 @@ __global__ void k_count_total(const int32_t* __restrict__ cnt, int64_t n, unsign
   if (threadIdx.x == 0) atomicAdd(total, sh[0]);
 }
 
-__global__ void k_row_bound(const int32_t* __restrict__ arp, const int32_t* __restrict__ aci,
-                            const int32_t* __restrict__ brp, int64_t n, int32_t* __restrict__ out) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t i = t / kL;
-  const int lane = (int)(t % kL);
-  int64_t sum = 0;
-  if (i < n)
-    for (int32_t q = arp[i] + lane; q < arp[i + 1]; q += kL) sum += brp[aci[q] + 1] - brp[aci[q]];
-#pragma unroll
-  for (int o = kL / 2; o > 0; o >>= 1) sum += __shfl_xor((long long)sum, o, kL);
-  if (i < n && lane == 0) out[i] = (int32_t)std::min<int64_t>(sum, 1 << 30);
-}
-
 int32_t dev_max(const int32_t* a, int64_t n, hipStream_t s) {
   NALU_REQUIRE(n > 0 && n < (int64_t)INT32_MAX, NALU_ERR_UNSUPPORTED, "amg: reduction size out of range");
   DevBuf<int32_t> mx(1);
@@ -606,7 +635,7 @@ int32_t dev_max(const int32_t* a, int64_t n, hipStream_t s) {
   return to_host(mx.p, s);
 }
 
-constexpr int kFirstHash = 1024;
+constexpr int kFirstHash = 256;  // slots of the first count
 constexpr int kMaxHash = 4096;
 
 Csr spgemm(const Csr& A, const double* av, const Csr& B, hipStream_t s) {
@@ -619,28 +648,30 @@ Csr spgemm(const Csr& A, const double* av, const Csr& B, hipStream_t s) {
     return C;
   }
   DevBuf<int32_t> cnt(A.n + 1);
-  hipLaunchKernelGGL(k_row_bound, dim3(nbl(A.n * kL)), dim3(kT), 0, s, A.rp.p, A.ci.p, B.rp.p, A.n, cnt.p);
-  const int64_t bound = std::min<int64_t>(dev_max(cnt.p, A.n, s), B.m);
-  // the bound (sum of the B rows met) overestimates the distinct columns of a
-  // product row several-fold: start with at most kFirstHash slots and grow to
-  // kMaxHash only when a row overflows
-  int H = 64;
-  while (H < 2 * bound && H < kFirstHash) H <<= 1;
   DevBuf<int> ovf(1);
-  const unsigned grid = (unsigned)std::min<int64_t>(A.n, 1 << 20);
-  for (;;) {
+  auto run = [&](auto phase, int H, const int32_t* crp, int32_t* cci, double* cv) {
+    constexpr int PH = decltype(phase)::value;
+    const size_t slot = sizeof(int32_t) + (PH == 1 ? sizeof(double) : 0);
+    int rows = kT / kGemmLanes;  // rows to a block: at most 48 KB of tables, at least one wave
+    while (rows > 2 && rows * H * slot > 48 * 1024) rows /= 2;
+    const size_t lds = rows * H * slot;
+    int shift = 32;
+    while ((1 << (32 - shift)) < H) --shift;
+    const auto kern = k_spgemm<PH>;
+    set_lds_limit((const void*)kern, lds);
+    hipLaunchKernelGGL(kern, dim3((unsigned)std::min<int64_t>((A.n + rows - 1) / rows, 1 << 20)),
+                       dim3(rows * kGemmLanes), lds, s, A.rp.p, A.ci.p, av, B.rp.p, B.ci.p, B.v.p, A.n, H, shift, crp,
+                       cnt.p, cci, cv, ovf.p);
+    NALU_HIP_CHECK(hipGetLastError());
+  };
+  for (int H = kFirstHash;; H = std::min(4 * H, kMaxHash)) {
     NALU_HIP_CHECK(hipMemsetAsync(ovf.p, 0, sizeof(int), s));
     NALU_HIP_CHECK(hipMemsetAsync(cnt.p, 0, sizeof(int32_t) * (A.n + 1), s));
-    const size_t lds = (size_t)H * (sizeof(double) + sizeof(int32_t));
-    hipLaunchKernelGGL(k_spgemm<0>, dim3(grid), dim3(64), lds, s, A.rp.p, A.ci.p, av, B.rp.p, B.ci.p, B.v.p, A.n,
-                       H, (const int32_t*)nullptr, cnt.p, (int32_t*)nullptr, (double*)nullptr, ovf.p);
-    NALU_HIP_CHECK(hipGetLastError());
+    run(std::integral_constant<int, 0>{}, H, nullptr, nullptr, nullptr);
     if (to_host(ovf.p, s) == 0) break;
-    NALU_REQUIRE(H < kMaxHash && H < 2 * bound, NALU_ERR_UNSUPPORTED,
+    NALU_REQUIRE(H < kMaxHash, NALU_ERR_UNSUPPORTED,
                  "amg: a product row has more than " + std::to_string(H) + " distinct columns");
-    while (H < 2 * bound && H < kMaxHash) H <<= 1;
   }
-  const size_t lds = (size_t)H * (sizeof(double) + sizeof(int32_t));
   {
     DevBuf<unsigned long long> tot(1);
     NALU_HIP_CHECK(hipMemsetAsync(tot.p, 0, sizeof(unsigned long long), s));
@@ -653,9 +684,9 @@ Csr spgemm(const Csr& A, const double* av, const Csr& B, hipStream_t s) {
   C.max_row = dev_max(cnt.p, A.n, s);
   C.ci.alloc(std::max<int64_t>(C.nnz, 1));
   C.v.alloc(std::max<int64_t>(C.nnz, 1));
-  hipLaunchKernelGGL(k_spgemm<1>, dim3(grid), dim3(64), lds, s, A.rp.p, A.ci.p, av, B.rp.p, B.ci.p, B.v.p, A.n, H,
-                     C.rp.p, cnt.p, C.ci.p, C.v.p, ovf.p);
-  NALU_HIP_CHECK(hipGetLastError());
+  int H = 64;
+  while (H < 2 * C.max_row && H < kMaxHash) H <<= 1;
+  run(std::integral_constant<int, 1>{}, H, C.rp.p, C.ci.p, C.v.p);
   return C;
 }
 
@@ -705,11 +736,15 @@ Csr transpose(const Csr& P, hipStream_t s) {
 // sum of squares of each row (R rows = P columns)
 __global__ void k_row_sumsq(const int32_t* __restrict__ rp, const double* __restrict__ v, int64_t n,
                             double* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t i = t / kL;
+  const int lane = (int)(t % kL);
   double s = 0.0;
-  for (int32_t q = rp[i]; q < rp[i + 1]; ++q) s += v[q] * v[q];
-  out[i] = s;
+  if (i < n)
+    for (int32_t q = rp[i] + lane; q < rp[i + 1]; q += kL) s += v[q] * v[q];
+#pragma unroll
+  for (int o = kL / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, kL);
+  if (i < n && lane == 0) out[i] = s;
 }
 
 __global__ void k_dense_fill(const int32_t* __restrict__ rp, const int32_t* __restrict__ ci,
@@ -901,16 +936,20 @@ void amg_setup(nalu_linsys* ls) {
                        pr.drop_tol, omega, strong.p, sv.p);
     DevBuf<int8_t> state(n);
     NALU_HIP_CHECK(hipMemsetAsync(state.p, 0, n, s));
-    DevBuf<uint64_t> key(n), m1(n), m2(n);
+    DevBuf<int8_t> live(n);
+    NALU_HIP_CHECK(hipMemsetAsync(live.p, 1, n, s));
+    DevBuf<uint64_t> m1(n);
     DevBuf<int> und(1);
-    int rounds = 0;
-    for (;; ++rounds) {
+    // two rounds to a host read: a round after the last one changes nothing
+    for (int rounds = 0;; rounds += 2) {
       NALU_REQUIRE(rounds <= 4096, NALU_ERR_NUMERIC, "amg: aggregation did not settle");
-      hipLaunchKernelGGL(k_mis_keys, dim3(nbl(n)), dim3(kT), 0, s, state.p, n, key.p);
-      hipLaunchKernelGGL(k_mis_max, dim3(nbl(n * kL)), dim3(kT), 0, s, L.A.rp.p, L.A.ci.p, strong.p, key.p, n, m1.p);
-      hipLaunchKernelGGL(k_mis_max, dim3(nbl(n * kL)), dim3(kT), 0, s, L.A.rp.p, L.A.ci.p, strong.p, m1.p, n, m2.p);
-      NALU_HIP_CHECK(hipMemsetAsync(und.p, 0, sizeof(int), s));
-      hipLaunchKernelGGL(k_mis_update, dim3(nbl(n)), dim3(kT), 0, s, key.p, m2.p, n, state.p, und.p);
+      for (int k = 0; k < 2; ++k) {
+        hipLaunchKernelGGL(k_mis_near, dim3(nbl(n * kL)), dim3(kT), 0, s, L.A.rp.p, L.A.ci.p, strong.p, state.p, n,
+                           live.p, m1.p);
+        if (k == 1) NALU_HIP_CHECK(hipMemsetAsync(und.p, 0, sizeof(int), s));
+        hipLaunchKernelGGL(k_mis_far, dim3(nbl(n * kL)), dim3(kT), 0, s, L.A.rp.p, L.A.ci.p, strong.p, m1.p, n, state.p,
+                           und.p);
+      }
       if (to_host(und.p, s) == 0) break;
     }
     DevBuf<int32_t> rflag(n + 1), rid(n + 1);
@@ -979,7 +1018,7 @@ void amg_setup(nalu_linsys* ls) {
     if (amg->lev.size() >= 2) {
       const Level& Lp = amg->lev[amg->lev.size() - 2];
       DevBuf<double> sq(nc);
-      hipLaunchKernelGGL(k_row_sumsq, dim3(nbl(nc)), dim3(kT), 0, s, Lp.R.rp.p, Lp.R.v.p, nc, sq.p);
+      hipLaunchKernelGGL(k_row_sumsq, dim3(nbl(nc * kL)), dim3(kT), 0, s, Lp.R.rp.p, Lp.R.v.p, nc, sq.p);
       scale = std::max(scale, host_absmax(Lp.diag.p, Lp.A.n) * host_absmax(sq.p, nc));
     }
     const double tiny = 1e-10 * scale;
