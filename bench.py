@@ -709,9 +709,9 @@ def main():
         "sgs_apply": (t_sgs * (iters + 1), byt["sgs_apply"], 2 * ncol - 1),
         "spmv": (t_spmv * (iters + 1), byt["spmv"], 1),
     }
-    kname = {"gather": ("k_scalar_gather<ContinuityOp>", "k_momentum_tile"),
+    kname = {"gather": ("k_scalar_rows<ContinuityOp>", "k_momentum_rows"),
              "atomic": ("k_scalar_atomic<ContinuityOp>", "k_momentum_atomic"),
-             "tile": ("k_scalar_tile<ContinuityOp>", "k_momentum_tile"),
+             "tile": ("k_scalar_rows<ContinuityOp>", "k_momentum_rows"),
              "etile": ("k_scalar_items<ContinuityEt> + k_scalar_etile", "k_momentum_items + k_momentum_etile")}
     if fused:
         del per_step["mdot"]

@@ -248,8 +248,8 @@ int nalu_linsys_solve_stacked(nalu_linsys *ls, int k, const double *B, double *X
  * the element kernel, and the scatter into the system (the consolidated
  * AssembleElemSolverAlgorithm::execute, src/AssembleElemSolverAlgorithm.C:75-100).
  * Contributions are ADDED to the system (call nalu_linsys_zero first).
- * mode: 0 = owner-computes row gather (deterministic, no atomics, scalar
- * systems), 1 = element-centric atomic scatter. */
+ * mode: 0 or 2 = owner-computes rows (scalar systems: deterministic), 1 =
+ * element-centric atomic scatter, 3 = element-visit tiles. */
 /* ScalarDiffElemKernel (src/kernel/ScalarDiffElemKernel.C:66-111). */
 int nalu_assemble_scalar_diff(nalu_linsys *ls, const nalu_mesh *m, const double *q_dev,
                               const double *diff_coeff_dev, int shifted_grad_op, int mode);
@@ -297,7 +297,7 @@ int nalu_assemble_continuity(nalu_linsys *ls, const nalu_mesh *m, const double *
 /* ContinuityAdvElemKernel and ComputeMdotElemAlgorithm
  * (src/ComputeMdotElemAlgorithm.C:85-250) from one evaluation of the scs
  * geometry, as the consolidated algorithm's kernels share their element data:
- * the continuity system as nalu_assemble_continuity (row gather) and mdot_dev
+ * the continuity system as nalu_assemble_continuity (rows) and mdot_dev
  * [E][12] as nalu_compute_mdot (same formula; sums in another order). */
 int nalu_assemble_continuity_mdot(nalu_linsys *ls, const nalu_mesh *m, const double *rho_dev,
                                   const double *p_dev, const double *u_dev, const double *gpdx_dev,
@@ -320,11 +320,11 @@ int nalu_assemble_momentum_mass(nalu_linsys *ls, const nalu_mesh *m, const doubl
 /* MomentumAdvDiffElemKernel and MomentumMassElemKernel in one pass over the
  * elements, as AssembleElemSolverAlgorithm::execute runs its kernel list
  * (src/AssembleElemSolverAlgorithm.C:75-100 with both kernels registered):
- * the arguments of nalu_assemble_momentum (node-tile scatter) and of
- * nalu_assemble_momentum_mass; one LDS row segment per tile, one write of the
+ * the arguments of nalu_assemble_momentum (rows) and of
+ * nalu_assemble_momentum_mass; one LDS row segment per block of rows, one write of the
  * matrix (the mass part is FP64 arithmetic on FP32-assembly systems too, as in
  * nalu_assemble_momentum_mass).  With skew or shifted set, or rows too long for
- * a node tile, the two kernels run as two passes. */
+ * one block's LDS, the two kernels run as two passes. */
 int nalu_assemble_momentum_with_mass(nalu_linsys *ls, const nalu_mesh *m, const double *u, const double *mu,
                                      const double *mdot, double include_divu, int skew, int shifted,
                                      const double *rho_nm1, const double *rho_n, const double *rho_np1,

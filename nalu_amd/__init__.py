@@ -787,8 +787,8 @@ class LearnedPreconditioner:
 
 
 # ------------------------------------------------------------------ assembly algorithms
-# scatter strategies: "gather" = one thread per row walks its elements (deterministic),
-# "atomic" = element-centric FP64 atomics, "tile" = node-tile LDS accumulation, "etile" =
+# scatter strategies: "gather" and "tile" = owner-computes rows accumulated in LDS
+# (deterministic on scalar systems), "atomic" = element-centric FP64 atomics, "etile" =
 # element-visit tiles (each incident element evaluated once per tile of rows)
 MODE = {"gather": 0, "atomic": 1, "tile": 2, "etile": 3}
 

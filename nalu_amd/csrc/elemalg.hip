@@ -15,7 +15,7 @@
 // owner-computes node pass for the mass kernels), all adding into the same
 // rows, which gives the same sums up to rounding order -- except that a
 // momentum advection-diffusion kernel and a momentum mass kernel of the same
-// list share one node-tile pass (nalu_assemble_momentum_with_mass).
+// list share one row pass (nalu_assemble_momentum_with_mass).
 #include <algorithm>
 #include <cmath>
 #include <vector>
