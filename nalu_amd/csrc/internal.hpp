@@ -261,6 +261,7 @@ struct nalu_linsys {
   nalu::DevBuf<uint64_t> elem_pos; // [8][E]
   // packed nodal fields of a row-assembly pass (assemble.hip)
   nalu::DevBuf<unsigned char> pack_ws;
+  bool pack_denied = false;  // no memory for pack_ws
 
   // expanded CSR (numDof rows interleaved, src/TpetraLinearSystem.C:1227-1246)
   nalu::DevBuf<int32_t> row_ptr;   // [nrows+1]
