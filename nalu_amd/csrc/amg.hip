@@ -886,7 +886,7 @@ void amg_setup(nalu_linsys* ls) {
   NALU_REQUIRE(ls->nrows > 0, NALU_ERR_STATE, "amg preconditioner: empty system");
   const nalu_muelu_params& pr = ls->muelu;
   hipStream_t s = ls->stream;
-  PoolScope scope(ls->pool, s);
+  PoolScope scope(ls->pool);
   NALU_HIP_CHECK(hipStreamSynchronize(s));
   const auto t0 = std::chrono::steady_clock::now();
   amg_release(ls);
@@ -1069,7 +1069,7 @@ void ensure_amg32(nalu_linsys* ls) {
   Amg* amg = amg_of(ls);
   if (amg->f32_ready) return;
   hipStream_t s = ls->stream;
-  PoolScope scope(ls->pool, s);
+  PoolScope scope(ls->pool);
   auto conv = [&](Csr& C) {
     if (C.nnz == 0) return;
     C.v32.alloc(C.nnz);

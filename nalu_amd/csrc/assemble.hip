@@ -1478,7 +1478,7 @@ extern "C" int nalu_linsys_apply_dirichlet(nalu_linsys* ls, int64_t nbc, const i
     materialize_pending_zero(ls);
     const int64_t n = nbc * (end - begin);
     if (n == 0) return NALU_OK;
-    PoolScope scope(ls->pool, ls->stream);
+    PoolScope scope(ls->pool);
     DevBuf<int> bad(1);
     NALU_HIP_CHECK(hipMemsetAsync(bad.p, 0, sizeof(int), ls->stream));
     hipLaunchKernelGGL(k_dirichlet, dim3(blocks_for(n, 256)), dim3(256), 0, ls->stream, nodes, nbc, ls->num_nodes,
@@ -1500,7 +1500,7 @@ extern "C" int nalu_linsys_reset_rows(nalu_linsys* ls, int64_t nn, const int32_t
     materialize_pending_zero(ls);
     const int64_t n = nn * (end - begin);
     if (n == 0) return NALU_OK;
-    PoolScope scope(ls->pool, ls->stream);
+    PoolScope scope(ls->pool);
     DevBuf<int> bad(1);
     NALU_HIP_CHECK(hipMemsetAsync(bad.p, 0, sizeof(int), ls->stream));
     hipLaunchKernelGGL(k_dirichlet, dim3(blocks_for(n, 256)), dim3(256), 0, ls->stream, nodes, nn, ls->num_nodes,

@@ -52,9 +52,12 @@ int guarded(F&& f) {
 // -------------------------------------------------------- device buffers
 // Device memory that a handle keeps between calls: buffers allocated in a
 // PoolScope return to the handle's pool instead of to the runtime (every hipFree
-// synchronizes the device; an AMG set-up at 96^3 makes about a hundred).  All work of
-// a handle runs in order on its stream, so a returned block can be taken again at
-// once; a scope on another stream than the last one waits for the device first.
+// synchronizes the device; an AMG set-up at 96^3 makes about a hundred).  Work of a
+// handle runs in order while it stays on one stream, so a returned block can be taken
+// again at once.  It may still be in use on any stream that the handle was on since
+// (an application of the preconditioner is asynchronous and opens no scope), so the
+// first scope after a change of stream waits for the device, also when the handle is
+// back on the stream of the last scope (set_stream reports each change).
 // One handle is used by one thread at a time, and so is its pool.  Idle memory is
 // bounded and goes back with the handle; blocks past the bound, and all idle ones
 // when an allocation fails, are freed.
@@ -64,10 +67,11 @@ class DevPool {
   DevPool(const DevPool&) = delete;
   DevPool& operator=(const DevPool&) = delete;
   ~DevPool() { trim(); }
-  void on_stream(hipStream_t s) {
-    if (used_ && s != stream_) NALU_HIP_CHECK(hipDeviceSynchronize());
+  void stream_changed() { changed_ = true; }
+  void enter() {
+    if (changed_ && used_) NALU_HIP_CHECK(hipDeviceSynchronize());
+    changed_ = false;
     used_ = true;
-    stream_ = s;
   }
   void* get(size_t bytes, size_t* cap) {
     // sizes recur from one set-up to the next but for a few per cent: round up to an
@@ -114,15 +118,15 @@ class DevPool {
   }
   std::multimap<size_t, void*> idle_;
   size_t idle_bytes_ = 0;
-  hipStream_t stream_ = nullptr;
   bool used_ = false;
+  bool changed_ = false;  // the handle's stream since the last scope
 };
 // Buffers allocated while it lives come from the pool.  Only for buffers that die
 // with the pool's handle or before it.
 struct PoolScope {
   DevPool* prev;
-  PoolScope(DevPool& p, hipStream_t s) : prev(DevPool::current()) {
-    p.on_stream(s);
+  explicit PoolScope(DevPool& p) : prev(DevPool::current()) {
+    p.enter();
     DevPool::current() = &p;
   }
   PoolScope(const PoolScope&) = delete;

@@ -1803,7 +1803,7 @@ extern "C" int nalu_gnn_loss_grad(nalu_gnn* g, nalu_linsys* ls, int batch, const
     hipStream_t s = ls->stream;
     nalu::Work w;
     {
-      nalu::PoolScope scope(ls->pool, s);
+      nalu::PoolScope scope(ls->pool);
       w.alloc(n, batch, g->L);
     }
     hipLaunchKernelGGL((nalu::k_gather_perm<float, float>), dim3(nalu::nblocks(T)), dim3(nalu::kThreads), 0, s, r_dev,

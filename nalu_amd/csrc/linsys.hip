@@ -149,6 +149,7 @@ extern "C" int nalu_linsys_destroy(nalu_linsys* ls) {
 extern "C" int nalu_linsys_set_stream(nalu_linsys* ls, void* stream) {
   return guarded([&]() -> int {
     NALU_REQUIRE(ls, NALU_ERR_ARG, "set_stream: null handle");
+    if (ls->stream != (hipStream_t)stream) ls->pool.stream_changed();
     ls->stream = (hipStream_t)stream;
     return NALU_OK;
   });

@@ -69,6 +69,37 @@ def test_repeated_setups_and_streams():
         assert close(x / (1.0 + k), ref)
 
 
+def test_setup_back_on_the_first_stream_waits_for_the_other():
+    """Set-up on A, applications on B (asynchronous), a set-up on A again: it returns the
+    hierarchy's memory and takes it anew, so it has to wait for B.  The matrix is the
+    same, so each application gives the same vector (1e-12: the hierarchy's products add
+    in an order that depends on timing)."""
+    P = Problem(40, 4)
+    ls = P.handle()
+    P.solve(ls)
+    n = P.f[1].shape[0]
+    r = dev(np.random.default_rng(1).normal(size=n))
+    ref = torch.zeros_like(r)
+    ls.precond_apply(r, ref)
+    A, B = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for k in range(4):
+        print("case: set-up on A, applications on B, set-up on A", k, flush=True)
+        ls.set_stream(A.cuda_stream)
+        ls.precond_setup()
+        A.synchronize()
+        ls.set_stream(B.cuda_stream)
+        z = [torch.zeros_like(r) for _ in range(8)]
+        torch.cuda.synchronize()
+        for q in z:
+            ls.precond_apply(r, q)
+        ls.set_stream(A.cuda_stream)
+        ls.precond_setup()
+        torch.cuda.synchronize()
+        for q in z:
+            assert float((q - ref).norm() / ref.norm()) <= 1e-12
+
+
 def test_threads_with_a_handle_each():
     probs = [Problem(10 + k, 5 + k) for k in range(3)]
     refs = [P.solve(P.handle()) for P in probs]
