@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "internal.hpp"
+#include "lookahead.hpp"
 
 // unroll depth of the SELL entry loops (loads in flight per lane)
 #ifndef NALU_SPARSE_UNROLL
@@ -1554,10 +1555,8 @@ int gmres_t(nalu_linsys* ls, const double* b, double* x, int m, int maxit, doubl
   std::vector<double> hcol(m + 2), y;
   (void)xt;
 
-  // The host decides from each column's norm whether to go on.  The next column's
-  // preconditioner and product are enqueued before it waits for that norm, so the
-  // device does not idle for the read (about 20 us of a 100 us iteration at 32^3);
-  // the last column of a cycle leaves one such product unused.
+  // the next column's product ahead of the host's read of this column's norm
+  LookAhead look(n, ls->cfg.precond, !always2);
   struct Event {
     hipEvent_t e = nullptr;
     Event() { NALU_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming)); }
@@ -1587,6 +1586,7 @@ int gmres_t(nalu_linsys* ls, const double* b, double* x, int m, int maxit, doubl
       spmv_m<TV, TV>(ls, nrhs, zc, V + (size_t)ldv * (c + 1), (const TV*)nullptr, 0);
     };
     bool ahead = false;  // product(k) is already enqueued
+    double res = beta;
     for (; k < m && iters < maxit; ++k) {
       ++iters;
       TV* vk1 = V + (size_t)ldv * (k + 1);
@@ -1612,21 +1612,25 @@ int gmres_t(nalu_linsys* ls, const double* b, double* x, int m, int maxit, doubl
         hipLaunchKernelGGL(k_reduce_rows, dim3(1), dim3(kThreads), 0, s, ls->red.p, (int)nb_upd, nrm, 0);
       }
       NALU_HIP_CHECK(hipMemcpyAsync(hpin, hbuf, hbytes, hipMemcpyDeviceToHost, s));
-      NALU_HIP_CHECK(hipEventRecord(col_read.e, s));
       auto normalize = [&]() {
         hipLaunchKernelGGL(k_scale_invnorm<TV>, dim3(nblocks(n)), dim3(kThreads), 0, s, vk1, n, nrm);
       };
-      normalize();
-      ahead = k + 1 < m && iters < maxit;
+      NALU_HIP_CHECK(hipEventRecord(col_read.e, s));
+      ahead = k + 1 < m && iters < maxit && look(res, tol * r0);
+      // scaled before the norm is read, a launch less between two columns, unless the
+      // column is likely to change again
+      const bool scaled = !look.cancelled;
+      if (scaled) normalize();
       if (ahead) product(k + 1);
       NALU_HIP_CHECK(hipEventSynchronize(col_read.e));
       for (int i = 0; i <= k; ++i) hcol[i] = hpin[i] + (always2 ? hpin[(m + 2) + i] : 0.0);
       hcol[k + 1] = std::sqrt(hpin[2 * (m + 2)]);
-      // FP32: severe cancellation (or NaN) reorthogonalizes once, on the vector
-      // already scaled by its norm n1, so the new coefficients and norm count n1
-      // times (a zero vector needs none)
-      if (!always2 && hcol[k + 1] != 0.0 && !(hpin[2 * (m + 2)] >= 0.01 * hpin[cnt])) {
-        const double n1 = hcol[k + 1];
+      // FP32: severe cancellation (or NaN) reorthogonalizes once; where the vector is
+      // already scaled by its norm n1, the new coefficients and norm count n1 times (a
+      // zero vector needs none)
+      look.cancelled = !always2 && hcol[k + 1] != 0.0 && !(hpin[2 * (m + 2)] >= 0.01 * hpin[cnt]);
+      if (look.cancelled) {
+        const double n1 = scaled ? hcol[k + 1] : 1.0;
         second_pass();
         NALU_HIP_CHECK(hipMemcpyAsync(hpin, hbuf, hbytes, hipMemcpyDeviceToHost, s));
         normalize();
@@ -1634,13 +1638,17 @@ int gmres_t(nalu_linsys* ls, const double* b, double* x, int m, int maxit, doubl
         for (int i = 0; i <= k; ++i) hcol[i] += n1 * hpin[(m + 2) + i];
         hcol[k + 1] = n1 * std::sqrt(hpin[2 * (m + 2)]);
         ahead = false;
+      } else if (!scaled) {
+        normalize();
       }
       if (learned_cycle && !std::isfinite(hcol[k + 1])) {
         learned_set_fallback(ls, true);  // drop this direction, finish the cycle with k columns
         break;
       }
       NALU_REQUIRE(std::isfinite(hcol[k + 1]), NALU_ERR_NUMERIC, "gmres: non-finite Arnoldi vector");
-      const double res = H.add_column(k, hcol.data());
+      const double before = res;
+      res = H.add_column(k, hcol.data());
+      look.fall = res / before;
       rel = res / r0;
       if (res <= tol * r0 || hcol[k + 1] == 0.0) {
         ++k;

@@ -1,7 +1,7 @@
 """AddressSanitizer + UndefinedBehaviorSanitizer runs on the CPU: the oracle
 (oracle/oracle.c, every entry on a small jittered lattice), the host side of
-the C ABI (every .hip source compiled host-only, plus the lattice generator) and
-its memory pool, built by tests/sanitize/Makefile.  A sanitizer report, a leak or a failed
+the C ABI (every .hip source compiled host-only, plus the lattice generator),
+its memory pool and the look-ahead rule of (F)GMRES, built by tests/sanitize/Makefile.  A sanitizer report, a leak or a failed
 check ends the driver with a non-zero status."""
 import os
 import shutil
@@ -25,7 +25,7 @@ def _build(target):
     return os.path.join(SAN, "_build", target)
 
 
-@pytest.mark.parametrize("target", ["oracle_driver", "host_abi", "pool"])
+@pytest.mark.parametrize("target", ["oracle_driver", "host_abi", "pool", "lookahead"])
 def test_sanitized_driver_is_clean(target):
     exe = _build(target)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=300, env=ENV)
