@@ -2,11 +2,14 @@
 more incident elements than a row has lanes (fan meshes), element axes that differ
 from element to element (every local node as the row node, both handednesses),
 row counts around the tile sizes, explicit node ids, and systems on both sides of
-the size from which the nodal fields are packed first (32768 nodes).
+the size from which the nodal fields are packed first (32768 nodes), in FP64 and with
+FP32 arithmetic (other records in the packed copy of the fluxes).
 
 Bar: 1e-12 of the row's (rhs: of the vector's) largest entry.  Entries are sums of
 at most 24 products of coordinate differences (about 1e2 eps), and the meshes have
-cells no smaller than 1/33 of their coordinates (a further factor of 1e2)."""
+cells no smaller than 1/33 of their coordinates (a further factor of 1e2).  FP32
+arithmetic: 3e-5, a few hundred operations an entry at unit roundoff 6e-8 (the bar of
+the mixed-precision tests); the geometry is FP64."""
 import numpy as np
 import pytest
 
@@ -18,7 +21,7 @@ from tests.fixtures import rel_err_rowwise  # noqa: E402
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
-TOL = 1e-12
+TOL = {"fp64": 1e-12, "mixed": 3e-5}
 # the 24 orientation-preserving relabelings of the reference hexahedron's nodes
 SIGN = np.array([[-1, -1, -1], [1, -1, -1], [1, 1, -1], [-1, 1, -1], [-1, -1, 1], [1, -1, 1], [1, 1, 1], [-1, 1, 1]])
 
@@ -91,22 +94,31 @@ def problem(name, seed):
     return X, conn, f, rng
 
 
-def check(what, v, r, ov, orhs, row_ptr):
+# every mesh in FP64; FP32 arithmetic gathering from the fields and from the packed copies
+CASES = [(m, "fp64") for m in MESHES] + [(m, "mixed") for m in ("fan9", "pack", "pack-odd")]
+
+
+def system(nd, precision):
+    return na.LinearSystem(nd, na.SolverConfig("gmres", "sgs", precision=precision))
+
+
+def check(what, v, r, ov, orhs, row_ptr, tol):
     e1 = rel_err_rowwise(v, ov, row_ptr) if v is not None else 0.0
     e2 = np.abs(r - orhs).max() / np.abs(orhs).max()
     print("  %s: matrix %.2e rhs %.2e" % (what, e1, e2), flush=True)
-    assert e1 <= TOL and e2 <= TOL, what
+    assert e1 <= tol and e2 <= tol, what
 
 
-@pytest.mark.parametrize("name", list(MESHES))
+@pytest.mark.parametrize("name,precision", CASES)
 @pytest.mark.parametrize("ids", [False, True])
-def test_rows(oracle, name, ids):
-    print("case: row tiles on", name, "ids" if ids else "", flush=True)
+def test_rows(oracle, name, precision, ids):
+    print("case: row tiles on", name, precision, "ids" if ids else "", flush=True)
+    tol = TOL[precision]
     X, conn, f, rng = problem(name, 3)
     N, E = X.shape[0], conn.shape[0]
     gid = (rng.permutation(N) + 1).astype(np.int64) if ids else None
     mesh = na.Mesh(X, conn, gid)
-    ls = na.LinearSystem(1)
+    ls = system(1, precision)
     ls.buildElemToNodeGraph(mesh)
     ls.finalizeLinearSystem()
     g = oracle.graph_build(N, conn, node_ids=gid)
@@ -119,7 +131,7 @@ def test_rows(oracle, name, ids):
             na.assemble_scalar_diff(ls, mesh, d["p"], d["mu"], shifted=shifted, mode=mode)
             _, _, v, r = ls.csr()
             check("diffusion shifted=%d %s" % (shifted, mode), v, r,
-                  *oracle.assemble_scalar_diff(g, conn, X, f["p"], f["mu"], shifted=shifted), g.row_ptr)
+                  *oracle.assemble_scalar_diff(g, conn, X, f["p"], f["mu"], shifted=shifted), g.row_ptr, tol)
     mdot = torch.zeros((E, 12), dtype=torch.float64, device=DEV)
     for sm, sp, red in ((0, 0, 0), (0, 0, 1), (1, 1, 0)) if big else np.ndindex(2, 2, 2):
         ls.zeroSystem()
@@ -127,28 +139,41 @@ def test_rows(oracle, name, ids):
                                reduced_sens=red, mode="gather", mdot_out=mdot)
         _, _, v, r = ls.csr()
         ov, orhs = oracle.assemble_continuity(g, conn, X, f["rho"][2], f["p"], f["u"][2], f["gp"], 0.7, sm, sp, red)
-        check("continuity %d%d%d" % (sm, sp, red), v, r, ov, orhs, g.row_ptr)
+        check("continuity %d%d%d" % (sm, sp, red), v, r, ov, orhs, g.row_ptr, tol)
         om = oracle.compute_mdot(conn, X, f["rho"][2], f["p"], f["u"][2], f["gp"], 0.7, sm, sp)
-        assert np.abs(mdot.cpu().numpy() - om.reshape(E, 12)).max() <= TOL * np.abs(om).max()
-        na.compute_mdot(mesh, rho[2], d["p"], u[2], d["gp"], mdot, tau=0.7, shift_mdot=sm, shift_poisson=sp)
-        assert np.abs(mdot.cpu().numpy() - om.reshape(E, 12)).max() <= TOL * np.abs(om).max()
+        assert np.abs(mdot.cpu().numpy() - om.reshape(E, 12)).max() <= tol * np.abs(om).max()
+        na.compute_mdot(mesh, rho[2], d["p"], u[2], d["gp"], mdot, tau=0.7, shift_mdot=sm, shift_poisson=sp,
+                        precision="fp32" if precision == "mixed" else "fp64")
+        assert np.abs(mdot.cpu().numpy() - om.reshape(E, 12)).max() <= tol * np.abs(om).max()
     # a second pass onto the assembled system accumulates
     na.assemble_continuity(ls, mesh, rho[2], d["p"], u[2], d["gp"], tau=0.7, shift_mdot=sm, shift_poisson=sp,
                            reduced_sens=red, mode="tile")
     _, _, v, r = ls.csr()
-    check("accumulate", v, r, 2 * ov, 2 * orhs, g.row_ptr)
+    check("accumulate", v, r, 2 * ov, 2 * orhs, g.row_ptr, tol)
+    if precision != "fp64":
+        return  # the rest is FP64 arithmetic in either case
     vol, grad = torch.zeros(N, dtype=torch.float64, device=DEV), torch.zeros((N, 3), dtype=torch.float64, device=DEV)
     na.compute_dual_volume(mesh, vol)
     ovol = oracle.dual_nodal_volume(conn, X)
-    assert np.abs(vol.cpu().numpy() - ovol).max() <= TOL * ovol.max()
+    assert np.abs(vol.cpu().numpy() - ovol).max() <= tol * ovol.max()
     na.compute_nodal_gradient(mesh, d["p"], vol, grad)
     og = oracle.nodal_grad(conn, X, f["p"], ovol)
-    assert np.abs(grad.cpu().numpy() - og).max() <= TOL * np.abs(og).max()
+    assert np.abs(grad.cpu().numpy() - og).max() <= tol * np.abs(og).max()
 
 
-@pytest.mark.parametrize("name", list(MESHES))
-def test_momentum_rows(oracle, name):
-    print("case: momentum row tiles on", name, flush=True)
+def scalar(v3, g1, g3):
+    """Entries (0, 0) of the 3x3 blocks of a numDof 3 matrix, on the numDof 1 graph."""
+    out = np.empty(g1.row_ptr[-1])
+    for a in range(len(g1.row_ptr) - 1):
+        b = g3.row_ptr[3 * a]
+        out[g1.row_ptr[a]:g1.row_ptr[a + 1]] = v3[b:g3.row_ptr[3 * a + 1]:3]
+    return out
+
+
+@pytest.mark.parametrize("name,precision", CASES)
+def test_momentum_rows(oracle, name, precision):
+    print("case: momentum row tiles on", name, precision, flush=True)
+    tol = TOL[precision]
     X, conn, f, rng = problem(name, 4)
     N = X.shape[0]
     mesh = na.Mesh(X, conn)
@@ -156,7 +181,7 @@ def test_momentum_rows(oracle, name):
     rho, u = [d["rho"][i].contiguous() for i in range(3)], [d["u"][i].contiguous() for i in range(3)]
     g1, g3 = oracle.graph_build(N, conn), oracle.graph_build(N, conn, num_dof=3)
     gam, dt = (1.5, -2.0, 0.5), 0.3
-    l1, l3 = na.LinearSystem(1), na.LinearSystem(3)
+    l1, l3 = system(1, precision), system(3, precision)
     for ls in (l1, l3):
         ls.buildElemToNodeGraph(mesh)
         ls.finalizeLinearSystem()
@@ -171,13 +196,13 @@ def test_momentum_rows(oracle, name):
             l3.zeroSystem()
             na.assemble_momentum(l3, *args, mode=mode, **kw)
             _, _, v, r = l3.csr()
-            check("coupled %s %d%d %g" % (mode, skew, shifted, divu), v, r, *a3, g3.row_ptr)
+            check("coupled %s %d%d %g" % (mode, skew, shifted, divu), v, r, *a3, g3.row_ptr, tol)
         rhs3 = torch.zeros((3, N), dtype=torch.float64, device=DEV)
         l1.zeroSystem()
         na.assemble_momentum_segregated(l1, *args, rhs3, **kw)
         _, _, v, _ = l1.csr()
         check("segregated %d%d %g" % (skew, shifted, divu), v, rhs3.cpu().numpy().ravel(), a1[0], a1[1].ravel(),
-              g1.row_ptr)
+              g1.row_ptr, tol)
         for lumped, balanced in ((False, False), (True, True)):
             m3 = oracle.assemble_momentum_mass(g3, conn, X, f["rho"], f["u"], f["gp"], dt, gam, lumped, balanced)
             for states in (u, [u[0], u[1], u[2].clone()]):  # the Np1 state is the advected field, or another array
@@ -185,22 +210,23 @@ def test_momentum_rows(oracle, name):
                 na.assemble_momentum_with_mass(l3, *args, rho, states, d["gp"], dt, gamma=gam, lumped=lumped,
                                                balanced_force=balanced, **kw)
                 _, _, v, r = l3.csr()
-                check("coupled + mass lumped=%d" % lumped, v, r, a3[0] + m3[0], a3[1] + m3[1], g3.row_ptr)
-            rhs3.zero_()
-            l1.zeroSystem()
-            na.assemble_momentum_with_mass_segregated(l1, *args, rho, u, d["gp"], dt, rhs3, gamma=gam, lumped=lumped,
-                                                      balanced_force=balanced, **kw)
-            _, _, v1, _ = l1.csr()
-            r1 = rhs3.cpu().numpy().copy()
+                check("coupled + mass lumped=%d" % lumped, v, r, a3[0] + m3[0], a3[1] + m3[1], g3.row_ptr, tol)
+                rhs3.zero_()
+                l1.zeroSystem()
+                na.assemble_momentum_with_mass_segregated(l1, *args, rho, states, d["gp"], dt, rhs3, gamma=gam,
+                                                          lumped=lumped, balanced_force=balanced, **kw)
+                _, _, v1, _ = l1.csr()
+                r1 = rhs3.cpu().numpy().copy()
+                check("segregated + mass lumped=%d" % lumped, v1, r1.T.ravel(), a1[0] + scalar(m3[0], g1, g3),
+                      a3[1] + m3[1], g1.row_ptr, tol)
             rhs3.zero_()
             l1.zeroSystem()
             na.assemble_momentum_segregated(l1, *args, rhs3, **kw)
             na.assemble_momentum_mass_segregated(l1, mesh, rho, u, d["gp"], dt, rhs3, gamma=gam, lumped=lumped,
                                                  balanced_force=balanced)
             _, _, v, _ = l1.csr()
-            check("segregated + mass, one pass and two", v, r1.ravel(), v1, rhs3.cpu().numpy().ravel(), g1.row_ptr)
-            check("segregated + mass rhs", None, r1.T.ravel(), None, a3[1] + m3[1], None)
+            check("segregated + mass, one pass and two", v, r1.ravel(), v1, rhs3.cpu().numpy().ravel(), g1.row_ptr, tol)
             l3.zeroSystem()
             na.assemble_momentum_mass(l3, mesh, rho, u, d["gp"], dt, gamma=gam, lumped=lumped, balanced_force=balanced)
             _, _, v, r = l3.csr()
-            check("mass alone lumped=%d" % lumped, v, r, *m3, g3.row_ptr)
+            check("mass alone lumped=%d" % lumped, v, r, *m3, g3.row_ptr, tol)
