@@ -41,6 +41,8 @@ void flush_timers(nalu_linsys* ls) {
     float ms = 0.f;
     if (hipEventSynchronize(t.b) == hipSuccess && hipEventElapsedTime(&ms, t.a, t.b) == hipSuccess)
       ls->phase[t.phase] += 1e-3 * ms;
+    else
+      (void)hipGetLastError();  // recorded under capture: no time, and no error for the next call
     (void)hipEventDestroy(t.a);
     (void)hipEventDestroy(t.b);
   }
