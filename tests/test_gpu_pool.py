@@ -5,8 +5,8 @@ handle gives the memory back.
 
 Bar: solutions of two solves to 1e-12 on the same matrix within 1e-8 of each other
 (condition number below 1e4)."""
+import concurrent.futures
 import gc
-import threading
 
 import numpy as np
 import pytest
@@ -103,20 +103,16 @@ def test_setup_back_on_the_first_stream_waits_for_the_other():
 def test_threads_with_a_handle_each():
     probs = [Problem(10 + k, 5 + k) for k in range(3)]
     refs = [P.solve(P.handle()) for P in probs]
-    bad = []
 
     def work(P, ref):
         st = torch.cuda.Stream()
         ls = P.handle(st)
-        for _ in range(3):
-            if not close(P.solve(ls), ref):
-                bad.append(P)
+        return [close(P.solve(ls), ref) for _ in range(3)]
 
     print("case: three threads", flush=True)
-    ts = [threading.Thread(target=work, args=a) for a in zip(probs, refs)]
-    [t.start() for t in ts]
-    [t.join() for t in ts]
-    assert not bad
+    with concurrent.futures.ThreadPoolExecutor(3) as ex:
+        runs = [ex.submit(work, *a) for a in zip(probs, refs)]
+        assert [r.result() for r in runs] == [[True] * 3] * 3  # result() raises what the thread raised
 
 
 def test_destroying_the_handle_gives_the_memory_back():
