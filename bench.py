@@ -7,7 +7,7 @@ viscosity 1e-3, dt = gamma1 = 1.  One step is the hot path once:
 
   1. mdot at the 12 scs of every element (ComputeMdotElemAlgorithm)
   2. continuity system: zeroSystem, ContinuityAdvElemKernel assembly, loadComplete
-     (by default 1 and 2 are one pass: the continuity row gather evaluates each
+     (by default 1 and 2 are one pass: the continuity row pass evaluates each
      scs's geometry and writes its mdot too; --separate-mdot runs them apart)
   3. momentum system (3 dof/node, 27-point block rows): zeroSystem, MomentumAdvDiffElemKernel
   4. pressure-Poisson solve: CG + multicolor SGS to 1e-8 FP64 true relative residual
@@ -52,9 +52,9 @@ def parse():
     ap.add_argument("--muelu-degree", type=int, default=2, help="Chebyshev degree of the AMG smoother")
     ap.add_argument("--no-mixed", action="store_true", help="skip the FP32-assembly / mixed-precision block")
     ap.add_argument("--assembly-mode", default="gather", choices=["gather", "atomic", "tile", "etile"],
-                    help="scatter strategy of the continuity and momentum assembly (default: row gather for continuity, row tiles for momentum)")
+                    help="scatter strategy of the continuity and momentum assembly (default: rows for both)")
     ap.add_argument("--separate-mdot", action="store_true",
-                    help="compute mdot in its own pass instead of inside the continuity row gather")
+                    help="compute mdot in its own pass instead of inside the continuity row pass")
     ap.add_argument("--learned-apply-only", type=int, default=0, metavar="K",
                     help="only time K applications of an untrained learned preconditioner on the n^3 "
                          "continuity system (profiling aid), print one JSON line and exit")
@@ -305,7 +305,7 @@ def mixed_block(args, na, torch, mesh, P, devc, stream):
         na.assemble_momentum(mom, mesh, u, mu, md[prec], mode="tile")
         mom.loadComplete()
 
-    def assemble_fused(prec):  # as the step does: mdot written by the continuity row gather
+    def assemble_fused(prec):  # as the step does: mdot written by the continuity row pass
         cont, mom = sys_[prec]
         cont.zeroSystem()
         na.assemble_continuity(cont, mesh, rho, p, u, gp, tau=P["tau"], mode="gather", mdot_out=md[prec])
@@ -621,7 +621,7 @@ def main():
 
     ev = lambda: torch.cuda.Event(enable_timing=True)
     cmode = args.assembly_mode
-    mmode = "tile" if args.assembly_mode == "gather" else args.assembly_mode  # no row gather for numDof 3
+    mmode = "tile" if args.assembly_mode == "gather" else args.assembly_mode  # numDof 3 rows are mode "tile"
     fused = cmode == "gather" and not args.separate_mdot
 
     def step(timers=None):
@@ -716,7 +716,7 @@ def main():
     if fused:
         del per_step["mdot"]
     kern_name = {"mdot": "k_mdot_elem", "continuity_assembly": kname[cmode][0] + (" (+ mdot)" if fused else ""),
-                 "momentum_assembly": kname[mmode][1], "sgs_apply": "k_sell_fwd + k_sell_bwd",
+                 "momentum_assembly": kname[mmode][1], "sgs_apply": "k_sell_sweep",
                  "spmv": "k_sell_spmv"}
     def unit_t(k):
         return {"sgs_apply": t_sgs, "spmv": t_spmv}.get(k, per_step[k][0])

@@ -7,10 +7,11 @@
 // All kernels share the row arithmetic of hex8_row.hpp: one thread evaluates the
 // row of one node in one incident element, its corners numbered relative to that
 // node, on one code path for all eight local nodes.  Two scatter strategies:
-//   * owner-computes row tiles (modes 0 and 2): a block owns consecutive rows,
-//     eight threads per row take its incident elements, the rows meet in the LDS
-//     copy of the block's CSR segment, which is written once, coalesced; a pending
-//     zeroSystem is folded into that write.
+//   * owner-computes row tiles (modes 0 and 2): a wave owns consecutive scalar rows
+//     and four lanes of a row take its incident elements, a block owns consecutive
+//     nodes of a numDof 3 system and eight threads take a node's; the rows meet in
+//     the wave's or block's LDS copy of their CSR segment, which is written once,
+//     coalesced; a pending zeroSystem is folded into that write.
 //   * element-centric atomic scatter (mode 1): a block evaluates one local node's
 //     row of a chunk of elements, FP64 atomic adds into the CSR.
 #include <hip/hip_runtime.h>
@@ -880,10 +881,15 @@ inline size_t lds_rows(const nalu_linsys* ls) {
   return (size_t)kRowsPerBlock * ls->max_node_row_len * sizeof(double);
 }
 
-// From this many nodes on, a row pass copies its fields first: 128^3 continuity 1.14 ms
-// gathering from the fields, 0.75 ms with the copy.  Below, the copy's launch takes
-// what it saves (10^3 heat 2.11 ms without, 2.13 ms with it), and the handle is spared
-// the workspace.  Past 2^28 nodes the 32-bit offsets end.
+// From this many nodes on, a row pass copies its fields first.  A pass in FP64, us,
+// gathering from the fields / with the copy: continuity 32 768 nodes 37 / 38, 50 653
+// nodes 55 / 45, 117 649 nodes 95 / 62, 128^3 1140 / 750; 3-rhs momentum with mass
+// 50 653 nodes 68 / 69, 117 649 nodes 105 / 100, 912 673 nodes 624 / 584; coupled
+// momentum with mass 68 921 nodes 95 / 96, 912 673 nodes 971 / 917; diffusion 50 653
+// nodes 34 / 40, 274 625 nodes 77 / 79, 912 673 nodes 197 / 193.  The line is
+// continuity's, which gains most; the others lose the copy's launch, up to 6 us, up to
+// some 100 000 nodes (diffusion 500 000).  Below it no pass gains and the handle is
+// spared the workspace.  Past 2^28 nodes the 32-bit offsets end.
 // The workspace has its full size (six fields) from the first pass on and never moves,
 // as a captured graph may hold its address; where it cannot be had (a first pass under
 // capture, or no memory left) the passes gather from the fields themselves.
@@ -898,7 +904,6 @@ bool use_pack(nalu_linsys* ls) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   NALU_HIP_CHECK(hipStreamIsCapturing(ls->stream, &cap));
   if (cap != hipStreamCaptureStatusNone) return false;
-  ls->pack_ws.release();  // of a smaller graph finalized before on this handle
   void* q = nullptr;
   if (hipMalloc(&q, bytes) != hipSuccess) {
     (void)hipGetLastError();
@@ -1018,7 +1023,7 @@ void check_flag(DevBuf<int>& flag, hipStream_t s, const char* msg) {
 // Dual nodal volume (ComputeGeometryInteriorAlgorithm, src/ComputeGeometryInteriorAlgorithm.C:77-120)
 // and the interior Green-Gauss nodal gradient (AssembleNodalGradElemAlgorithm,
 // src/AssembleNodalGradElemAlgorithm.C:85-140), owner-computes: the node's scv and
-// its three adjacent scs are all that touch it.  Eight lanes per node take its
+// its three adjacent scs are all that touch it.  kSlots lanes per node take its
 // incident elements (as in k_scalar_rows), every result is written once.
 template <int NC, class Eval, class Store>
 __device__ __forceinline__ void node_sums(const int32_t* __restrict__ conn, const int32_t* __restrict__ inc_ptr,
@@ -1342,8 +1347,10 @@ extern "C" int nalu_compute_mdot_f32(const nalu_mesh* m, const double* rho, cons
 }
 
 namespace {
-// The longest node rows that the numDof 3 row tiles take: 64 of them (and their
-// rhs) fit the LDS of a CU (35 columns).
+// The longest node rows that mode 2 and the one-pass forms accept: 64 of them (and
+// their rhs) fit the LDS of a CU (35 columns).  Longer ones are refused by mode 2 and
+// take the atomic form and the mass gather.  A block of k_momentum_rows holds half as
+// many rows, so this limit is the entry points' and not the kernel's.
 bool numdof3_rows_fit(const nalu_linsys* ls) {
   return (64 * (size_t)ls->max_node_row_len * 9 + 3 * 64) * sizeof(double) <= kMaxLds;
 }

@@ -998,8 +998,10 @@ __global__ __launch_bounds__(SellBlock<P>::threads) void k_sell_sweep_dot(
 // not fill the chip and its time is one wave's chain plus the launch (about 2 us).
 // Sweeps, forward / backward: 74 chunks (32^3) 4.4 / 4.4 us with two waves, 3.3 / 3.3
 // with eight; 536 chunks (64^3, with r.z) 5.2 / 6.0 and 5.0 / 5.4; 4194 chunks (128^3)
-// four waves were already slower than two.  Product: 562 chunks (32^3) 9.2 us with
-// one wave, 6.2 with four; 4292 chunks (64^3) run at 4.9 TB/s with one.
+// four waves were already slower than two.  One SGS application with two / eight: 67.2
+// / 60.3 us at 759 chunks a color (72^3), 76.6 / 78.2 at 1038 (80^3), 177 / 253 at 4194.
+// Product, one wave / four: 7.7 / 5.7 us at 562 chunks (32^3), 10.0 / 8.9 at 1839 (48^3),
+// 11.6 / 12.9 at 2327 (52^3); 4292 chunks (64^3) run at 4.9 TB/s with one.
 constexpr int64_t kFewSweepChunks = 1024, kFewSpmvChunks = 2048;
 inline bool few_sweep(int64_t nch) { return nch <= kFewSweepChunks; }
 inline bool few_spmv(int64_t nch) { return nch <= kFewSpmvChunks; }
